@@ -11,8 +11,8 @@
 //     h1 = relu(W1 x + b1)  (128)    h2 = relu(W2 h1 + b2)  (128)
 //     logits = W3 h2 + b3   (16, one per candidate slot)
 //
-// bf16 operands, fp32 accumulation, on MFMA (v_mfma_f32_16x16x32_bf16 for the
-// locator, v_mfma_f32_16x16x16_bf16 in the training GEMM). The
+// bf16 operands, fp32 accumulation, on MFMA (v_mfma_f32_16x16x32_bf16, and
+// v_mfma_f32_16x16x16_bf16 where the contraction is over the 16 slots). The
 // locator tests the candidates in the order of their logits with the exact FP64
 // point-in-polygon test of the quadtree path (same edge table, same arithmetic)
 // and stops at the first polygon that contains the point away from its edges.
@@ -20,9 +20,9 @@
 // candidates, or that have no hit after max_tests tests, are marked for the
 // exact quadtree path; everything else is final.
 //
-// Training runs forward and backward passes on the same MFMA tiles (a generic
-// 16x16-tile GEMM with strided operands) plus small kernels for the masked
-// softmax cross-entropy, bias and embedding gradients and Adam.
+// Training runs the forward pass, the masked softmax cross-entropy and the backward
+// pass in one kernel per batch (mlp_kernel, which also gives the logits alone), a
+// reduction of the workgroups' weight gradients, and Adam.
 #include <algorithm>
 #include <cmath>
 
@@ -34,10 +34,9 @@ namespace {
 
 constexpr int kCand   = 16;  // candidate slots per grid cell
 constexpr int kEmb    = 64;  // cell embedding width
-constexpr int kFour   = 32;  // Fourier features
-constexpr int kIn     = 96;  // kEmb + kFour
+constexpr int kIn     = 96;  // kEmb + 32 Fourier features
 constexpr int kHid    = 128; // hidden width
-constexpr int kFreqs  = 8;   // frequencies per axis (kFour = 2 axes x 8 x sin/cos)
+constexpr int kFreqs  = 8;   // frequencies per axis (2 axes x 8 x sin/cos = 32 features)
 
 typedef short bf16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
@@ -149,147 +148,8 @@ __global__ void __launch_bounds__(256)
   }
 }
 
-// C(m, n) = sum_k A(m, k) B(k, n) over 16x16 tiles, one wave per (tile, K chunk).
-// A(m, k) = A[m a_m + k a_k], B(k, n) = B[k b_k + n b_n] (bf16). M and N are
-// multiples of 16. atomic: C += partial (fp32) for split-K; otherwise the
-// epilogue adds bias[n], applies relu and the gate (keep where gate(m, n) > 0)
-// and stores fp32 C and/or bf16 Cb.
-struct GemmArgs {
-  uint16_t const* A;
-  int64_t a_m, a_k;
-  uint16_t const* B;
-  int64_t b_k, b_n;
-  int64_t M, N, K, kchunk;
-  float* C;
-  int64_t c_m, c_n;
-  uint16_t* Cb;
-  int64_t cb_m, cb_n;
-  float const* bias;
-  uint16_t const* gate;
-  int64_t g_m, g_n;
-  int relu, atomic;
-};
-
-__global__ void __launch_bounds__(256) gemm_kernel(GemmArgs a)
-{
-  int64_t const w      = (static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x) / kWave;
-  int64_t const tiles_n = a.N / 16;
-  int64_t const chunks  = (a.K + a.kchunk - 1) / a.kchunk;
-  if (w >= (a.M / 16) * tiles_n * chunks) return;
-  int64_t const chunk = w % chunks;
-  int64_t const t     = w / chunks;
-  int64_t const tm = t / tiles_n, tn = t % tiles_n;
-  int const l = lane_id(), g = l >> 4, r = l & 15;
-  int64_t const am = tm * 16 + r;
-  int64_t const bn = tn * 16 + r;
-  int64_t const k0 = chunk * a.kchunk;
-  int64_t const k1 = k0 + a.kchunk < a.K ? k0 + a.kchunk : a.K;
-  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-  for (int64_t k = k0; k < k1; k += 16) {
-    bf16x4 av, bv;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      int64_t const kk = k + 4 * g + j;
-      bool const in    = kk < k1;
-      av[j] = in ? static_cast<short>(a.A[am * a.a_m + kk * a.a_k]) : short{0};
-      bv[j] = in ? static_cast<short>(a.B[kk * a.b_k + bn * a.b_n]) : short{0};
-    }
-    acc = mfma16(av, bv, acc);
-  }
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    int64_t const m = tm * 16 + 4 * g + j;
-    int64_t const n = tn * 16 + r;
-    float v         = acc[j];
-    if (a.atomic) {
-      atomicAdd(a.C + m * a.c_m + n * a.c_n, v);
-      continue;
-    }
-    if (a.bias) v += a.bias[n];
-    if (a.relu) v = fmaxf(v, 0.f);
-    if (a.gate && !(from_bf16(a.gate[m * a.g_m + n * a.g_n]) > 0.f)) v = 0.f;
-    if (a.C) a.C[m * a.c_m + n * a.c_n] = v;
-    if (a.Cb) a.Cb[m * a.cb_m + n * a.cb_n] = to_bf16(v);
-  }
-}
-
-// Masked softmax cross-entropy over the first count[cell] slots. Rows with
-// label < 0 (or outside the mask) contribute nothing. dZ = (p - onehot) * scale.
-// stats += {loss sum, correct top-1, labelled rows}.
-__global__ void __launch_bounds__(256)
-  xent_kernel(float const* __restrict__ Z, uint32_t const* __restrict__ cells,
-              uint8_t const* __restrict__ count, int32_t const* __restrict__ labels, int64_t n,
-              int64_t rows, float scale, uint16_t* __restrict__ dZ, float* __restrict__ stats)
-{
-  int64_t const i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i >= rows) return;
-  int const c   = i < n ? (count[cells[i]] < kCand ? count[cells[i]] : kCand) : 0;
-  int const y   = i < n ? labels[i] : -1;
-  float const* z = Z + i * kCand;
-  if (y < 0 || y >= c) {
-    for (int s = 0; s < kCand; ++s) dZ[i * kCand + s] = 0;
-    return;
-  }
-  float mx = -INFINITY;
-  int best = 0;
-  for (int s = 0; s < c; ++s)
-    if (z[s] > mx) {
-      mx   = z[s];
-      best = s;
-    }
-  float sum = 0.f;
-  for (int s = 0; s < c; ++s) sum += expf(z[s] - mx);
-  for (int s = 0; s < kCand; ++s) {
-    float const p = s < c ? expf(z[s] - mx) / sum : 0.f;
-    dZ[i * kCand + s] = to_bf16((p - (s == y ? 1.f : 0.f)) * scale);
-  }
-  atomicAdd(stats + 0, logf(sum) - (z[y] - mx));
-  if (best == y) atomicAdd(stats + 1, 1.f);
-  atomicAdd(stats + 2, 1.f);
-}
-
-// out[c] += sum over rows of D[row][c] (bf16, `cols` columns, a divisor of 256).
-// Thread t reads column t % cols of rows t / cols, t / cols + 256 / cols, ...
-// (consecutive threads read consecutive bf16 of a row: coalesced), 16 rows each;
-// the block's partial sums per column meet in LDS, one atomic per column.
-constexpr int kColsumIters = 16;
-inline int64_t colsum_rows_per_block(int cols) { return int64_t{256} / cols * kColsumIters; }
-
-__global__ void __launch_bounds__(256)
-  colsum_kernel(uint16_t const* __restrict__ D, int64_t rows, int cols, float* __restrict__ out)
-{
-  __shared__ float part[256];
-  int const c            = threadIdx.x % cols;
-  int64_t const step     = 256 / cols;
-  int64_t const r0       = static_cast<int64_t>(blockIdx.x) * step * kColsumIters;
-  int64_t const r_end    = r0 + step * kColsumIters < rows ? r0 + step * kColsumIters : rows;
-  float s = 0.f;
-#pragma unroll
-  for (int k = 0; k < kColsumIters; ++k) {
-    int64_t const r = r0 + threadIdx.x / cols + k * step;
-    if (r < r_end) s += from_bf16(D[r * cols + c]);
-  }
-  part[threadIdx.x] = s;
-  __syncthreads();
-  if (threadIdx.x < cols) {
-    float t = 0.f;
-    for (int k = threadIdx.x; k < 256; k += cols) t += part[k];
-    atomicAdd(out + threadIdx.x, t);
-  }
-}
-
-// gE[cell_i][d] += dXe[i][d]
-__global__ void __launch_bounds__(256)
-  embed_grad_kernel(float const* __restrict__ dXe, uint32_t const* __restrict__ cells, int64_t n,
-                    float* __restrict__ gE)
-{
-  int64_t const t = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (t >= n * kEmb) return;
-  int64_t const i = t / kEmb;
-  int const d     = static_cast<int>(t % kEmb);
-  atomicAdd(gE + static_cast<int64_t>(cells[i]) * kEmb + d, dXe[t]);
-}
-
+// The step's other kernels: Adam, and the fill of the embedding gradient with the
+// packing of the weights.
 __global__ void __launch_bounds__(256)
   adam_kernel(float* __restrict__ p, uint16_t* __restrict__ pb, float const* __restrict__ grad,
               float* __restrict__ m, float* __restrict__ v, int64_t n, float lr, float b1, float b2,
@@ -307,17 +167,557 @@ __global__ void __launch_bounds__(256)
   pb[i]          = to_bf16(q);
 }
 
-__global__ void __launch_bounds__(256) fill_f32_kernel(float* __restrict__ p, int64_t n, float v)
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef short s16x2 __attribute__((ext_vector_type(2)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef uint16_t u16x8 __attribute__((ext_vector_type(8)));
+
+constexpr int kKT = 32;  // K per v_mfma_f32_16x16x32_bf16
+
+// D = A B + C on one 16x16x32 bf16 tile (gfx950). Lane l supplies
+// A[l % 16][8 (l / 16) + j] and B[8 (l / 16) + j][l % 16] (j = 0..7) and holds
+// D[4 (l / 16) + j][l % 16] (j = 0..3).
+__device__ __forceinline__ f32x4 mfma32(bf16x8 a, bf16x8 b, f32x4 c)
 {
-  int64_t const i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i < n) p[i] = v;
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
+}
+
+// Input column of k-slot j of K tile c for lane group g of a layer fed by the
+// previous layer's output tiles: the B operand of that tile is output tiles 2c
+// (slots 0..3: rows 4g + j) and 2c + 1 (slots 4..7: rows 16 + 4g + j - 4), so the
+// weights of slot j sit in that column. The first layer's input is in natural
+// order (32c + 8g + j).
+__host__ __device__ __forceinline__ int chained_col(int c, int g, int j)
+{
+  return 32 * c + (j < 4 ? 4 * g + j : 16 + 4 * g + (j - 4));
+}
+
+__device__ __forceinline__ __bf16 bf(float f) { return static_cast<__bf16>(f); }
+
+// The weights in the order the MLP kernel's A operands take them, one fragment of
+// 64 lanes x 8 (mfma32) or x 4 (mfma16) bf16 after another: a wave then reads a
+// fragment with one coalesced 16- or 8-byte load per lane. The backward layers need
+// the transposed weights, whose 8 values per lane lie a row apart in the parameters.
+constexpr int kF1    = 0;                        // W1 forward: 8 M tiles x 3 K tiles
+constexpr int kF2    = kF1 + 24 * 512;           // W2 forward: 8 x 4, chained columns
+constexpr int kF3    = kF2 + 32 * 512;           // W3 forward: 1 x 4, chained columns
+constexpr int kB2    = kF3 + 4 * 512;            // W2 transposed: 8 x 4, chained rows
+constexpr int kB1    = kB2 + 32 * 512;           // W1 transposed, embedding inputs: 4 x 4
+constexpr int kB3    = kB1 + 16 * 512;           // W3 transposed: 8 x 1, mfma16
+constexpr int kPack  = kB3 + 8 * 256;            // elements
+constexpr int kForward  = kB2;                   // the forward layers' share
+constexpr int kBackward = kPack - kB2;
+static_assert(kForward % 512 == 0 && kBackward % 512 == 0 && kBackward <= kForward,
+              "staged 1 KB at a time into one slot");
+constexpr int kPackThreads = kB3 / 8 + 8 * 64;   // one lane of one fragment each
+
+__device__ __forceinline__ void pack_lane(uint16_t const* __restrict__ pb, Layout const& lay, int t,
+                                          uint16_t* __restrict__ out)
+{
+  if (t >= kB3 / 8) {  // W3^T: A[m][4g + j] = W3[4g + j][16 mt + m]
+    int const u = t - kB3 / 8, mt = u / kWave, l = u % kWave, g = l >> 4, r = l & 15;
+    for (int j = 0; j < 4; ++j)
+      out[kB3 + 4 * u + j] = pb[lay.w3 + static_cast<int64_t>(4 * g + j) * kHid + 16 * mt + r];
+    return;
+  }
+  int const f = t / kWave, l = t % kWave, g = l >> 4, r = l & 15;
+  for (int j = 0; j < 8; ++j) {
+    int64_t at;
+    if (f < 24) {
+      at = lay.w1 + static_cast<int64_t>(16 * (f / 3) + r) * kIn + kKT * (f % 3) + 8 * g + j;
+    } else if (f < 56) {
+      int const q = f - 24;
+      at = lay.w2 + static_cast<int64_t>(16 * (q / 4) + r) * kHid + chained_col(q % 4, g, j);
+    } else if (f < 60) {
+      at = lay.w3 + static_cast<int64_t>(r) * kHid + chained_col(f - 56, g, j);
+    } else if (f < 92) {
+      int const q = f - 60;
+      at = lay.w2 + static_cast<int64_t>(chained_col(q % 4, g, j)) * kHid + 16 * (q / 4) + r;
+    } else {
+      int const q = f - 92;
+      at = lay.w1 + static_cast<int64_t>(chained_col(q % 4, g, j)) * kIn + 16 * (q / 4) + r;
+    }
+    out[8 * t + j] = pb[at];
+  }
+}
+
+// Packs the weights (the first blocks) and zeroes gE (the others, 16 bytes per
+// store where gE is aligned).
+constexpr int kPackBlocks = (kPackThreads + 255) / 256;
+__global__ void __launch_bounds__(256)
+  mlp_prepare_kernel(uint16_t const* __restrict__ pb, Layout lay, uint16_t* __restrict__ packed,
+                     float* __restrict__ gE, int64_t n, bool vec)
+{
+  if (blockIdx.x < kPackBlocks) {
+    int const t = static_cast<int>(blockIdx.x) * 256 + threadIdx.x;
+    if (t < kPackThreads) pack_lane(pb, lay, t, packed);
+    return;
+  }
+  int64_t const i0     = static_cast<int64_t>(blockIdx.x - kPackBlocks) * 256 + threadIdx.x;
+  int64_t const stride = static_cast<int64_t>(gridDim.x - kPackBlocks) * 256;
+  if (vec) {
+    float4* v = reinterpret_cast<float4*>(gE);
+    for (int64_t i = i0; i < n / 4; i += stride) v[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+    for (int64_t i = n / 4 * 4 + i0; i < n; i += stride) gE[i] = 0.f;
+  } else {
+    for (int64_t i = i0; i < n; i += stride) gE[i] = 0.f;
+  }
+}
+
+// The ranker's whole network over one batch: logits (TRAIN = false), or the masked
+// softmax cross-entropy, the backward pass, the embedding gradient (atomics on gE) and
+// each workgroup's share of the weight gradients (partials, reduced by
+// mlp_reduce_kernel in a fixed order).
+//
+// A workgroup of 4 waves takes tiles of 128 points, 32 per wave (two 16-point column
+// tiles, so that a weight fragment serves two MFMAs). The layers chain in registers
+// (chained_col), forward and backward. The weight gradients contract over the points,
+// which lie across lanes, so each layer's activations and deltas pass through LDS as
+// [feature][point] rows (272 bytes apart: the 16 rows a fragment reads start 4 banks
+// apart), one layer at a time in the same two slots; wave w owns M tiles 2w and
+// 2w + 1, whose accumulators stay in registers over all the workgroup's tiles. A bias
+// gradient is one more column tile, against ones.
+//
+// The packed weights pass through LDS once per tile (global_load_lds, the backward
+// ones during the loss): read as fragments straight from L2 by every wave they took
+// the kernel 63 us instead of 27. Bound by latency: at the default batch of 16,384
+// points each of 128 workgroups runs one tile, about 350 MFMAs per wave between its
+// copies and barriers. Whole step (with Adam, 20 us at 6.4 TB/s) at that batch and
+// 65,536 cells: 377 us as nine 16x16-tile GEMMs with 2-byte loads and their helper
+// kernels, 63 us now.
+constexpr int kMlpWaves = 4;
+constexpr int kMlpCols  = 2;                            // 16-point tiles per wave
+constexpr int kMlpTile  = kMlpWaves * kMlpCols * 16;    // points per workgroup tile
+constexpr int kTPitch   = kMlpTile + 8;                 // bf16 per transposed row
+constexpr int kTail     = kHid * kIn + kHid + kHid * kHid + kHid + kCand * kHid + kCand;
+constexpr int kDxPitch  = kEmb + 4;                     // floats per point's embedding delta
+static_assert(kMlpTile * kDxPitch * 4 <= 2 * kHid * kTPitch * 2, "the deltas fit the row slots");
+static_assert(kTail % 4 == 0, "the reduction reads 16 bytes per lane");
+
+struct MlpArgs {
+  GridView g;
+  uint16_t const* emb;     // bf16 embeddings
+  uint16_t const* packed;  // kPack bf16
+  float const* p;          // fp32 parameters (biases)
+  Layout lay;
+  double const* xy;
+  int64_t n, tiles;
+  float* Z;  // TRAIN = false: logits, n x 16
+  int32_t const* labels;
+  float scale;  // 1 / n
+  float* gE;
+  float* partials;  // gridDim.x x kTail
+  float* stats;
+};
+
+template <bool TRAIN>
+__global__ void __launch_bounds__(kMlpWaves * kWave, 1) mlp_kernel(MlpArgs a)
+{
+  __shared__ __attribute__((aligned(16))) uint16_t T[TRAIN ? 2 : 1][TRAIN ? kHid * kTPitch : 8];
+  __shared__ __attribute__((aligned(16))) uint16_t W[kForward];  // forward, then backward
+  __shared__ __attribute__((aligned(16))) float s_bias[2 * kHid + kCand];
+  __shared__ float s_stats[3];
+  int const wave = static_cast<int>(uniform(threadIdx.x / kWave));
+  int const l = lane_id(), g = l >> 4, r = l & 15;
+  for (int t = threadIdx.x; t < 2 * kHid + kCand; t += blockDim.x)
+    s_bias[t] = a.p[t < kHid ? a.lay.b1 + t
+                             : (t < 2 * kHid ? a.lay.b2 + t - kHid : a.lay.b3 + t - 2 * kHid)];
+  f32x4 const zero = {0.f, 0.f, 0.f, 0.f};
+  if (TRAIN && threadIdx.x < 3) s_stats[threadIdx.x] = 0.f;
+  float loss = 0.f, correct = 0.f, labelled = 0.f;
+  f32x4 dw1[2][kIn / 16], dw2[2][kHid / 16], dw3[2], db1[2], db2[2], db3 = zero;
+#pragma unroll
+  for (int m = 0; m < 2; ++m) {
+    dw3[m] = db1[m] = db2[m] = zero;
+#pragma unroll
+    for (int t = 0; t < kIn / 16; ++t) dw1[m][t] = zero;
+#pragma unroll
+    for (int t = 0; t < kHid / 16; ++t) dw2[m][t] = zero;
+  }
+  bf16x8 ones;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) ones[j] = bf(1.f);
+
+  // copies packed weights [at, at + 512 n) to the start of W, a KB per instruction
+  auto stage = [&](int at, int n) {
+    for (int f = wave; f < n; f += kMlpWaves)
+      __builtin_amdgcn_global_load_lds(
+        (__attribute__((address_space(1))) void const*)(a.packed + at + f * 512 + l * 8),
+        (__attribute__((address_space(3))) void*)(W + f * 512), 16, 0, 0);
+  };
+  auto staged = [] {  // every wave's copies have landed
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+  };
+  auto frag = [&](int at, int f) {  // of the staged range: fragment f from `at`
+    return *reinterpret_cast<bf16x8 const*>(W + at + (f * kWave + l) * 8);
+  };
+  auto bias4 = [&](int at) {  // the bias of rows 4g .. 4g + 3 of a tile
+    return *reinterpret_cast<f32x4 const*>(s_bias + at + 4 * g);
+  };
+  auto put = [&](f32x4 h, bf16x8& out, int half) {  // four rows into one half of a B operand
+#pragma unroll
+    for (int j = 0; j < 4; ++j) out[4 * half + j] = bf(h[j]);
+  };
+  auto relu = [](f32x4 h) {
+    return f32x4{fmaxf(h[0], 0.f), fmaxf(h[1], 0.f), fmaxf(h[2], 0.f), fmaxf(h[3], 0.f)};
+  };
+  // rows [0, 16 x tiles of v) of a slot from chained operands, this wave's columns
+  auto store_rows = [&](int slot, int t, int c, bf16x8 v) {
+    uint16_t* row = T[slot] + (32 * c + 4 * g) * kTPitch + (wave * kMlpCols + t) * 16 + r;
+    u16x8 const w = __builtin_bit_cast(u16x8, v);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) row[(j < 4 ? j : 16 + j - 4) * kTPitch] = w[j];
+  };
+  auto rows = [&](int slot, int tile, int ks) {
+    return *reinterpret_cast<bf16x8 const*>(T[slot] + (16 * tile + r) * kTPitch + 32 * ks + 8 * g);
+  };
+
+  for (int64_t tile = blockIdx.x; tile < a.tiles; tile += gridDim.x) {
+    stage(0, kForward / 512);
+    int64_t const base = tile * kMlpTile + wave * (kMlpCols * 16);
+    uint32_t cell[kMlpCols];
+    bf16x8 X[kMlpCols][kIn / kKT], H1[kMlpCols][kHid / kKT], H2[kMlpCols][kHid / kKT];
+#pragma unroll
+    for (int t = 0; t < kMlpCols; ++t) {
+      int64_t const p = base + 16 * t + r;
+      bool const in   = p < a.n;
+      Loc const L     = locate_cell(a.g, in ? a.xy[2 * p] : 0.0, in ? a.xy[2 * p + 1] : 0.0);
+      cell[t]         = L.cell;
+      uint16_t const* e = a.emb + static_cast<int64_t>(L.cell) * kEmb;
+#pragma unroll
+      for (int c = 0; c < kEmb / kKT; ++c)
+        X[t][c] = *reinterpret_cast<bf16x8 const*>(e + kKT * c + 8 * g);
+      // features 64 + 8g + j: frequencies 2g (j < 4) and 2g + 1 (j >= 4)
+      float f0[4], f1[4];
+      fourier4(L.u, L.v, 2 * g, f0);
+      fourier4(L.u, L.v, 2 * g + 1, f1);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        X[t][kEmb / kKT][j]     = bf(f0[j]);
+        X[t][kEmb / kKT][j + 4] = bf(f1[j]);
+      }
+      if (!in)  // padding rows: zero features
+        for (int c = 0; c < kIn / kKT; ++c) X[t][c] = bf16x8{};
+    }
+    staged();
+#pragma unroll
+    for (int mt = 0; mt < kHid / 16; ++mt) {
+      f32x4 h[kMlpCols];
+#pragma unroll
+      for (int t = 0; t < kMlpCols; ++t) h[t] = bias4(16 * mt);
+#pragma unroll
+      for (int c = 0; c < kIn / kKT; ++c) {
+        bf16x8 const w = frag(kF1, mt * (kIn / kKT) + c);
+#pragma unroll
+        for (int t = 0; t < kMlpCols; ++t) h[t] = mfma32(w, X[t][c], h[t]);
+      }
+#pragma unroll
+      for (int t = 0; t < kMlpCols; ++t) put(relu(h[t]), H1[t][mt / 2], mt % 2);
+    }
+#pragma unroll
+    for (int mt = 0; mt < kHid / 16; ++mt) {
+      f32x4 h[kMlpCols];
+#pragma unroll
+      for (int t = 0; t < kMlpCols; ++t) h[t] = bias4(kHid + 16 * mt);
+#pragma unroll
+      for (int c = 0; c < kHid / kKT; ++c) {
+        bf16x8 const w = frag(kF2, mt * (kHid / kKT) + c);
+#pragma unroll
+        for (int t = 0; t < kMlpCols; ++t) h[t] = mfma32(w, H1[t][c], h[t]);
+      }
+#pragma unroll
+      for (int t = 0; t < kMlpCols; ++t) put(relu(h[t]), H2[t][mt / 2], mt % 2);
+    }
+    // logits: slots 4g + j of point r
+    f32x4 z[kMlpCols];
+#pragma unroll
+    for (int t = 0; t < kMlpCols; ++t) z[t] = bias4(2 * kHid);
+#pragma unroll
+    for (int c = 0; c < kHid / kKT; ++c) {
+      bf16x8 const w = frag(kF3, c);
+#pragma unroll
+      for (int t = 0; t < kMlpCols; ++t) z[t] = mfma32(w, H2[t][c], z[t]);
+    }
+    if constexpr (!TRAIN) {
+#pragma unroll
+      for (int t = 0; t < kMlpCols; ++t) {
+        int64_t const p = base + 16 * t + r;
+        if (p < a.n)
+          for (int j = 0; j < 4; ++j) a.Z[p * kCand + 4 * g + j] = z[t][j];
+      }
+      __syncthreads();  // the next tile's weights overwrite W
+    } else {
+      __syncthreads();
+      stage(kB2, kBackward / 512);  // lands during the loss
+      // Masked softmax cross-entropy over the first count[cell] slots; the four lanes
+      // of a point (g = 0..3) hold four slots each. A row whose label is negative or
+      // outside the mask contributes nothing. dZ = (p - onehot) * scale.
+      bf16x4 dz[kMlpCols];
+#pragma unroll
+      for (int t = 0; t < kMlpCols; ++t) {
+        int64_t const p = base + 16 * t + r;
+        int const cnt   = p < a.n ? (a.g.count[cell[t]] < kCand ? a.g.count[cell[t]] : kCand) : 0;
+        int const y     = p < a.n ? a.labels[p] : -1;
+        bool const use  = y >= 0 && y < cnt;
+        float mx = -INFINITY;
+        int best = 0;
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          if (4 * g + j < cnt && z[t][j] > mx) {
+            mx   = z[t][j];
+            best = 4 * g + j;
+          }
+#pragma unroll
+        for (int o = 16; o < kWave; o <<= 1) {
+          float const om = __shfl_xor(mx, o, kWave);
+          int const ob   = __shfl_xor(best, o, kWave);
+          if (om > mx || (om == mx && ob < best)) {
+            mx   = om;
+            best = ob;
+          }
+        }
+        float e[4], sum = 0.f, zy = 0.f;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          e[j] = 4 * g + j < cnt ? expf(z[t][j] - mx) : 0.f;
+          sum += e[j];
+          if (4 * g + j == y) zy = z[t][j];
+        }
+#pragma unroll
+        for (int o = 16; o < kWave; o <<= 1) {
+          sum += __shfl_xor(sum, o, kWave);
+          zy += __shfl_xor(zy, o, kWave);  // the other lanes of the point hold 0
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          float const q = 4 * g + j < cnt ? e[j] / sum : 0.f;
+          dz[t][j] = use ? static_cast<short>(
+                             to_bf16((q - (4 * g + j == y ? 1.f : 0.f)) * a.scale))
+                         : short{0};
+        }
+        if (use && g == 0) {
+          loss += logf(sum) - (zy - mx);
+          correct += best == y ? 1.f : 0.f;
+          labelled += 1.f;
+        }
+      }
+      // slot 0: H2, slot 1: dZ
+#pragma unroll
+      for (int t = 0; t < kMlpCols; ++t) {
+#pragma unroll
+        for (int c = 0; c < kHid / kKT; ++c) store_rows(0, t, c, H2[t][c]);
+        uint16_t* row = T[1] + 4 * g * kTPitch + (wave * kMlpCols + t) * 16 + r;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) row[j * kTPitch] = static_cast<uint16_t>(dz[t][j]);
+      }
+      staged();
+      // dH2 = (W3^T dZ) where H2 > 0
+      auto gated = [](f32x4 d, bf16x8 h, int half) {
+        f32x4 o;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) o[j] = static_cast<float>(h[4 * half + j]) > 0.f ? d[j] : 0.f;
+        return o;
+      };
+      bf16x8 D2[kMlpCols][kHid / kKT];
+#pragma unroll
+      for (int mt = 0; mt < kHid / 16; ++mt) {
+        bf16x4 const w =
+          *reinterpret_cast<bf16x4 const*>(W + kB3 - kB2 + (mt * kWave + l) * 4);
+#pragma unroll
+        for (int t = 0; t < kMlpCols; ++t)
+          put(gated(mfma16(w, dz[t], zero), H2[t][mt / 2], mt % 2), D2[t][mt / 2], mt % 2);
+      }
+#pragma unroll
+      for (int ks = 0; ks < kMlpTile / 32; ++ks) {
+        bf16x8 const d = rows(1, 0, ks);
+#pragma unroll
+        for (int m = 0; m < 2; ++m) dw3[m] = mfma32(d, rows(0, 2 * wave + m, ks), dw3[m]);
+        if (wave == 0) db3 = mfma32(d, ones, db3);
+      }
+      __syncthreads();
+      // slot 0: H1, slot 1: dH2
+#pragma unroll
+      for (int t = 0; t < kMlpCols; ++t)
+#pragma unroll
+        for (int c = 0; c < kHid / kKT; ++c) {
+          store_rows(0, t, c, H1[t][c]);
+          store_rows(1, t, c, D2[t][c]);
+        }
+        // dH1 = (W2^T dH2) where H1 > 0
+      bf16x8 D1[kMlpCols][kHid / kKT];
+#pragma unroll
+      for (int mt = 0; mt < kHid / 16; ++mt) {
+        f32x4 d[kMlpCols];
+#pragma unroll
+        for (int t = 0; t < kMlpCols; ++t) d[t] = zero;
+#pragma unroll
+        for (int c = 0; c < kHid / kKT; ++c) {
+          bf16x8 const w = frag(0, mt * (kHid / kKT) + c);
+#pragma unroll
+          for (int t = 0; t < kMlpCols; ++t) d[t] = mfma32(w, D2[t][c], d[t]);
+        }
+#pragma unroll
+        for (int t = 0; t < kMlpCols; ++t)
+          put(gated(d[t], H1[t][mt / 2], mt % 2), D1[t][mt / 2], mt % 2);
+      }
+      __syncthreads();
+#pragma unroll
+      for (int ks = 0; ks < kMlpTile / 32; ++ks) {
+        bf16x8 d[2];
+#pragma unroll
+        for (int m = 0; m < 2; ++m) {
+          d[m]   = rows(1, 2 * wave + m, ks);
+          db2[m] = mfma32(d[m], ones, db2[m]);
+        }
+#pragma unroll
+        for (int k = 0; k < kHid / 16; ++k) {
+          bf16x8 const h = rows(0, k, ks);
+#pragma unroll
+          for (int m = 0; m < 2; ++m) dw2[m][k] = mfma32(d[m], h, dw2[m][k]);
+        }
+      }
+      __syncthreads();
+      // slot 0: X (natural order: features 32c + 8g + j), slot 1: dH1
+#pragma unroll
+      for (int t = 0; t < kMlpCols; ++t) {
+#pragma unroll
+        for (int c = 0; c < kHid / kKT; ++c) store_rows(1, t, c, D1[t][c]);
+#pragma unroll
+        for (int c = 0; c < kIn / kKT; ++c) {
+          uint16_t* row = T[0] + (32 * c + 8 * g) * kTPitch + (wave * kMlpCols + t) * 16 + r;
+          u16x8 const w = __builtin_bit_cast(u16x8, X[t][c]);
+#pragma unroll
+          for (int j = 0; j < 8; ++j) row[j * kTPitch] = w[j];
+        }
+      }
+        // embedding gradient: dX = W1^T dH1 (the embedding's inputs), rows 16 mt + 4g + j
+      f32x4 dx[kMlpCols][kEmb / 16];
+#pragma unroll
+      for (int mt = 0; mt < kEmb / 16; ++mt) {
+#pragma unroll
+        for (int t = 0; t < kMlpCols; ++t) dx[t][mt] = zero;
+#pragma unroll
+        for (int c = 0; c < kHid / kKT; ++c) {
+          bf16x8 const w = frag(kB1 - kB2, mt * (kHid / kKT) + c);
+#pragma unroll
+          for (int t = 0; t < kMlpCols; ++t) dx[t][mt] = mfma32(w, D1[t][c], dx[t][mt]);
+        }
+      }
+      __syncthreads();
+#pragma unroll
+      for (int ks = 0; ks < kMlpTile / 32; ++ks) {
+        bf16x8 d[2];
+#pragma unroll
+        for (int m = 0; m < 2; ++m) {
+          d[m]   = rows(1, 2 * wave + m, ks);
+          db1[m] = mfma32(d[m], ones, db1[m]);
+        }
+#pragma unroll
+        for (int k = 0; k < kIn / 16; ++k) {
+          bf16x8 const x = rows(0, k, ks);
+#pragma unroll
+          for (int m = 0; m < 2; ++m) dw1[m][k] = mfma32(d[m], x, dw1[m][k]);
+        }
+      }
+      __syncthreads();
+      // Through this wave's quarter of the slots, so that an atomic instruction adds one
+      // point's 64 consecutive values (from the tile layout an instruction touched 16
+      // points' lines for 16 bytes each, and the batch took 19 us more); after the last
+      // barrier, which would wait for them.
+      float* const row0 = reinterpret_cast<float*>(&T[0][0]) + wave * (kMlpCols * 16 * kDxPitch);
+#pragma unroll
+      for (int t = 0; t < kMlpCols; ++t)
+#pragma unroll
+        for (int mt = 0; mt < kEmb / 16; ++mt)
+          *reinterpret_cast<f32x4*>(row0 + (16 * t + r) * kDxPitch + 16 * mt + 4 * g) = dx[t][mt];
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+      for (int t = 0; t < kMlpCols; ++t)
+#pragma unroll 4
+        for (int q = 0; q < 16; ++q) {
+          if (base + 16 * t + q >= a.n) break;
+          uint32_t const c = __builtin_amdgcn_readlane(cell[t], q);
+          atomicAdd(a.gE + static_cast<int64_t>(c) * kEmb + l, row0[(16 * t + q) * kDxPitch + l]);
+        }
+      __syncthreads();  // the next tile's rows overwrite the slots
+    }
+  }
+  if constexpr (TRAIN) {
+    // this workgroup's share, in the parameters' order from w1 on
+    float* o          = a.partials + static_cast<int64_t>(blockIdx.x) * kTail;
+    float* const o_b1 = o + kHid * kIn;
+    float* const o_w2 = o_b1 + kHid;
+    float* const o_b2 = o_w2 + kHid * kHid;
+    float* const o_w3 = o_b2 + kHid;
+    float* const o_b3 = o_w3 + kCand * kHid;
+#pragma unroll
+    for (int m = 0; m < 2; ++m)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        int const row = 16 * (2 * wave + m) + 4 * g + j;
+#pragma unroll
+        for (int k = 0; k < kIn / 16; ++k) o[row * kIn + 16 * k + r] = dw1[m][k][j];
+#pragma unroll
+        for (int k = 0; k < kHid / 16; ++k) o_w2[row * kHid + 16 * k + r] = dw2[m][k][j];
+        o_w3[(4 * g + j) * kHid + 16 * (2 * wave + m) + r] = dw3[m][j];
+        if (r == 0) {
+          o_b1[row] = db1[m][j];
+          o_b2[row] = db2[m][j];
+          if (wave == 0 && m == 0) o_b3[4 * g + j] = db3[j];
+        }
+      }
+    loss     = wave_sum(loss);
+    correct  = wave_sum(correct);
+    labelled = wave_sum(labelled);
+    if (l == 0) {
+      atomicAdd(s_stats + 0, loss);
+      atomicAdd(s_stats + 1, correct);
+      atomicAdd(s_stats + 2, labelled);
+    }
+    __syncthreads();
+    if (threadIdx.x < 3) atomicAdd(a.stats + threadIdx.x, s_stats[threadIdx.x]);
+  }
+}
+
+// out[i] = sum over the workgroups' shares, in their order within each of four
+// threads (16 bytes per load, eight loads in flight), then over the four.
+__global__ void __launch_bounds__(256)
+  mlp_reduce_kernel(float const* __restrict__ partials, int count, float* __restrict__ out)
+{
+  __shared__ float4 part[3][kWave];
+  int const q = threadIdx.x / kWave, l = threadIdx.x % kWave;
+  int const i = static_cast<int>(blockIdx.x) * kWave + l;  // float4 index
+  float4 s    = make_float4(0.f, 0.f, 0.f, 0.f);
+  if (i < kTail / 4) {
+    float4 const* p = reinterpret_cast<float4 const*>(partials) + i;
+#pragma unroll 8
+    for (int b = q; b < count; b += 4) {
+      float4 const v = p[static_cast<int64_t>(b) * (kTail / 4)];
+      s.x += v.x, s.y += v.y, s.z += v.z, s.w += v.w;
+    }
+  }
+  if (q > 0) part[q - 1][l] = s;
+  __syncthreads();
+  if (q == 0 && i < kTail / 4) {
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      float4 const v = part[k][l];
+      s.x += v.x, s.y += v.y, s.z += v.z, s.w += v.w;
+    }
+    float const v[4] = {s.x, s.y, s.z, s.w};
+    for (int j = 0; j < 4; ++j) out[4 * i + j] = v[j];
+  }
 }
 
 // ---------------------------------------------------------------------------------
 // Locator: MLP on MFMA + exact test in predicted order
 // ---------------------------------------------------------------------------------
 constexpr int kLocTiles   = 4;  // 16-point tiles per wave round: 64 points, one per lane
-constexpr int kKT         = 32;  // K per v_mfma_f32_16x16x32_bf16
 constexpr int kW1Frags    = (kHid / 16) * (kIn / kKT);    // 24
 constexpr int kW2Frags    = (kHid / 16) * (kHid / kKT);   // 32
 constexpr int kW3Frags    = (kCand / 16) * (kHid / kKT);  // 4
@@ -444,37 +844,11 @@ __device__ __forceinline__ void exact_test(PolyView const& P, uint32_t poly, dou
   near_out   = near;
 }
 
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-typedef short s16x2 __attribute__((ext_vector_type(2)));
-typedef float f32x2 __attribute__((ext_vector_type(2)));
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-
-// D = A B + C on one 16x16x32 bf16 tile (gfx950). Lane l supplies
-// A[l % 16][8 (l / 16) + j] and B[8 (l / 16) + j][l % 16] (j = 0..7) and holds
-// D[4 (l / 16) + j][l % 16] (j = 0..3).
-__device__ __forceinline__ f32x4 mfma32(bf16x8 a, bf16x8 b, f32x4 c)
-{
-  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
-}
-
 __device__ __forceinline__ bf16x8 load_frag(uint16_t const* lds, int frag, int lane)
 {
   return *reinterpret_cast<bf16x8 const*>(lds +
                                           (static_cast<int64_t>(frag) * kWave + lane) * kFragElems);
 }
-
-// Input column of k-slot j of K tile c for lane group g of a layer fed by the
-// previous layer's output tiles: the B operand of that tile is output tiles 2c
-// (slots 0..3: rows 4g + j) and 2c + 1 (slots 4..7: rows 16 + 4g + j - 4), so the
-// weights of slot j sit in that column. The first layer's input is in natural
-// order (32c + 8g + j).
-__host__ __device__ __forceinline__ int chained_col(int c, int g, int j)
-{
-  return 32 * c + (j < 4 ? 4 * g + j : 16 + 4 * g + (j - 4));
-}
-
-__device__ __forceinline__ __bf16 bf(float f) { return static_cast<__bf16>(f); }
 
 // Two waves per SIMD (at most 256 registers, which also keeps the accumulators in
 // VGPRs: no AGPR copies before the bf16 conversions), as many as two workgroups'
@@ -730,65 +1104,25 @@ void check_model(qpip_ranker const* m, qpip_grid const* g)
                "ranker embedding count must equal the grid's cell count");
 }
 
-void launch_gemm(GemmArgs const& a, hipStream_t stream)
+// Packed weights of one call, and with gE (cells x 64 floats) its zero fill.
+void mlp_prepare(qpip_ranker const* m, Layout const& lay, uint16_t* packed, float* gE,
+                 hipStream_t stream)
 {
-  int64_t const waves = (a.M / 16) * (a.N / 16) * ((a.K + a.kchunk - 1) / a.kchunk);
-  if (waves == 0) return;
-  gemm_kernel<<<grid_for(static_cast<uint64_t>(waves), 256 / kWave, 1u << 30), 256, 0, stream>>>(a);
+  int64_t const n    = gE ? lay.w1 : 0;
+  unsigned const fill = gE ? grid_for(static_cast<uint64_t>(n), 256 * 4, 2048) : 0u;
+  mlp_prepare_kernel<<<kPackBlocks + fill, 256, 0, stream>>>(
+    m->params_bf16, lay, packed, gE, n, reinterpret_cast<uintptr_t>(gE) % 16 == 0);
   QPIP_LAUNCH_CHECK();
 }
 
-GemmArgs gemm(uint16_t const* A, int64_t a_m, int64_t a_k, uint16_t const* B, int64_t b_k,
-              int64_t b_n, int64_t M, int64_t N, int64_t K)
+MlpArgs mlp_args(qpip_ranker const* m, GridView const& g, Layout const& lay,
+                 uint16_t const* packed, double const* xy, int64_t n)
 {
-  GemmArgs a{};
-  a.A = A, a.a_m = a_m, a.a_k = a_k, a.B = B, a.b_k = b_k, a.b_n = b_n;
-  a.M = M, a.N = N, a.K = K, a.kchunk = ((K + 15) / 16) * 16;
+  MlpArgs a{};
+  a.g = g, a.emb = m->params_bf16 + lay.e, a.packed = packed, a.p = m->params, a.lay = lay;
+  a.xy = xy, a.n = n, a.tiles = (n + kMlpTile - 1) / kMlpTile;
   return a;
 }
-
-void fill_f32(float* p, int64_t n, float v, hipStream_t stream)
-{
-  if (n <= 0) return;
-  fill_f32_kernel<<<grid_for(static_cast<uint64_t>(n), 256, 1u << 30), 256, 0, stream>>>(p, n, v);
-  QPIP_LAUNCH_CHECK();
-}
-
-// Forward pass of `rows` (multiple of 16, >= n) rows; fills X, cells, H1, H2, Z.
-struct Activations {
-  dbuf<uint16_t> X, H1, H2;
-  dbuf<uint32_t> cells;
-  dbuf<float> Z;
-  explicit Activations(int64_t rows)
-    : X(rows * kIn), H1(rows * kHid), H2(rows * kHid), cells(rows), Z(rows * kCand)
-  {
-  }
-};
-
-void forward(qpip_ranker const* m, GridView const& g, double const* xy, int64_t n, int64_t rows,
-             Activations& act, hipStream_t stream)
-{
-  Layout const lay(m->num_cells);
-  uint16_t const* pb = m->params_bf16;
-  {
-    KernelTimer kt("ranker_features", stream);
-    features_kernel<<<grid_for(static_cast<uint64_t>(rows), 256, 1u << 30), 256, 0, stream>>>(
-      g, pb + lay.e, xy, n, rows, act.X.get(), act.cells.get());
-    QPIP_LAUNCH_CHECK();
-  }
-  KernelTimer kt("ranker_forward", stream);
-  GemmArgs l1 = gemm(act.X.get(), kIn, 1, pb + lay.w1, 1, kIn, rows, kHid, kIn);
-  l1.bias = m->params + lay.b1, l1.relu = 1, l1.Cb = act.H1.get(), l1.cb_m = kHid, l1.cb_n = 1;
-  launch_gemm(l1, stream);
-  GemmArgs l2 = gemm(act.H1.get(), kHid, 1, pb + lay.w2, 1, kHid, rows, kHid, kHid);
-  l2.bias = m->params + lay.b2, l2.relu = 1, l2.Cb = act.H2.get(), l2.cb_m = kHid, l2.cb_n = 1;
-  launch_gemm(l2, stream);
-  GemmArgs l3 = gemm(act.H2.get(), kHid, 1, pb + lay.w3, 1, kHid, rows, kCand, kHid);
-  l3.bias = m->params + lay.b3, l3.C = act.Z.get(), l3.c_m = kCand, l3.c_n = 1;
-  launch_gemm(l3, stream);
-}
-
-int64_t round16(int64_t n) { return ((n + 15) / 16) * 16; }
 
 }  // namespace
 
@@ -838,11 +1172,15 @@ extern "C" int qpip_ranker_logits(const qpip_ranker* model,
     if (num_points == 0) return;
     auto stream        = static_cast<hipStream_t>(stream_);
     StreamScope scope(stream);
-    int64_t const rows = round16(num_points);
-    Activations act(rows);
-    forward(model, g, xy, num_points, rows, act, stream);
-    QPIP_HIP(hipMemcpyAsync(logits, act.Z.get(), num_points * kCand * sizeof(float),
-                            hipMemcpyDeviceToDevice, stream));
+    Layout const lay(model->num_cells);
+    dbuf<uint16_t> packed(kPack);
+    KernelTimer kt("ranker_forward", stream);
+    mlp_prepare(model, lay, packed.get(), nullptr, stream);
+    MlpArgs a = mlp_args(model, g, lay, packed.get(), xy, num_points);
+    a.Z       = logits;
+    mlp_kernel<false><<<grid_for(static_cast<uint64_t>(a.tiles), 1, 1u << 30),
+                        kMlpWaves * kWave, 0, stream>>>(a);
+    QPIP_LAUNCH_CHECK();
   });
 }
 
@@ -862,56 +1200,26 @@ extern "C" int qpip_ranker_gradients(const qpip_ranker* model,
     auto stream        = static_cast<hipStream_t>(stream_);
     StreamScope scope(stream);
     Layout const lay(model->num_cells);
-    uint16_t const* pb = model->params_bf16;
-    int64_t const rows = round16(num_points);
-    Activations act(rows);
-    forward(model, g, xy, num_points, rows, act, stream);
-    KernelTimer kt("ranker_backward", stream);
-    fill_f32(grad, lay.total, 0.f, stream);
-    dbuf<uint16_t> dZ(rows * kCand), dH2(rows * kHid), dH1(rows * kHid);
-    dbuf<float> dXe(rows * kEmb);
-    xent_kernel<<<grid_for(static_cast<uint64_t>(rows), 256, 1u << 30), 256, 0, stream>>>(
-      act.Z.get(), act.cells.get(), g.count, labels, num_points, rows,
-      1.f / static_cast<float>(num_points), dZ.get(), stats);
+    // One workgroup per CU at most: its weight gradients stay in registers over its
+    // tiles, and fewer shares are left to reduce.
+    int dev = 0, cus = 0;
+    QPIP_HIP(hipGetDevice(&dev));
+    QPIP_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+    dbuf<uint16_t> packed(kPack);
+    MlpArgs a            = mlp_args(model, g, lay, packed.get(), xy, num_points);
+    unsigned const wgs   = static_cast<unsigned>(std::min<int64_t>(a.tiles, cus));
+    dbuf<float> partials(static_cast<size_t>(wgs) * kTail);
+    a.labels   = labels;
+    a.scale    = 1.f / static_cast<float>(num_points);
+    a.gE       = grad + lay.e;
+    a.partials = partials.get();
+    a.stats    = stats;
+    KernelTimer kt("ranker_gradients", stream);
+    mlp_prepare(model, lay, packed.get(), a.gE, stream);
+    mlp_kernel<true><<<wgs, kMlpWaves * kWave, 0, stream>>>(a);
     QPIP_LAUNCH_CHECK();
-    int64_t const kc = 1024;
-    // dW3[o][k] = sum_i dZ[i][o] H2[i][k]
-    GemmArgs w3 = gemm(dZ.get(), 1, kCand, act.H2.get(), kHid, 1, kCand, kHid, rows);
-    w3.kchunk = kc, w3.atomic = 1, w3.C = grad + lay.w3, w3.c_m = kHid, w3.c_n = 1;
-    launch_gemm(w3, stream);
-    static_assert(256 % kCand == 0 && 256 % kHid == 0, "colsum_kernel needs cols | 256");
-    auto colsum_grid = [&](int cols) {
-      return static_cast<unsigned>((rows + colsum_rows_per_block(cols) - 1) /
-                                   colsum_rows_per_block(cols));
-    };
-    colsum_kernel<<<colsum_grid(kCand), 256, 0, stream>>>(dZ.get(), rows, kCand, grad + lay.b3);
-    QPIP_LAUNCH_CHECK();
-    // dH2 = (dZ W3) * (H2 > 0)
-    GemmArgs h2 = gemm(dZ.get(), kCand, 1, pb + lay.w3, kHid, 1, rows, kHid, kCand);
-    h2.gate = act.H2.get(), h2.g_m = kHid, h2.g_n = 1, h2.Cb = dH2.get(), h2.cb_m = kHid, h2.cb_n = 1;
-    launch_gemm(h2, stream);
-    // dW2[o][k] = sum_i dH2[i][o] H1[i][k]
-    GemmArgs w2 = gemm(dH2.get(), 1, kHid, act.H1.get(), kHid, 1, kHid, kHid, rows);
-    w2.kchunk = kc, w2.atomic = 1, w2.C = grad + lay.w2, w2.c_m = kHid, w2.c_n = 1;
-    launch_gemm(w2, stream);
-    colsum_kernel<<<colsum_grid(kHid), 256, 0, stream>>>(dH2.get(), rows, kHid, grad + lay.b2);
-    QPIP_LAUNCH_CHECK();
-    // dH1 = (dH2 W2) * (H1 > 0)
-    GemmArgs h1 = gemm(dH2.get(), kHid, 1, pb + lay.w2, kHid, 1, rows, kHid, kHid);
-    h1.gate = act.H1.get(), h1.g_m = kHid, h1.g_n = 1, h1.Cb = dH1.get(), h1.cb_m = kHid, h1.cb_n = 1;
-    launch_gemm(h1, stream);
-    // dW1[o][k] = sum_i dH1[i][o] X[i][k]
-    GemmArgs w1 = gemm(dH1.get(), 1, kHid, act.X.get(), kIn, 1, kHid, kIn, rows);
-    w1.kchunk = kc, w1.atomic = 1, w1.C = grad + lay.w1, w1.c_m = kIn, w1.c_n = 1;
-    launch_gemm(w1, stream);
-    colsum_kernel<<<colsum_grid(kHid), 256, 0, stream>>>(dH1.get(), rows, kHid, grad + lay.b1);
-    QPIP_LAUNCH_CHECK();
-    // dX[:, :64] = dH1 W1[:, :64], scattered into the cells' embeddings
-    GemmArgs xe = gemm(dH1.get(), kHid, 1, pb + lay.w1, kIn, 1, rows, kEmb, kHid);
-    xe.C = dXe.get(), xe.c_m = kEmb, xe.c_n = 1;
-    launch_gemm(xe, stream);
-    embed_grad_kernel<<<grid_for(static_cast<uint64_t>(num_points) * kEmb, 256, 1u << 30), 256, 0,
-                        stream>>>(dXe.get(), act.cells.get(), num_points, grad + lay.e);
+    mlp_reduce_kernel<<<(kTail / 4 + kWave - 1) / kWave, 256, 0, stream>>>(
+      partials.get(), static_cast<int>(wgs), grad + lay.w1);
     QPIP_LAUNCH_CHECK();
   });
 }

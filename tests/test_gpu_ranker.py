@@ -93,6 +93,36 @@ def test_gradients_match_oracle(env):
         assert relerr(g[o[a]:o[b]], go[o[a]:o[b]]) < 2e-2, (a, relerr(g[o[a]:o[b]], go[o[a]:o[b]]))
 
 
+@pytest.mark.parametrize("n", [1, 16, 127, 128, 129, 33000])
+def test_batch_sizes_match_oracle(env, n):
+    """Gradients and logits at the edges of the 128-point tiles (one point, a tile, one
+    less and one more) and with more tiles than workgroups. The oracle rounds to bf16
+    where the kernel does, so only fp32 accumulation order differs: the bar is the
+    other gradient tests'."""
+    torch, cs, ranker, rk, _ = env
+    _, P, grid, xy, x, y = voronoi(env, n, 150, 21, 16)
+    model = ranker.Ranker(grid.num_cells, seed=22)
+    rng = np.random.default_rng(n)
+    c = grid.counts.cpu().numpy().astype(np.int64)[grid.cells_of(xy).cpu().numpy()]
+    labels = np.where(rng.uniform(size=n) < 0.9, rng.integers(0, np.maximum(c, 1)), -1)
+    labels[0] = 0
+    grad, stats = model.gradients(grid, xy, torch.as_tensor(labels.astype(np.int32),
+                                                            device="cuda"))
+    g, st = grad.cpu().numpy(), stats.cpu().numpy()
+    X, cells = model.features(grid, xy)
+    Xg = rk.from_bf16_bits(X.cpu().numpy().view(np.uint16)).astype(np.float64)
+    p = model.params.cpu().numpy().astype(np.float64)
+    loss, go, so = rk.loss_and_grad(p, grid.num_cells, Xg, cells.cpu().numpy().astype(np.int64),
+                                    grid.counts.cpu().numpy(), labels)
+    assert st[2] == so["labelled"] and abs(st[0] - so["loss_sum"]) <= 1e-3 * so["loss_sum"] + 1e-6
+    o = rk.layout(grid.num_cells)
+    for a, b in (("e", "w1"), ("w1", "b1"), ("b1", "w2"), ("w2", "b2"), ("b2", "w3"),
+                 ("w3", "b3"), ("b3", "total")):
+        assert relerr(g[o[a]:o[b]], go[o[a]:o[b]]) < 2e-2, (a, relerr(g[o[a]:o[b]], go[o[a]:o[b]]))
+    zo = rk.forward(p, grid.num_cells, Xg)["Z"]
+    assert relerr(model.logits(grid, xy).cpu().numpy(), zo) < 2e-2
+
+
 def test_adam_step_matches_rule(env):
     torch, cs, ranker, rk, _ = env
     model = ranker.Ranker(16, seed=4)
