@@ -1134,8 +1134,7 @@ __global__ void clamp_count_kernel(uint64_t const* in, uint64_t cap, uint64_t* o
 
 // --- brute force: every point against every polygon ------------------------------
 // point_in_polygon (detail/point_in_polygon.cuh:42-102): bit j of the result of point
-// i is point i inside polygon j, for at most 31 polygons. One wave per 128 points
-// (2 per lane); each polygon's edges are wave-uniform, as in the quadtree test.
+// i is point i inside polygon j, for at most 31 polygons.
 __device__ __forceinline__ void load_point(PipArgs const& a, uint64_t i, double& px, double& py)
 {
   if (a.xy) {
@@ -1153,48 +1152,154 @@ __device__ __forceinline__ void load_point(PipArgs const& a, uint64_t i, double&
   }
 }
 
-__global__ void __launch_bounds__(256)
-  pip_bitmask_kernel(PipArgs a, uint64_t n, int32_t* __restrict__ out)
+// One wave holds up to kBmChunks chunks of 64 points in LDS and takes the polygons one
+// after the other: the points inside the polygon's vertex box (box_excludes, with the
+// wave's largest coordinate in place of the point's own: a wider margin, so it keeps
+// no fewer) queue up, and every 64 of them (and the rest, in lane groups) run over
+// the ring's edges. Random points against regions: a box holds a few percent of them,
+// so most (point, polygon) pairs cost four comparisons instead of the ring's edges.
+// What a polygon's test reads first (its box, ring range and first ring's entries)
+// is loaded once per workgroup, one polygon per thread, instead of as a chain of
+// dependent loads by every wave and polygon.
+// Bound by the edge steps (five FP64 instructions each, 40 cycles of a SIMD). 2,000,003
+// points, 31 polygons of 4 to 256 vertices, boxes of about a tenth of the square: every
+// point over every edge (two slots of 64 points) took 2020 us, this 620 us. Loading the
+// next polygon's first batch a polygon ahead with eight edges' LDS reads in flight
+// took 595 us for twice the vector registers, and is not done.
+constexpr int kBmChunks = 8;    // 64-point chunks per wave at most
+constexpr int kBmWaves  = 2;    // waves per workgroup
+constexpr int kBmStage  = 128;  // edges per staged batch
+constexpr int kBmPolys  = 31;
+
+struct BmPoly {
+  PolyBox box;
+  RingHint hint;
+};
+
+struct BmWave {
+  double2 p[kBmChunks * kWave];
+  uint32_t bits[kBmChunks * kWave];
+  uint16_t queue[2 * kWave];
+  PipStage<kBmStage> stage;
+};
+
+__device__ __forceinline__ double uniform_f64(double v)
 {
-  __shared__ PipStage<kStageEdges> s_stage[256 / kWave];
-  PipStage<kStageEdges>* const stage = &s_stage[threadIdx.x / kWave];
-  uint64_t const w  = static_cast<uint64_t>(blockIdx.x) * (blockDim.x / kWave) + threadIdx.x / kWave;
-  uint64_t const p0 = w * kSlots * kWave;
-  if (p0 >= n) return;
-  int const lane    = lane_id();
-  uint64_t const left = (n - p0 + kWave - 1) / kWave;
-  uint32_t const nu   = left < kSlots ? static_cast<uint32_t>(left) : kSlots;
-  double px[kSlots], py[kSlots];
-  uint64_t valid_m[kSlots];
-#pragma unroll
-  for (int u = 0; u < kSlots; ++u) {
-    uint64_t const i = p0 + static_cast<uint64_t>(u) * kWave + lane;
-    bool const valid = i < n;
-    px[u] = py[u] = 0.0;
-    if (valid) load_point(a, i, px[u], py[u]);
-    valid_m[u] = ballot(valid);
+  uint64_t const b = static_cast<uint64_t>(__double_as_longlong(v));
+  uint64_t const h = uniform(static_cast<uint32_t>(b >> 32));
+  return __longlong_as_double(static_cast<long long>((h << 32) | uniform(static_cast<uint32_t>(b))));
+}
+
+__global__ void __launch_bounds__(kBmWaves * kWave)
+  pip_bitmask_kernel(PipArgs a, uint64_t n, uint32_t chunks, int32_t* __restrict__ out)
+{
+  __shared__ BmPoly s_poly[kBmPolys];
+  __shared__ BmWave s_wave[kBmWaves];
+  for (uint32_t j = threadIdx.x; j < a.num_polys; j += kBmWaves * kWave) {
+    BmPoly r{a.poly_box[j], RingHint{a.poly_offsets[j], a.poly_offsets[j + 1], 0u, 0u, 0.0, 0.0}};
+    if (r.hint.r1 > a.num_rings) r.hint.r1 = static_cast<uint32_t>(a.num_rings);
+    if (r.hint.r0 < r.hint.r1) {
+      r.hint.e0   = a.ring_offsets[r.hint.r0];
+      r.hint.ne   = a.ring_edges[r.hint.r0];
+      r.hint.amax = a.ring_amax[r.hint.r0];
+      if (r.hint.ne > 0) r.hint.by0 = ring_last_y(a, r.hint.r0);
+    }
+    s_poly[j] = r;
   }
-  double const pmax = wave_max_abs(px, py, nu);
-  uint32_t bits[kSlots];
+  __syncthreads();
+  BmWave& s         = s_wave[threadIdx.x / kWave];
+  uint64_t const w  = static_cast<uint64_t>(blockIdx.x) * kBmWaves + threadIdx.x / kWave;
+  uint64_t const p0 = w * chunks * kWave;
+  if (p0 >= n) return;
+  int const lane      = lane_id();
+  uint64_t const left = (n - p0 + kWave - 1) / kWave;
+  uint32_t const nc   = uniform(left < chunks ? static_cast<uint32_t>(left) : chunks);
+  double pmax         = 0.0;
+  for (uint32_t c = 0; c < nc; ++c) {
+    uint64_t const i = p0 + c * kWave + lane;
+    double px = 0.0, py = 0.0;
+    if (i < n) load_point(a, i, px, py);
+    pmax                   = fmax(pmax, fmax(fabs(px), fabs(py)));
+    s.p[c * kWave + lane]    = make_double2(px, py);
+    s.bits[c * kWave + lane] = 0;
+  }
 #pragma unroll
-  for (int u = 0; u < kSlots; ++u) bits[u] = 0;
+  for (int o = kWave / 2; o > 0; o >>= 1) pmax = fmax(pmax, __shfl_xor(pmax, o, kWave));
+  pmax = uniform_f64(pmax);
+  auto fence = [] {  // the wave's LDS writes before its reads, and the other way round
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  };
+  fence();
   bool err = false;
   for (uint32_t j = 0; j < a.num_polys; ++j) {
-    uint64_t hit_m[kSlots];
-#pragma unroll
-    for (int u = 0; u < kSlots; ++u) hit_m[u] = 0;
-    if (nu == 1)
-      test_polygon<1>(a, j, px, py, valid_m, pmax, hit_m, err, stage);
-    else
-      test_polygon<2>(a, j, px, py, valid_m, pmax, hit_m, err, stage);
-#pragma unroll
-    for (int u = 0; u < kSlots; ++u) bits[u] |= static_cast<uint32_t>((hit_m[u] >> lane) & 1ull) << j;
+    BmPoly const& r = s_poly[j];
+    RingHint const rh{uniform(r.hint.r0), uniform(r.hint.r1), uniform(r.hint.e0),
+                      uniform(r.hint.ne), uniform_f64(r.hint.amax), uniform_f64(r.hint.by0)};
+    PolyBox const fb = r.box;
+    double const bm  = fmax(fmax(fabs(fb.minx), fabs(fb.maxx)), fmax(fabs(fb.miny), fabs(fb.maxy)));
+    double const s3  = pmax + pmax + bm;
+    double const inf = __builtin_inf();
+    double const d   = s3 < 0x1p402 ? fma(s3, 0x1p-48, 0x1p-300) : inf;
+    double const x0 = fb.minx - d, x1 = fb.maxx + d;  // an empty box may give NaN: keeps all
+    uint32_t qn = 0;
+    auto flush = [&](uint32_t q) {  // the first q queued points
+      uint32_t const g    = q > 1 ? 32u - static_cast<uint32_t>(__builtin_clz(q - 1)) : 0u;
+      uint32_t const src  = static_cast<uint32_t>(lane) & ((1u << g) - 1u);  // 2^g >= q lanes
+      uint32_t const slot = s.queue[src < q ? src : 0];
+      double2 const pt    = s.p[slot];
+      double px[kSlots] = {pt.x, 0.0}, py[kSlots] = {pt.y, 0.0};
+      uint64_t hit_m[kSlots] = {0, 0};
+      uint64_t const test_m[kSlots] = {q >= kWave ? ~0ull : ((1ull << q) - 1ull), 0};
+      test_polygon<1, kBmStage>(a, j, px, py, test_m, pmax, hit_m, err, &s.stage, 6u - g, &rh);
+      if ((hit_m[0] >> lane) & 1ull) s.bits[slot] |= 1u << j;
+    };
+    for (uint32_t c = 0; c < nc; ++c) {
+      double2 const pt = s.p[c * kWave + lane];
+      bool const keep  = p0 + c * kWave + lane < n &&
+                        !(pt.y < fb.miny || pt.y > fb.maxy || pt.x < x0 || pt.x > x1);
+      uint64_t const km = ballot(keep);
+      if (km == 0) continue;
+      fence();
+      if (keep)
+        s.queue[qn + static_cast<uint32_t>(__popcll(km & lanemask_lt()))] =
+          static_cast<uint16_t>(c * kWave + lane);
+      fence();
+      qn += static_cast<uint32_t>(__popcll(km));
+      if (qn < kWave) continue;
+      flush(kWave);
+      fence();
+      uint16_t const rest = s.queue[kWave + lane];
+      fence();
+      s.queue[lane] = rest;
+      qn -= kWave;
+    }
+    if (qn > 0) {
+      fence();
+      flush(qn);
+    }
   }
-#pragma unroll
-  for (int u = 0; u < kSlots; ++u) {
-    uint64_t const i = p0 + static_cast<uint64_t>(u) * kWave + lane;
-    if (i < n) out[i] = static_cast<int32_t>(bits[u]);
+  fence();
+  for (uint32_t c = 0; c < nc; ++c) {
+    uint64_t const i = p0 + c * kWave + lane;
+    if (i < n) out[i] = static_cast<int32_t>(s.bits[c * kWave + lane]);
   }
+}
+
+// Enqueues the test of n points against a.num_polys <= 31 polygons. Chunks per wave:
+// as many as leave 4,096 waves (four per SIMD), since the more points a wave holds
+// the fuller its queue's flushes are.
+void launch_bitmask(PipArgs const& a, uint64_t n, int32_t* out, hipStream_t stream)
+{
+  KernelTimer kt("pip_bitmask", stream);
+  uint64_t const all = (n + kWave - 1) / kWave;
+  uint32_t const chunks =
+    static_cast<uint32_t>(std::min<uint64_t>(kBmChunks, std::max<uint64_t>(1, all / 4096)));
+  uint64_t const per = uint64_t{chunks} * kWave * kBmWaves;
+  pip_bitmask_kernel<<<static_cast<unsigned>((n + per - 1) / per), kBmWaves * kWave, 0, stream>>>(
+    a, n, chunks, out);
+  QPIP_LAUNCH_CHECK();
 }
 
 // pairwise_point_in_polygon (detail/point_in_polygon.cuh:104-160): point i against
@@ -1568,12 +1673,21 @@ int point_in_polygon_entry(const double* x,
     dbuf<uint32_t> ring_edges(std::max<uint64_t>(num_rings, 1));
     dbuf<LineEdge> lines(pairwise ? 1 : std::max<int64_t>(num_poly_x, 1));
     dbuf<double> ring_amax(pairwise ? 1 : std::max<uint64_t>(num_rings, 1));
+    dbuf<PolyBox> ring_box(pairwise ? 1 : std::max<uint64_t>(num_rings, 1));
+    dbuf<PolyBox> poly_box(pairwise ? 1 : std::max<int64_t>(num_polys, 1));
     if (num_rings > 0) {
       KernelTimer kt("pip_edges", stream);
       build_edges_kernel<<<grid_for(num_rings, 256 / kWave), 256, 0, stream>>>(
         reinterpret_cast<uint32_t const*>(ring_offsets), static_cast<int64_t>(num_rings), poly_x,
         poly_y, num_poly_x, nullptr, nullptr, ring_edges.get(),
-        pairwise ? nullptr : lines.get(), pairwise ? nullptr : ring_amax.get(), nullptr);
+        pairwise ? nullptr : lines.get(), pairwise ? nullptr : ring_amax.get(),
+        pairwise ? nullptr : ring_box.get());
+      QPIP_LAUNCH_CHECK();
+    }
+    if (!pairwise && num_polys > 0) {
+      poly_box_kernel<<<1, 256, 0, stream>>>(
+        reinterpret_cast<uint32_t const*>(poly_offsets), static_cast<uint64_t>(num_polys),
+        num_rings, ring_box.get(), poly_box.get());
       QPIP_LAUNCH_CHECK();
     }
     PipArgs a{};
@@ -1592,6 +1706,7 @@ int point_in_polygon_entry(const double* x,
     a.num_vertices = static_cast<uint64_t>(num_poly_x);
     a.lines        = lines.get();
     a.ring_amax    = ring_amax.get();
+    a.poly_box     = poly_box.get();
     OutputAllocator oa(mr, stream);
     if (pairwise) {
       uint8_t* out = oa.make<uint8_t>(n);
@@ -1601,10 +1716,7 @@ int point_in_polygon_entry(const double* x,
       *result = out;
     } else {
       int32_t* out = oa.make<int32_t>(n);
-      KernelTimer kt("pip_bitmask", stream);
-      uint64_t const waves = (n + kSlots * kWave - 1) / (kSlots * kWave);
-      pip_bitmask_kernel<<<static_cast<unsigned>((waves + 3) / 4), 256, 0, stream>>>(a, n, out);
-      QPIP_LAUNCH_CHECK();
+      launch_bitmask(a, n, out, stream);
       *result = out;
     }
     oa.keep();
@@ -1666,19 +1778,22 @@ extern "C" int qpip_pairwise_point_in_polygon(const double* x,
 // --- allocation-free bitmask point-in-polygon ---------------------------------------
 // qpip_point_in_polygon_noalloc runs the kernels of qpip_point_in_polygon with the
 // edge table in `scratch`, a fixed device array of this file, instead of pool
-// memory: the edges' line forms (32 B per vertex) and each ring's largest
-// |coordinate| and edge count (12 B per ring); the exact retest reads the caller's
-// vertices. 8.75 MiB per device, held by every device the library runs on until
-// the process ends.
+// memory: the edges' line forms (32 B per vertex), each ring's box, largest
+// |coordinate| and edge count (44 B per ring) and the polygons' boxes; the exact
+// retest reads the caller's vertices. 10.75 MiB per device, held by every device the
+// library runs on until the process ends.
 namespace {
 
 constexpr size_t kNoAllocLinesOff  = 0;
 constexpr size_t kNoAllocAmaxOff   = kNoAllocLinesOff + sizeof(qpip::LineEdge) * QPIP_NOALLOC_MAX_VERTICES;
 constexpr size_t kNoAllocRingsOff  = kNoAllocAmaxOff + sizeof(double) * QPIP_NOALLOC_MAX_RINGS;
-constexpr size_t kNoAllocBytes     = kNoAllocRingsOff + sizeof(uint32_t) * QPIP_NOALLOC_MAX_RINGS;
+constexpr size_t kNoAllocBoxOff    = kNoAllocRingsOff + sizeof(uint32_t) * QPIP_NOALLOC_MAX_RINGS;
+constexpr size_t kNoAllocPolyOff   = kNoAllocBoxOff + sizeof(qpip::PolyBox) * QPIP_NOALLOC_MAX_RINGS;
+constexpr size_t kNoAllocBytes     = kNoAllocPolyOff + sizeof(qpip::PolyBox) * 32;
 static_assert(kNoAllocLinesOff % alignof(qpip::LineEdge) == 0 && kNoAllocAmaxOff % 8 == 0,
               "scratch layout");
-static_assert(kNoAllocRingsOff % 4 == 0, "scratch carving keeps each table aligned");
+static_assert(kNoAllocRingsOff % 4 == 0 && kNoAllocBoxOff % alignof(qpip::PolyBox) == 0,
+              "scratch carving keeps each table aligned");
 
 static __device__ __align__(256) unsigned char scratch[kNoAllocBytes];
 
@@ -1743,13 +1858,21 @@ extern "C" int qpip_point_in_polygon_noalloc(const double* x,
     uint32_t* const ring_edges = reinterpret_cast<uint32_t*>(base + kNoAllocRingsOff);
     LineEdge* const lines      = reinterpret_cast<LineEdge*>(base + kNoAllocLinesOff);
     double* const ring_amax    = reinterpret_cast<double*>(base + kNoAllocAmaxOff);
+    PolyBox* const ring_box    = reinterpret_cast<PolyBox*>(base + kNoAllocBoxOff);
+    PolyBox* const poly_box    = reinterpret_cast<PolyBox*>(base + kNoAllocPolyOff);
     // Every ring's entry and every edge a ring keeps are written below before the
     // test reads them; the test reads nothing else of the scratch, so nothing a
     // previous call left there needs clearing.
     if (num_rings > 0) {
       build_edges_kernel<<<grid_for(num_rings, 256 / kWave), 256, 0, stream>>>(
         reinterpret_cast<uint32_t const*>(ring_offsets), static_cast<int64_t>(num_rings), poly_x,
-        poly_y, num_poly_x, nullptr, nullptr, ring_edges, lines, ring_amax, nullptr);
+        poly_y, num_poly_x, nullptr, nullptr, ring_edges, lines, ring_amax, ring_box);
+      QPIP_LAUNCH_CHECK();
+    }
+    if (num_polys > 0) {
+      poly_box_kernel<<<1, 256, 0, stream>>>(
+        reinterpret_cast<uint32_t const*>(poly_offsets), static_cast<uint64_t>(num_polys),
+        num_rings, ring_box, poly_box);
       QPIP_LAUNCH_CHECK();
     }
     uint64_t const n = static_cast<uint64_t>(num_x);
@@ -1767,9 +1890,8 @@ extern "C" int qpip_point_in_polygon_noalloc(const double* x,
     a.num_vertices = static_cast<uint64_t>(num_poly_x);
     a.lines        = lines;
     a.ring_amax    = ring_amax;
-    uint64_t const waves = (n + kSlots * kWave - 1) / (kSlots * kWave);
-    pip_bitmask_kernel<<<static_cast<unsigned>((waves + 3) / 4), 256, 0, stream>>>(a, n, result);
-    QPIP_LAUNCH_CHECK();
+    a.poly_box     = poly_box;
+    launch_bitmask(a, n, result, stream);
     return QPIP_SUCCESS;
   } catch (...) {
     return qpip::error_status();

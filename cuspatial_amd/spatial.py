@@ -377,10 +377,16 @@ def point_in_polygon(points: Points, polygons: Polygons):
     if len(polygons) == 0:
         return Table()
     bits = _brute_force(points, polygons, pairwise=False)
-    out = Table()
-    for j in range(len(polygons)):
-        out[j] = ((bits >> j) & 1).to(torch.bool)
-    return out
+    # Byte plane k holds bits 8k .. 8k + 7 of every point; eight points' bytes per
+    # word, one shift and one mask turn a plane into its eight columns of 0 / 1 bytes.
+    n = bits.numel()
+    planes = torch.empty((4, (n + 255) // 256 * 256), dtype=torch.uint8, device=bits.device)
+    planes[:, :n] = bits.view(torch.uint8).view(n, 4).t()
+    shifts = torch.arange(8, device=bits.device)
+    words = planes.view(torch.int64)[:, None, :] >> shifts[None, :, None]
+    words &= 0x0101010101010101
+    table = words.view(32, -1).view(torch.bool)
+    return Table((j, table[j, :n]) for j in range(len(polygons)))
 
 
 def point_in_polygon_bitmask(points: Points, polygons: Polygons) -> torch.Tensor:

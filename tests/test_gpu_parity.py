@@ -514,6 +514,43 @@ def test_point_in_polygon_bitmask_random(cs, oracle_mod, seed, n, npoly, layout)
         assert np.array_equal(np_(tbl[j]), ((ref >> j) & 1).astype(bool))
 
 
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 129, 600001, 2200003])
+def test_bitmask_box_filter_and_queue(cs, oracle_mod, n):
+    """The bitmask test's box filter and queue at the edges of its 64-point chunks and
+    at several and eight chunks per wave: small polygons (a few points per flush),
+    large ones (several flushes), long rings, a polygon without vertices, points a
+    ULP outside a box, NaN, infinite and huge coordinates. Exact."""
+    rng = np.random.default_rng(n)
+    parts = [star_polygons(rng, 20, 100.0, 0.5, 3.0, kmax=200, holes=0.3),
+             star_polygons(rng, 6, 100.0, 30.0, 60.0, kmin=100, kmax=300),
+             (np.array([0, 1, 1, 1], np.int32), np.array([0, 0], np.int32), np.zeros(0),
+              np.zeros(0))]
+    part, ring, vx, vy = [np.zeros(1, np.int32)], [np.zeros(1, np.int32)], [], []
+    for p, r, x, y in parts:
+        part.append(p[1:] + len(np.concatenate(ring)) - 1)
+        ring.append(r[1:] + sum(map(len, vx)))
+        vx.append(x)
+        vy.append(y)
+    part, ring, vx, vy = map(np.concatenate, (part, ring, vx, vy))
+    x, y = rng.uniform(-5, 105, n), rng.uniform(-5, 105, n)
+    k = min(n // 2, 400)
+    i = rng.integers(0, len(vx), k)
+    x[:k] = np.nextafter(vx[i], np.where(rng.uniform(size=k) < 0.5, -1e9, 1e9))
+    y[:k] = vy[i]
+    for m, v in enumerate((np.nan, np.inf, -np.inf, 1e130, -1e200)):
+        if k + 2 * m + 1 < n:
+            x[k + 2 * m] = v
+            y[k + 2 * m + 1] = v
+    ref = oracle_mod.point_in_polygon_bitmask(x, y, part, ring, vx, vy)
+    P = cs.Polygons(part.astype(np.int32), ring.astype(np.int32), vx, vy, device="cuda")
+    got = cs.point_in_polygon_bitmask(cs.Points(x, y, device="cuda"), P)
+    assert np.array_equal(np_(got).astype(np.int64), ref.astype(np.int64))
+    tbl = cs.point_in_polygon(cs.Points(x, y, device="cuda"), P)
+    assert tbl.columns == list(range(len(P)))
+    for j in range(len(P)):
+        assert len(tbl[j]) == n and np.array_equal(np_(tbl[j]), ((ref >> j) & 1).astype(bool))
+
+
 @pytest.mark.parametrize("seed,n", [(61, 1), (62, 5000), (63, 200001)])
 def test_pairwise_point_in_polygon_random(cs, oracle_mod, seed, n):
     rng = np.random.default_rng(seed)
