@@ -15,15 +15,17 @@
 // point in a paired leaf. The reference leaves the two index columns of the other
 // rows uninitialized (distance 0); here they are (p, 0xffffffff, 0).
 //
-// One wave per pair: the waves of a run (pairs on one leaf, adjacent in the
-// join's order, which sorts pairs by leaf offset) split the leaf's 64-point chunks
-// between them (chunk c goes to the
-// run's pair c mod R); each lane holds one point and folds over the run's
-// linestrings, whose vertices are wave-uniform.
+// The join sorts pairs by leaf offset, so the pairs on one leaf form a run. One wave
+// per 64-point chunk of a run's leaf (nearest_chunk_kernel) finds each point's nearest
+// linestring with a float32 distance in coordinates local to the chunk, and computes
+// the reference's double arithmetic for that linestring alone; points whose float32
+// distances do not decide fold over every linestring. Pairs that are not sorted, or
+// that put two quadrants on one offset, take nearest_kernel, which finds the run of
+// every pair as the reference does (lower and upper bound of its leaf's offset).
 #include <algorithm>
 #include <cmath>
 
-#include "qpip_internal.hpp"
+#include "qpip_scan.hpp"
 
 namespace qpip {
 
@@ -51,6 +53,10 @@ struct NearestArgs {
   uint32_t* bad;
 };
 
+// *bad: bit 1 an index out of range, bit 2 pairs that do not form runs of one leaf in
+// offset order (or more chunks than the work list holds): nearest_kernel runs then.
+constexpr uint32_t kBadIndex = 1u, kIrregular = 2u;
+
 template <class T>
 __device__ __forceinline__ T uniform_load(T const* p)
 {
@@ -76,28 +82,85 @@ __device__ __forceinline__ double dot2(double ax, double ay, double bx, double b
 // point_linestring_distance (detail/algorithm/point_linestring_distance.cuh:33-51):
 // min over the segments (v[i], v[i+1]) of the squared distance, then the square
 // root.
+// One segment's squared distance, folded into dsq.
+__device__ __forceinline__ double fold_segment(double dsq, double ax, double ay, double bx,
+                                               double by, double px, double py)
+{
+  double const v1x = px - ax, v1y = py - ay;
+  double const v2x = px - bx, v2y = py - by;
+  double const ex = bx - ax, ey = by - ay;
+  double const d0 = dot2(v1x, v1y, v1x, v1y);
+  double const d1 = dot2(v2x, v2y, v2x, v2y);
+  double const d2 = dot2(ex, ey, ex, ey);
+  double const d3 = dot2(v1x, v1y, ex, ey);
+  double const r  = d3 * d3 / d2;
+  double const d  = (d3 <= 0.0 || r >= d2) ? fmin(d0, d1) : d0 - r;
+  return fmin(dsq, d);
+}
+
+constexpr double kNoDistance = 1.7976931348623157e308;  // numeric_limits<double>::max()
+
+// The linestring is the same in every lane (its vertices are loaded once per wave).
 __device__ __forceinline__ double point_linestring_distance(NearestArgs const& a, uint32_t ls,
                                                             double px, double py)
 {
   uint64_t v0 = uniform_load(a.ls_offsets + ls);
   uint64_t v1 = uniform_load(a.ls_offsets + ls + 1);
   if (v1 > a.num_vertices) v1 = a.num_vertices;
-  double dsq = 1.7976931348623157e308;  // numeric_limits<double>::max()
-  for (uint64_t i = v0; i + 1 < v1; ++i) {
-    double const ax = uniform_d(a.lx + i), ay = uniform_d(a.ly + i);
-    double const bx = uniform_d(a.lx + i + 1), by = uniform_d(a.ly + i + 1);
-    double const v1x = px - ax, v1y = py - ay;
-    double const v2x = px - bx, v2y = py - by;
-    double const ex = bx - ax, ey = by - ay;
-    double const d0 = dot2(v1x, v1y, v1x, v1y);
-    double const d1 = dot2(v2x, v2y, v2x, v2y);
-    double const d2 = dot2(ex, ey, ex, ey);
-    double const d3 = dot2(v1x, v1y, ex, ey);
-    double const r  = d3 * d3 / d2;
-    double const d  = (d3 <= 0.0 || r >= d2) ? fmin(d0, d1) : d0 - r;
-    dsq             = fmin(dsq, d);
+  double dsq = kNoDistance;
+  for (uint64_t i = v0; i + 1 < v1; ++i)
+    dsq = fold_segment(dsq, uniform_d(a.lx + i), uniform_d(a.ly + i), uniform_d(a.lx + i + 1),
+                       uniform_d(a.ly + i + 1), px, py);
+  return sqrt(dsq);
+}
+
+// Each lane has its own linestring.
+__device__ __forceinline__ double own_linestring_distance(NearestArgs const& a, uint32_t ls,
+                                                          double px, double py)
+{
+  uint64_t v0 = a.ls_offsets[ls], v1 = a.ls_offsets[ls + 1];
+  if (v1 > a.num_vertices) v1 = a.num_vertices;
+  double dsq = kNoDistance;
+  if (v0 + 1 < v1) {
+    double ax = a.lx[v0], ay = a.ly[v0];
+    for (uint64_t i = v0 + 1; i < v1; ++i) {
+      double const bx = a.lx[i], by = a.ly[i];
+      dsq = fold_segment(dsq, ax, ay, bx, by, px, py);
+      ax  = bx;
+      ay  = by;
+    }
   }
   return sqrt(dsq);
+}
+
+// The reference's choice between the kept (linestring, distance) and the next pair's
+// (quadtree_point_to_nearest_linestring.cuh:279-294, lhs = kept, rhs = next).
+__device__ __forceinline__ bool take_next(double best_d, uint32_t best_ls, double d, uint32_t ls)
+{
+  if (best_d == 0.0) return true;
+  if (d == 0.0) return false;
+  if (best_d == d) return !(best_ls < ls);
+  return !(best_d < d);
+}
+
+// The fold over a run's pairs [rs, re), for every active lane.
+__device__ __forceinline__ void fold_run(NearestArgs const& a, uint64_t rs, uint64_t re, double px,
+                                         double py, uint32_t& best_ls, double& best_d, bool& err)
+{
+  best_ls = 0;
+  best_d  = 0.0;
+  for (uint64_t k = rs; k < re; ++k) {
+    uint32_t const ls = uniform_load(a.pair_ls + k);
+    if (ls >= a.num_ls) {
+      err = true;
+      continue;
+    }
+    double const d = point_linestring_distance(a, ls, px, py);
+    if (k == rs || take_next(best_d, best_ls, d, ls)) {
+      best_ls = ls;
+      best_d  = d;
+    }
+  }
 }
 
 __global__ void __launch_bounds__(256) nearest_fill_kernel(NearestArgs a)
@@ -118,7 +181,7 @@ __global__ void __launch_bounds__(256) nearest_kernel(NearestArgs a, uint64_t ba
   if (k0 >= a.num_pairs) return;
   uint32_t const quad = uniform_load(a.pair_quad + k0);
   if (quad >= a.num_nodes) {
-    if (lane_id() == 0) atomicOr(a.bad, 1u);
+    if (lane_id() == 0) atomicOr(a.bad, kBadIndex);
     return;
   }
   uint32_t const len   = uniform_load(a.length + quad);
@@ -164,36 +227,247 @@ __global__ void __launch_bounds__(256) nearest_kernel(NearestArgs a, uint64_t ba
       continue;
     }
     double const px = a.x[idx], py = a.y[idx];
-    uint32_t best_ls = 0;
-    double best_d    = 0.0;
-    for (uint64_t k = rs; k < re; ++k) {
-      uint32_t const ls = uniform_load(a.pair_ls + k);
-      if (ls >= a.num_ls) {
-        err = true;
-        continue;
-      }
-      double const d = point_linestring_distance(a, ls, px, py);
-      if (k == rs) {
-        best_ls = ls;
-        best_d  = d;
-        continue;
-      }
-      // quadtree_point_to_nearest_linestring.cuh:279-294, lhs = best, rhs = this pair
-      bool take_rhs;
-      if (best_d == 0.0) take_rhs = true;
-      else if (d == 0.0) take_rhs = false;
-      else if (best_d == d) take_rhs = !(best_ls < ls);
-      else take_rhs = !(best_d < d);
-      if (take_rhs) {
-        best_ls = ls;
-        best_d  = d;
-      }
-    }
+    uint32_t best_ls;
+    double best_d;
+    fold_run(a, rs, re, px, py, best_ls, best_d, err);
     a.out_point[pos] = static_cast<uint32_t>(pos);
     a.out_ls[pos]    = best_ls;
     a.out_dist[pos]  = best_d;
   }
-  if (err) atomicOr(a.bad, 1u);
+  if (err) atomicOr(a.bad, kBadIndex);
+}
+
+// Work list: the 64-point chunks of every run's leaf, as (first pair, chunk).
+struct RunChunkOp {
+  NearestArgs a;
+  uint2* items;
+  uint64_t cap;
+  __device__ __forceinline__ uint32_t off(uint64_t k, uint32_t& q) const
+  {
+    q = a.pair_quad[k];
+    return q < a.num_nodes ? a.offset[q] : 0xffffffffu;
+  }
+  __device__ uint64_t count(uint64_t k) const
+  {
+    uint32_t q, p = 0xffffffffu;
+    uint32_t const o = off(k, q);
+    if (q >= a.num_nodes) {
+      atomicOr(a.bad, kBadIndex);
+      return 0;
+    }
+    if (k > 0) {
+      uint32_t const before = off(k - 1, p);
+      if (before > o || (before == o && p != q)) atomicOr(a.bad, kIrregular);
+    }
+    return p == q ? 0ull : (static_cast<uint64_t>(a.length[q]) + kWave - 1) / kWave;
+  }
+  __device__ void emit(uint64_t k, uint64_t prefix) const
+  {
+    uint64_t const n = count(k);
+    if (n == 0) return;
+    if (prefix + n > cap) {
+      atomicOr(a.bad, kIrregular);
+      return;
+    }
+    for (uint64_t c = 0; c < n; ++c)
+      items[prefix + c] = make_uint2(static_cast<uint32_t>(k), static_cast<uint32_t>(c));
+  }
+};
+
+// One wave per work item. Each lane holds one point; a chunk of at most 32 points is
+// held in 64 / 2^ceil(log2 points) copies that take different segments. The run's
+// linestrings pass through the wave's LDS slot 63 segments at a time, in float32
+// coordinates relative to the chunk's first point (start, direction and 1 / length^2
+// per segment: 11 float32 instructions per point and segment instead of about 45
+// double ones with a division), the vertices of the next batch in flight meanwhile.
+//
+// With M the largest float32 coordinate met (points and vertices), every float32
+// distance is within 2^-19 M of the exact one (rounded ends, direction, projection and
+// difference: at most 31 roundings of 2^-24 M) and the reference's double result
+// within 2^-25 M (the cancellation of d0 - r), so E = 2^-17 M + 1e-14 bounds both: a
+// linestring whose distance is more than 2 E below every other's is the reference's
+// nearest (and no other one's distance is zero). Its distance is then computed as the
+// reference does. Otherwise (two linestrings that near, a zero distance, a linestring
+// without segments, coordinates that are not finite or above 1e15) the lane folds over
+// the run's pairs.
+//
+// Bound by the float32 instructions. 1e6 points, 20,000 linestrings of 2 to 32
+// vertices (about 15 per leaf of 61 points): one wave per pair, each segment a chain of
+// scalar loads and a double division, took 1232 us; this takes 362 us.
+constexpr int kNearWaves = 4;
+struct NearSegments {
+  float4 s[kWave];  // start, direction
+  float inv[kWave];
+};
+
+__global__ void __launch_bounds__(kNearWaves * kWave)
+  nearest_chunk_kernel(NearestArgs a, uint2 const* __restrict__ items,
+                       uint64_t const* __restrict__ total, uint64_t cap)
+{
+  __shared__ NearSegments s_seg[kNearWaves];
+  NearSegments& S   = s_seg[threadIdx.x / kWave];
+  uint64_t const w  = static_cast<uint64_t>(blockIdx.x) * kNearWaves + threadIdx.x / kWave;
+  uint64_t const T  = *total;
+  if (w >= T || T > cap) return;
+  int const lane    = lane_id();
+  uint2 const item  = items[w];
+  uint64_t const rs = uniform(item.x);
+  uint32_t const c  = uniform(item.y);
+  uint32_t const quad  = uniform_load(a.pair_quad + rs);
+  uint32_t const len   = uniform_load(a.length + quad);
+  uint32_t const first = uniform_load(a.offset + quad);
+  // the run's end: its pairs name the same quadrant
+  uint64_t R = 0;
+  while (true) {
+    uint64_t const k = rs + R + lane;
+    uint64_t const b = ballot(k < a.num_pairs && a.pair_quad[k] == quad);
+    R += b == ~0ull ? 64 : __builtin_ctzll(~b);
+    if (b != ~0ull) break;
+  }
+  uint32_t const q  = len - c * kWave < kWave ? len - c * kWave : kWave;
+  uint32_t const lq = q > 1 ? 32u - static_cast<uint32_t>(__builtin_clz(q - 1)) : 0u;
+  uint32_t const Q = 1u << lq, G = kWave >> lq;  // lanes per copy, copies
+  uint32_t const at = static_cast<uint32_t>(lane) & (Q - 1), g = static_cast<uint32_t>(lane) >> lq;
+  bool err       = false;
+  bool valid     = at < q;
+  uint64_t const pos = static_cast<uint64_t>(first) + c * static_cast<uint64_t>(kWave) + at;
+  double px = 0.0, py = 0.0;
+  if (valid) {
+    uint32_t const idx = pos < a.num_points ? a.point_indices[pos] : 0xffffffffu;
+    if (idx >= a.num_points) {
+      err   = true;
+      valid = false;
+    } else {
+      px = a.x[idx];
+      py = a.y[idx];
+    }
+  }
+  // readfirstlane of the first copy's first point (0 where that is not finite)
+  auto first_lane = [](double v) {
+    uint64_t const b = static_cast<uint64_t>(__double_as_longlong(v));
+    return __longlong_as_double(static_cast<long long>(
+      (static_cast<uint64_t>(uniform(static_cast<uint32_t>(b >> 32))) << 32) |
+      uniform(static_cast<uint32_t>(b))));
+  };
+  double const ox = first_lane(isfinite(px) ? px : 0.0), oy = first_lane(isfinite(py) ? py : 0.0);
+  float const fx = static_cast<float>(px - ox), fy = static_cast<float>(py - oy);
+  constexpr float kTop = 1e15f;  // squares and their sums stay finite
+  auto small = [](float x, float y) { return fabsf(x) <= kTop && fabsf(y) <= kTop; };  // not NaN
+  bool decided = valid && small(fx, fy);
+  float M      = decided ? fmaxf(fabsf(fx), fabsf(fy)) : 0.f;
+  float m1 = INFINITY, m2 = INFINITY;
+  uint64_t l1 = rs;
+  bool odd    = false;  // a vertex or linestring index the float32 pass cannot take
+  auto fence = [] {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  };
+  for (uint64_t kb = 0; kb < R; kb += kWave) {
+    // the next 64 pairs' vertex ranges, one per lane
+    uint32_t const nj = R - kb < kWave ? static_cast<uint32_t>(R - kb) : kWave;
+    uint32_t v_lo = 0, v_n = 0;  // first vertex, segments
+    if (static_cast<uint32_t>(lane) < nj) {
+      uint32_t const ls = a.pair_ls[rs + kb + lane];
+      if (ls >= a.num_ls) {
+        err = true;
+      } else {
+        uint64_t const b = a.ls_offsets[ls];
+        uint64_t e       = a.ls_offsets[ls + 1];
+        if (e > a.num_vertices) e = a.num_vertices;
+        if (b + 1 < e) {
+          v_lo = static_cast<uint32_t>(b);
+          v_n  = static_cast<uint32_t>(e - b - 1);
+        }
+      }
+    }
+    // batches (pair j, segment s): 63 segments are 64 vertices, one per lane
+    auto next_pair = [&](uint32_t j) {  // the first pair from j on with a segment
+      uint64_t const m = ballot(v_n > 0) & (j < kWave ? ~0ull << j : 0ull);
+      return m ? static_cast<uint32_t>(__builtin_ctzll(m)) : static_cast<uint32_t>(kWave);
+    };
+    auto rl = [](uint32_t v, uint32_t j) {
+      return static_cast<uint32_t>(
+        __builtin_amdgcn_readlane(static_cast<int>(v), static_cast<int>(j)));
+    };
+    uint32_t j = next_pair(0), sb = 0;
+    double vx = 0.0, vy = 0.0;
+    auto load = [&](uint32_t jj, uint32_t ss) {
+      uint32_t const n = rl(v_n, jj) - ss < 63u ? rl(v_n, jj) - ss : 63u;
+      if (static_cast<uint32_t>(lane) <= n) {
+        uint64_t const v = static_cast<uint64_t>(rl(v_lo, jj)) + ss + lane;
+        vx               = a.lx[v];
+        vy               = a.ly[v];
+      }
+    };
+    if (j < kWave) load(j, 0);
+    float m = INFINITY;
+    while (j < kWave) {
+      uint32_t const left = rl(v_n, j) - sb;
+      uint32_t const n    = left < 63u ? left : 63u;
+      float const sx = static_cast<float>(vx - ox), sy = static_cast<float>(vy - oy);
+      if (static_cast<uint32_t>(lane) <= n) {
+        if (small(sx, sy))
+          M = fmaxf(M, fmaxf(fabsf(sx), fabsf(sy)));
+        else
+          odd = true;
+      }
+      float const ex = __shfl_down(sx, 1, kWave) - sx, ey = __shfl_down(sy, 1, kWave) - sy;
+      float const l2 = ex * ex + ey * ey;
+      fence();
+      if (static_cast<uint32_t>(lane) < n) {
+        S.s[lane]   = make_float4(sx, sy, ex, ey);
+        S.inv[lane] = l2 > 1e-30f ? 1.f / l2 : 0.f;
+      }
+      fence();
+      // the next batch's vertices
+      bool const last   = left <= 63u;
+      uint32_t const jn = last ? next_pair(j + 1) : j, sn = last ? 0u : sb + 63u;
+      if (jn < kWave) load(jn, sn);
+#pragma unroll 4
+      for (uint32_t s = g; s < n; s += G) {
+        float4 const e = S.s[s];
+        float const wx = fx - e.x, wy = fy - e.y;
+        float const t =
+          __builtin_amdgcn_fmed3f(fmaf(wx, e.z, wy * e.w) * S.inv[s], 0.f, 1.f);
+        float const dx = fmaf(-t, e.z, wx), dy = fmaf(-t, e.w, wy);
+        m = fminf(m, fmaf(dx, dx, dy * dy));
+      }
+      if (last) {
+        for (uint32_t o = Q; o < kWave; o <<= 1) m = fminf(m, __shfl_xor(m, o, kWave));
+        if (m < m1) {
+          m2 = m1;
+          m1 = m;
+          l1 = rs + kb + j;
+        } else {
+          m2 = fminf(m2, m);
+        }
+        m = INFINITY;
+      }
+      j  = jn;
+      sb = sn;
+    }
+  }
+  if (ballot(odd || err)) decided = false;
+#pragma unroll
+  for (int o = kWave / 2; o > 0; o >>= 1) M = fmaxf(M, __shfl_xor(M, o, kWave));
+  float const E = fmaf(M, 0x1p-17f, 1e-14f);
+  decided       = decided && m1 < INFINITY && sqrtf(m1) + E < sqrtf(m2) - E;
+  bool const own = valid && g == 0;
+  uint32_t best_ls = 0;
+  double best_d    = 0.0;
+  if (own && decided) {
+    best_ls = a.pair_ls[l1];
+    best_d  = own_linestring_distance(a, best_ls, px, py);
+    decided = best_d != 0.0;
+  }
+  if (own && !decided) fold_run(a, rs, rs + R, px, py, best_ls, best_d, err);
+  if (own) {
+    a.out_point[pos] = static_cast<uint32_t>(pos);
+    a.out_ls[pos]    = best_ls;
+    a.out_dist[pos]  = best_d;
+  }
+  if (err) atomicOr(a.bad, kBadIndex);
 }
 
 __global__ void iota_i32_kernel(int32_t* __restrict__ p, int64_t n)
@@ -269,23 +543,48 @@ extern "C" int qpip_quadtree_point_to_nearest_linestring(const uint32_t* linestr
                   linestring_offsets, static_cast<uint64_t>(num_linestring_offsets - 1),
                   linestring_x, linestring_y, static_cast<uint64_t>(num_linestring_x), o_point,
                   o_ls, o_dist, bad.get()};
-    {
+    uint64_t const K = static_cast<uint64_t>(num_pairs);
+    auto fill = [&] {
       KernelTimer kt("nearest_fill", stream);
       nearest_fill_kernel<<<grid_for(static_cast<uint64_t>(n), 256, 1u << 30), 256, 0, stream>>>(a);
       QPIP_LAUNCH_CHECK();
+    };
+    uint32_t h_bad = 0;
+    auto status = [&] {
+      QPIP_HIP(hipMemcpyAsync(&h_bad, bad.get(), sizeof(uint32_t), hipMemcpyDeviceToHost, stream));
+      QPIP_HIP(hipStreamSynchronize(stream));
+    };
+    fill();
+    // chunks of the paired leaves: a tree's leaves hold each point once
+    uint64_t const cap = static_cast<uint64_t>(n) / kWave +
+                         std::min<uint64_t>(K, static_cast<uint64_t>(num_nodes));
+    if (K < (uint64_t{1} << 32) && cap < (uint64_t{1} << 31)) {
+      dbuf<uint2> items(cap);
+      dbuf<uint64_t> partials(kScanBlocks), total(1);
+      count_scan_emit<RunChunkOp, uint64_t, uint64_t>(RunChunkOp{a, items.get(), cap}, nullptr, K,
+                                                      partials.get(), total.get(), stream,
+                                                      scan_blocks_for(K), "nearest_chunks");
+      {
+        KernelTimer kt("nearest_linestring", stream);
+        nearest_chunk_kernel<<<static_cast<unsigned>((cap + kNearWaves - 1) / kNearWaves),
+                               kNearWaves * kWave, 0, stream>>>(a, items.get(), total.get(), cap);
+        QPIP_LAUNCH_CHECK();
+      }
+      status();
+    } else {
+      h_bad = kIrregular;
     }
-    {
+    if (h_bad & kIrregular) {
+      fill_u32(bad.get(), 1, 0u, stream);
+      fill();
       KernelTimer kt("nearest_linestring", stream);
-      uint64_t const K = static_cast<uint64_t>(num_pairs);
       for (uint64_t b = 0; b < K; b += uint64_t{1} << 22) {
         uint64_t const m = std::min<uint64_t>(K - b, uint64_t{1} << 22);
         nearest_kernel<<<static_cast<unsigned>((m + 3) / 4), 256, 0, stream>>>(a, b);
         QPIP_LAUNCH_CHECK();
       }
+      status();
     }
-    uint32_t h_bad = 0;
-    QPIP_HIP(hipMemcpyAsync(&h_bad, bad.get(), sizeof(uint32_t), hipMemcpyDeviceToHost, stream));
-    QPIP_HIP(hipStreamSynchronize(stream));
     if (h_bad)  // the outputs are released by `oa`
       throw logic_error(
         "cuSpatial failure: a quadrant, point or linestring index is out of range");

@@ -92,6 +92,64 @@ def test_random_matches_oracle(cs, oracle_mod, seed, n, L, d, ms, radius):
         assert covered < n  # some points lie in leaves with no pair
 
 
+def edge_lines(rng, ext):
+    """Linestrings at the batch edges (62 to 130 segments), coincident ones (ties),
+    zero-length segments, and one far longer than the area."""
+    lines = []
+    for k in (2, 3, 63, 64, 65, 66, 127, 128, 131):
+        c = rng.uniform(0, ext, 2)
+        lines.append(c + np.cumsum(rng.normal(0, 0.01 * ext, (k, 2)), 0))
+    lines += [lines[0].copy(), lines[4].copy(), np.repeat(rng.uniform(0, ext, (1, 2)), 3, 0),
+              np.array([[-40 * ext, 0.3 * ext], [40 * ext, 0.31 * ext]])]
+    offs = np.concatenate([[0], np.cumsum([len(v) for v in lines])]).astype(np.int32)
+    v = np.concatenate(lines)
+    return offs, v[:, 0].copy(), v[:, 1].copy()
+
+
+@pytest.mark.parametrize("case", ["plain", "offset", "nan", "huge", "tiny", "permuted"])
+@pytest.mark.parametrize("n,ms", [(1, 4), (33, 64), (5000, 64), (5000, 700)])
+def test_chunks_and_undecided_points_match_oracle(cs, oracle_mod, case, n, ms):
+    """The float32 choice and its fallbacks: chunks of 1 to 64 points (copies of the
+    points), points on vertices (zero distances), coincident linestrings (ties to the
+    lower id), coordinates far from the origin, not finite, above 1e15 and of 1e-18
+    extent, and a run's pairs in another order. Indices and distances bit for bit."""
+    rng = np.random.default_rng(n * 7 + ms)
+    ext, at = {"offset": (100.0, 3e7), "huge": (4e15, 0.0), "tiny": (1e-18, 0.0)}.get(
+        case, (100.0, 0.0))
+    offs, lx, ly = edge_lines(rng, ext)
+    x, y = rng.uniform(0, ext, n), rng.uniform(0, ext, n)
+    k = min(n // 4, 300)
+    i = rng.integers(0, len(lx) - 2, k)
+    x[:k], y[:k] = np.clip(lx[i], 0, ext), np.clip(ly[i], 0, ext)
+    x, y, lx, ly = x + at, y + at, lx + at, ly + at
+    if case == "nan":
+        lx[offs[2] + 1] = np.nan
+        ly[offs[3] + 1] = np.inf
+    bbox = (at, at + ext, at, at + ext)
+    d = 4
+    pts, L = cs.Points(x, y, device="cuda"), cs.Linestrings(offs, lx, ly, device="cuda")
+    pi, tree = cs.quadtree_on_points(pts, *bbox, ext / (1 << d), d, ms)
+    t = tuple(np_(tree[c]) for c in ("key", "level", "is_internal_node", "length", "offset"))
+    # every linestring against every leaf, in leaf-offset order
+    leaves = np.nonzero(t[2] == 0)[0]
+    leaves = leaves[np.argsort(t[4][leaves].astype(np.int64), kind="stable")]
+    order = np.arange(len(offs) - 1)
+    if case == "permuted":
+        order = rng.permutation(order)
+    pq = np.repeat(leaves, len(order)).astype(np.uint32)
+    pl = np.tile(order, len(leaves)).astype(np.uint32)
+    import torch
+
+    pairs = {"a": torch.as_tensor(pl.astype(np.int64), device="cuda"),
+             "b": torch.as_tensor(pq.astype(np.int64), device="cuda")}
+    res = cs.quadtree_point_to_nearest_linestring(pairs, tree, pi, pts, L)
+    opt, ols, od = oracle_mod.quadtree_point_to_nearest_linestring(
+        (pl, pq), t, np_(pi), x, y, offs, lx, ly)
+    assert np.array_equal(np_(res["point_index"]), opt)
+    assert np.array_equal(np_(res["linestring_index"]), ols)
+    assert np.array_equal(np_(res["distance"]).view(np.int64), od.view(np.int64))
+
+
 def test_empty_and_errors(cs):
     import torch
 
