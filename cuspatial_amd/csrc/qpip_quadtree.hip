@@ -13,20 +13,22 @@
 //   1. keygen (fused with the radix sort's first digit count);
 //   2. stable LSD radix sort of (key, point index) over the 2d+2 (at most 32)
 //      key bits that can be non-zero;
-//   3. level 0: the distinct values of key >> 2(d-1), found by binary search;
-//   4. level l -> l+1: every node with more than max_size points and l <= d-2
-//      (exactly the reference's internal nodes) is split into its non-empty
-//      child quadrants by three binary searches inside its sorted point range;
-//      children are appended in (parent, quadrant) order, i.e. level-major and
-//      key order within a level - the order of reverse_tree_levels;
-//   5. finalize: internal nodes get (length, offset) = (child count, first child
-//      position) and leaves (point count, first point position).
+//   3. starts: the node of level l that begins at sorted position i has more than
+//      max_size points iff keys i and i + max_size share its prefix, so the nodes that
+//      begin at a position, and which of them are internal, follow from a handful of
+//      keys near it, for every level at once (tree_count_kernel marks the positions
+//      and counts their nodes per level and block);
+//   4. a scan of the blocks' counts gives every level's and block's first node number;
+//   5. emit: each marked position writes its nodes straight into the output columns,
+//      level-major and in key order within a level - the order of
+//      reverse_tree_levels. Internal nodes get (length, offset) = (child count, first
+//      child position) and leaves (point count, first point position).
 //
 // Equivalences with the reference (for the 5 output columns):
 //   * a level-l node is kept by remove_unqualified_quads iff its parent has more
 //     than max_size points (phase_2.cuh:256-281); since point counts shrink
-//     downwards, that is iff all its ancestors are internal - the nodes generated
-//     in step 4;
+//     downwards, that is iff all its ancestors are internal - the nodes of steps 3
+//     to 5;
 //   * a leaf's offset is the exclusive scan of leaf point counts in Morton order
 //     (phase_2.cuh:105-184); leaves tile the sorted points in Morton order, so it
 //     is the leaf's first sorted point position;
@@ -51,9 +53,8 @@ constexpr int kMaxLevels = 16;
 constexpr int kMaxMarked = 16;
 
 struct TreeMeta {
-  uint64_t sizes[kMaxLevels + 1];  // nodes per level (sizes[l] for l < d)
-  uint32_t overflow;
-  uint32_t num_marked;             // E = R - 1 (d >= 1)
+  uint32_t level_begin[kMaxLevels + 1];  // first node of each level; [levels]: all nodes
+  uint32_t num_marked;                   // E = R - 1 (d >= 1)
   uint32_t marked_key[kMaxMarked];
   uint32_t marked_internal[kMaxMarked];
   uint32_t marked_start[kMaxMarked];
@@ -156,145 +157,386 @@ __global__ void __launch_bounds__(256)
   counts[static_cast<uint64_t>(blockIdx.x) * kRadix + threadIdx.x] = s;
 }
 
-// --- 3. level 0 and the root-level quirk ----------------------------------------
-// One wave. Lane v tests the level-0 prefix v (key >> shift0 == v, v < 64).
-__global__ void __launch_bounds__(64)
-  level0_kernel(uint32_t const* __restrict__ K,
-                uint32_t n,
-                int d,
-                uint32_t* __restrict__ nkey,
-                uint32_t* __restrict__ nstart,
-                uint32_t* __restrict__ ncount,
-                uint8_t* __restrict__ nlevel,
-                TreeMeta* __restrict__ meta)
-{
-  int const v        = lane_id();
-  int const shift0   = d >= 1 ? 2 * (d - 1) : 0;
-  uint32_t const lo  = lower_bound_u32(K, 0, n, static_cast<uint64_t>(v) << shift0);
-  uint32_t const hi  = lower_bound_u32(K, lo, n, static_cast<uint64_t>(v + 1) << shift0);
-  bool const present = hi > lo;
-  uint64_t const m   = ballot(present);
-  if (present) {
-    uint32_t const slot = static_cast<uint32_t>(__popcll(m & lanemask_lt()));
-    nkey[slot]          = static_cast<uint32_t>(v);
-    nstart[slot]        = lo;
-    ncount[slot]        = hi - lo;
-    nlevel[slot]        = 0;
-  }
-  // Root level: distinct key >> 2d (d >= 1); at most 16 values.
-  bool root_present = false;
-  if (d >= 1 && v < 16) {
-    uint32_t const rlo = lower_bound_u32(K, 0, n, static_cast<uint64_t>(v) << (2 * d));
-    uint32_t const rhi = lower_bound_u32(K, rlo, n, static_cast<uint64_t>(v + 1) << (2 * d));
-    root_present       = rhi > rlo;
-  }
-  uint64_t const rm = ballot(root_present);
-  if (v == 0) {
-    for (int l = 0; l <= kMaxLevels; ++l) meta->sizes[l] = 0;
-    meta->sizes[0]     = static_cast<uint64_t>(__popcll(m));
-    meta->overflow     = 0;
-    int const R        = __popcll(rm);
-    uint32_t const E   = (d >= 1 && R > 1) ? static_cast<uint32_t>(R - 1) : 0u;
-    meta->num_marked   = E;
-    // The first E distinct bottom-level keys (the extra "parents").
-    uint32_t pos = 0;
-    for (uint32_t e = 0; e < E && pos < n; ++e) {
-      uint32_t const k      = K[pos];
-      meta->marked_key[e]   = k;
-      meta->marked_internal[e] = 0;
-      meta->marked_start[e] = 0;
-      meta->marked_count[e] = 0;
-      pos                   = lower_bound_u32(K, pos, n, static_cast<uint64_t>(k) + 1);
-    }
-  }
-}
+// --- 3. starts --------------------------------------------------------------------
+// Levels run from 0 to last = max(d, 1) - 1; a level-l node is the run of keys equal
+// above bit 2 (last - l).
+struct TreeShape {
+  uint32_t const* K;  // sorted keys
+  uint32_t n;
+  int last;           // deepest level
+  uint32_t max_size;
 
-// After all levels: total node count and the kept extra "parents".
-__global__ void __launch_bounds__(64)
-  post_levels_kernel(uint32_t const* __restrict__ nkey,
-                     uint32_t const* __restrict__ nstart,
-                     uint32_t const* __restrict__ ncount,
-                     int d,
-                     uint32_t max_size,
-                     uint64_t cap,
-                     TreeMeta* __restrict__ meta)
-{
-  if (threadIdx.x != 0) return;
-  uint64_t total = 0, bottom_begin = 0;
-  int const levels = d >= 1 ? d : 1;
-  for (int l = 0; l < levels; ++l) {
-    if (l == levels - 1) bottom_begin = total;
-    total += meta->sizes[l];
+  __device__ __forceinline__ bool share(uint32_t a, uint32_t b, int l) const
+  {
+    return ((a ^ b) >> (2 * (last - l))) == 0;
   }
-  meta->num_nodes = total;
-  if (total > cap) {
-    meta->overflow = 1;
-    return;
+  // The deepest level at which keys a and b are in one node, -1 if none.
+  __device__ __forceinline__ int common(uint32_t a, uint32_t b) const
+  {
+    if (a == b) return last;
+    int const l = last - 1 - ((31 - __builtin_clz(a ^ b)) >> 1);
+    return l < 0 ? -1 : l;
   }
-  uint32_t const lo0 = static_cast<uint32_t>(bottom_begin);
-  uint32_t const hi0 = static_cast<uint32_t>(total);
-  for (uint32_t e = 0; e < meta->num_marked; ++e) {
-    uint32_t const mk = meta->marked_key[e];
-    uint32_t const at = lower_bound_u32(nkey, lo0, hi0, mk);
-    if (at < hi0 && nkey[at] == mk && ncount[at] > max_size) {
-      meta->marked_internal[e] = 1;
-      meta->marked_start[e]    = nstart[at];
-      meta->marked_count[e]    = ncount[at];
+  // What may_start reads.
+  struct Near {
+    uint32_t k, before, low, high;  // keys i, i - 1, i - 1 - h, i + h, h = max_size / 2
+  };
+  __device__ __forceinline__ Near load_near(uint32_t i) const
+  {
+    uint32_t const h = max_size / 2;
+    return Near{K[i], K[i > 0 ? i - 1 : 0], K[i > h ? i - 1 - h : 0], K[n - i > h ? i + h : n - 1]};
+  }
+  // False for most positions that begin no kept node (inside a leaf). The first node that
+  // can begin at i > 0 is a child of the node of level c = common(K[i - 1], K[i]), which
+  // holds both and is internal only if it holds more than max_size positions; such a
+  // range reaches i - 1 - h or i + h.
+  __device__ __forceinline__ bool may_start(uint32_t i, Near const& v) const
+  {
+    int const c = common(v.before, v.k);
+    if (i == 0 || c < 0) return true;
+    uint32_t const h = max_size / 2;
+    return c < last &&
+           ((i > h && share(v.low, v.k, c)) || (n - i > h && share(v.high, v.k, c)));
+  }
+  // The level of the first node that begins at position i if it is kept (its parent,
+  // which then holds i - 1 too, is internal), else last + 1.
+  __device__ __forceinline__ int first_level(uint32_t i, uint32_t k) const
+  {
+    if (i == 0) return 0;
+    int const c = common(K[i - 1], k);  // the parent's level
+    if (c < 0) return 0;
+    if (c == last) return last + 1;
+    uint32_t const ms = max_size;
+    if (i >= ms && share(K[i - ms], k, c)) return c + 1;
+    // the parent begins after i - max_size
+    uint32_t lo = i >= ms ? i - ms + 1 : 0, hi = i - 1;
+    while (lo < hi) {
+      uint32_t const mid = lo + ((hi - lo) >> 1);
+      if (share(K[mid], k, c))
+        hi = mid;
+      else
+        lo = mid + 1;
     }
+    return n - lo > ms && share(K[lo + ms], k, c) ? c + 1 : last + 1;
   }
-}
+  // The leaf level of the chain of nodes that begins at i with level f: each node with
+  // more than max_size points has its first child at i too.
+  __device__ __forceinline__ int leaf_level(uint32_t i, uint32_t k, int f) const
+  {
+    int const c = n - i > max_size ? common(k, K[i + max_size]) : -1;
+    if (c < f) return f;
+    return c + 1 < last ? c + 1 : last;
+  }
+};
 
-// --- 5. finalize: the five output columns (detail/point_quadtree.cuh:88-133) ----
+// Per block: nodes per level [0, 16) and the first marked position [16] (all ones:
+// none); after the scan, the nodes before the block per level and the first marked
+// position after it.
+constexpr int kTreeCols   = 17;
+constexpr int kTreeBlocks = 1024;  // entries per column
+
+// Marks the positions of block b's range [b * per, (b + 1) * per) at which kept nodes
+// begin (per is a multiple of kTreeStep: the blocks share no word of `marks`) and counts
+// their nodes. Per kTreeSpan positions: first the positions that may start a node
+// (eight per thread in flight), compacted in LDS, then those one per thread, so that a
+// wave does not wait for a binary search in nearly every word (1e8 keys took 1109 us
+// that way, 275 us so). Bound by the latency of its loads: 0.4 GB of keys from HBM, the
+// other three reads of each are in the caches. With the scan and the emit the tree
+// of 1e8 keys at depth 15 (1.2M nodes) takes 0.37 ms in 4 launches, against 0.46 ms in
+// 30 as two launches per level (a search for every node's child boundaries), and that
+// of 1e6 keys at depth 7 24 us in 4 launches against 95 us in 15.
+constexpr int kTreeItems = 8;
+constexpr int kTreeStep  = 256 * kTreeItems;  // positions per block and round
+constexpr int kTreeSpan  = 256 * kWave;       // positions per LDS list
+
 __global__ void __launch_bounds__(256)
-  finalize_kernel(uint32_t const* __restrict__ nkey,
-                  uint32_t const* __restrict__ nstart,
-                  uint32_t const* __restrict__ ncount,
-                  uint8_t const* __restrict__ nlevel,
-                  uint32_t const* __restrict__ cfirst,
-                  uint32_t const* __restrict__ ccount,
-                  TreeMeta const* __restrict__ meta,
-                  int d,
-                  uint32_t max_size,
-                  uint64_t m,
-                  uint32_t* __restrict__ out_key,
-                  uint8_t* __restrict__ out_level,
-                  uint8_t* __restrict__ out_internal,
-                  uint32_t* __restrict__ out_length,
-                  uint32_t* __restrict__ out_offset)
+  tree_count_kernel(TreeShape t, uint32_t per, uint64_t* __restrict__ marks,
+                    uint32_t* __restrict__ cols)
 {
-  for (uint64_t i = static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < m;
-       i += static_cast<uint64_t>(gridDim.x) * blockDim.x)
-    [&] {
-      uint32_t const key   = nkey[i];
-      int const level      = nlevel[i];
-      uint32_t const count = ncount[i];
-      uint32_t const start = nstart[i];
-      bool internal        = level <= d - 2 && count > max_size;
-      uint32_t length      = internal ? ccount[i] : count;
-      uint32_t offset      = internal ? cfirst[i] : start;
-      uint32_t const E     = meta->num_marked;
-      if (E > 0 && !internal) {
-        bool marked = false;
-        uint32_t skipped = 0;
-        for (uint32_t e = 0; e < E; ++e) {
-          if (!meta->marked_internal[e]) continue;
-          if (level == d - 1 && meta->marked_key[e] == key) marked = true;
-          if (meta->marked_start[e] < start) skipped += meta->marked_count[e];
-        }
-        if (marked) {
-          internal = true;
-          length   = 0;
-          offset   = static_cast<uint32_t>(m);
-        } else {
-          offset = start - skipped;
+  __shared__ uint16_t s_at[kTreeSpan];
+  __shared__ unsigned long long s_word[kTreeSpan / kWave];
+  __shared__ uint32_t s_cols[kTreeCols];
+  __shared__ uint32_t s_total;
+  if (threadIdx.x < kTreeCols) s_cols[threadIdx.x] = threadIdx.x == 16 ? 0xffffffffu : 0u;
+  uint64_t const lo = static_cast<uint64_t>(blockIdx.x) * per;
+  uint64_t const hi = lo + per < t.n ? lo + per : t.n;
+  int const lane    = lane_id();
+  uint32_t cnt = 0, first = 0xffffffffu;  // lane l: level l's nodes
+  for (uint64_t i0 = lo; i0 < hi; i0 += kTreeSpan) {
+    uint64_t const i1 = i0 + kTreeSpan < hi ? i0 + kTreeSpan : hi;
+    s_word[threadIdx.x] = 0;
+    if (threadIdx.x == 0) s_total = 0;
+    __syncthreads();
+    for (uint64_t r = i0; r < i1; r += kTreeStep) {
+      TreeShape::Near v[kTreeItems];
+#pragma unroll
+      for (int u = 0; u < kTreeItems; ++u) {
+        uint64_t const i = r + u * 256 + threadIdx.x;
+        v[u]             = t.load_near(static_cast<uint32_t>(i < i1 ? i : i1 - 1));
+      }
+#pragma unroll
+      for (int u = 0; u < kTreeItems; ++u) {
+        uint64_t const i = r + u * 256 + threadIdx.x;
+        bool const may   = i < i1 && t.may_start(static_cast<uint32_t>(i), v[u]);
+        uint64_t const b = ballot(may);
+        if (b == 0) continue;
+        uint32_t at = 0;
+        if (lane == 0) at = atomicAdd(&s_total, static_cast<uint32_t>(__popcll(b)));
+        at = uniform(at) + static_cast<uint32_t>(__popcll(b & lanemask_lt()));
+        if (may) s_at[at] = static_cast<uint16_t>(i - i0);
+      }
+    }
+    __syncthreads();
+    uint32_t const total = s_total;
+    for (uint32_t q = threadIdx.x; q - lane < total; q += 256) {
+      int f = t.last + 1, leaf = -1;
+      if (q < total) {
+        uint32_t const at = s_at[q];
+        uint32_t const i  = static_cast<uint32_t>(i0) + at;
+        uint32_t const k  = t.K[i];
+        f                 = t.first_level(i, k);
+        if (f <= t.last) {
+          leaf  = t.leaf_level(i, k, f);
+          first = i < first ? i : first;
+          atomicOr(&s_word[at / kWave], 1ull << (at % kWave));
         }
       }
-      out_key[i]      = key;
-      out_level[i]    = static_cast<uint8_t>(level);
-      out_internal[i] = internal ? 1 : 0;
-      out_length[i]   = length;
-      out_offset[i]   = offset;
-    }();
+      for (int l = 0; l <= t.last; ++l) {
+        uint64_t const b = ballot(f <= l && l <= leaf);
+        if (lane == l) cnt += static_cast<uint32_t>(__popcll(b));
+      }
+    }
+    __syncthreads();
+    if (i0 + threadIdx.x * kWave < i1) marks[i0 / kWave + threadIdx.x] = s_word[threadIdx.x];
+    __syncthreads();
+  }
+  if (lane < 16 && cnt) atomicAdd(&s_cols[lane], cnt);
+  if (first != 0xffffffffu) atomicMin(&s_cols[16], first);
+  __syncthreads();
+  if (threadIdx.x < kTreeCols) cols[threadIdx.x * kTreeBlocks + blockIdx.x] = s_cols[threadIdx.x];
+}
+
+// --- 4. scan of the blocks' counts, level sizes and the root-level quirk -----------
+__global__ void __launch_bounds__(1024)
+  tree_scan_kernel(TreeShape t, int d, uint32_t blocks, uint32_t* __restrict__ cols,
+                   TreeMeta* __restrict__ meta)
+{
+  __shared__ uint32_t s_total[kMaxLevels];
+  int const w = static_cast<int>(uniform(threadIdx.x / kWave)), lane = lane_id();
+  // Waves 0 .. last scan the levels' columns and wave 15 (last <= 14) the first marked
+  // positions; the values of up to 1024 blocks are loaded before they are scanned.
+  if (w <= t.last || w == 15) {
+    int const col = w == 15 ? 16 : w;
+    uint32_t v[kTreeBlocks / kWave];
+#pragma unroll
+    for (int c = 0; c < kTreeBlocks / kWave; ++c) {
+      uint32_t const b = static_cast<uint32_t>(c * kWave + lane);
+      v[c]             = b < blocks ? cols[col * kTreeBlocks + b] : w == 15 ? 0xffffffffu : 0u;
+    }
+    if (w == 15) {
+      uint32_t next = 0xffffffffu;
+#pragma unroll
+      for (int c = kTreeBlocks / kWave - 1; c >= 0; --c) {
+        if (static_cast<uint32_t>(c * kWave) >= blocks) continue;
+        uint32_t m = v[c];  // smallest of this lane's and the higher lanes'
+#pragma unroll
+        for (int o = 1; o < kWave; o <<= 1) {
+          uint32_t const x = __shfl_down(m, o, kWave);
+          if (lane + o < kWave) m = x < m ? x : m;
+        }
+        uint32_t const above = __shfl_down(m, 1, kWave);
+        uint32_t const b     = static_cast<uint32_t>(c * kWave + lane);
+        if (b < blocks)
+          cols[16 * kTreeBlocks + b] = lane + 1 < kWave && above < next ? above : next;
+        uint32_t const all = __shfl(m, 0, kWave);
+        next               = all < next ? all : next;
+      }
+    } else {
+      uint32_t run = 0;
+#pragma unroll
+      for (int c = 0; c < kTreeBlocks / kWave; ++c) {
+        if (static_cast<uint32_t>(c * kWave) >= blocks) break;
+        uint32_t const b    = static_cast<uint32_t>(c * kWave + lane);
+        uint32_t const incl = wave_incl_scan(v[c]);
+        if (b < blocks) cols[w * kTreeBlocks + b] = run + incl - v[c];
+        run += __shfl(incl, kWave - 1, kWave);
+      }
+      if (lane == 0) s_total[w] = run;
+    }
+  }
+  __syncthreads();
+  if (w != 0) return;
+  // Root level: distinct key >> 2d (d >= 1); at most 16 values.
+  bool root_present = false;
+  bool const many   = d >= 1 && (t.K[0] >> (2 * d)) != (t.K[t.n - 1] >> (2 * d));
+  if (many && lane < 16) {
+    uint32_t const lo = lower_bound_u32(t.K, 0, t.n, static_cast<uint64_t>(lane) << (2 * d));
+    uint32_t const hi = lower_bound_u32(t.K, lo, t.n, static_cast<uint64_t>(lane + 1) << (2 * d));
+    root_present      = hi > lo;
+  }
+  uint64_t const rm = ballot(root_present);
+  if (lane != 0) return;
+  uint32_t total = 0;
+  for (int l = 0; l <= kMaxLevels; ++l) {
+    meta->level_begin[l] = total;
+    if (l <= t.last) total += s_total[l];
+  }
+  meta->num_nodes = total;
+  int const R      = __popcll(rm);
+  uint32_t const E = R > 1 ? static_cast<uint32_t>(R - 1) : 0u;
+  meta->num_marked = E;
+  // The first E distinct bottom-level keys (the extra "parents").
+  uint32_t pos = 0;
+  for (uint32_t e = 0; e < E; ++e) {
+    meta->marked_internal[e] = meta->marked_start[e] = meta->marked_count[e] = 0;
+    uint32_t const k    = pos < t.n ? t.K[pos] : 0xffffffffu;
+    meta->marked_key[e] = k;
+    if (pos < t.n) pos = lower_bound_u32(t.K, pos, t.n, static_cast<uint64_t>(k) + 1);
+  }
+}
+
+// --- 5. emit ------------------------------------------------------------------------
+struct TreeOut {
+  uint32_t* key;
+  uint8_t* level;
+  uint8_t* internal;
+  uint32_t* length;  // zeroed: an internal node's is counted by its children
+  uint32_t* offset;
+};
+
+// Block b writes the nodes that begin in its range (tree_count_kernel's), 256 marked
+// positions at a time: one per thread, ranked per level by ballots. A position's first
+// node is a child of the last node of the level above that began before it.
+__global__ void __launch_bounds__(256)
+  tree_emit_kernel(TreeShape t, uint32_t per, uint64_t const* __restrict__ marks,
+                   uint32_t const* __restrict__ cols, TreeMeta const* __restrict__ meta, TreeOut o)
+{
+  constexpr int NW = 256 / kWave;
+  __shared__ uint16_t s_at[256 * kWave];  // marked positions of 256 words, relative
+  __shared__ uint32_t s_scan[NW + 1];
+  __shared__ uint32_t s_run[kMaxLevels];  // per level: the next node's number
+  __shared__ uint32_t s_cnt[NW][kMaxLevels];
+  __shared__ uint32_t s_open[2];  // the last leaf written, whose end is not known yet
+  int const w = threadIdx.x / kWave, lane = lane_id();
+  uint64_t const lo = static_cast<uint64_t>(blockIdx.x) * per;
+  uint64_t const hi = lo + per < t.n ? lo + per : t.n;
+  if (threadIdx.x < kMaxLevels)
+    s_run[threadIdx.x] = meta->level_begin[threadIdx.x] + cols[threadIdx.x * kTreeBlocks + blockIdx.x];
+  bool open = false;
+  for (uint64_t i0 = lo; i0 < hi; i0 += 256 * kWave) {
+    uint64_t const at = i0 + threadIdx.x * kWave;
+    uint64_t word     = at < hi ? marks[at / kWave] : 0ull;
+    uint32_t total;
+    uint32_t slot = block_excl_scan<256>(static_cast<uint32_t>(__popcll(word)), s_scan, &total);
+    while (word) {
+      s_at[slot++] = static_cast<uint16_t>(threadIdx.x * kWave + __builtin_ctzll(word));
+      word &= word - 1;
+    }
+    __syncthreads();
+    if (total == 0) continue;
+    if (open && threadIdx.x == 0)
+      o.length[s_open[0]] = static_cast<uint32_t>(i0) + s_at[0] - s_open[1];
+    open = true;
+    for (uint32_t s0 = 0; s0 < total; s0 += 256) {
+      uint32_t const s = s0 + threadIdx.x;
+      bool const live  = s < total;
+      uint32_t i = 0, k = 0;
+      int f = t.last + 1, leaf = -1;
+      if (live) {
+        i    = static_cast<uint32_t>(i0) + s_at[s];
+        k    = t.K[i];
+        f    = i == 0 ? 0 : t.common(t.K[i - 1], k) + 1;
+        leaf = t.leaf_level(i, k, f);
+      }
+      for (int l = 0; l <= t.last; ++l) {
+        uint64_t const b = ballot(f <= l && l <= leaf);
+        if (lane == 0) s_cnt[w][l] = static_cast<uint32_t>(__popcll(b));
+      }
+      __syncthreads();
+      uint32_t above = 0;  // the node one level up (this position's, or its parent)
+      for (int l = 0; l <= t.last; ++l) {
+        uint64_t const b = ballot(f <= l && l <= leaf);
+        uint32_t node    = s_run[l] + static_cast<uint32_t>(__popcll(b & lanemask_lt()));
+        for (int q = 0; q < w; ++q) node += s_cnt[q][l];
+        if (live && l == f - 1) above = node - 1;
+        if (!(f <= l && l <= leaf)) continue;
+        if (l > 0) {
+          atomicAdd(&o.length[above], 1u);
+          if (l > f) o.offset[above] = node;  // its first child
+        }
+        o.key[node]      = k >> (2 * (t.last - l));
+        o.level[node]    = static_cast<uint8_t>(l);
+        o.internal[node] = l < leaf ? 1 : 0;
+        if (l == leaf) {
+          o.offset[node] = i;
+          if (s + 1 < total) {
+            o.length[node] = static_cast<uint32_t>(i0) + s_at[s + 1] - i;
+          } else {
+            s_open[0] = node;
+            s_open[1] = i;
+          }
+        }
+        above = node;
+      }
+      __syncthreads();
+      if (threadIdx.x <= static_cast<unsigned>(t.last)) {
+        uint32_t add = 0;
+        for (int q = 0; q < NW; ++q) add += s_cnt[q][threadIdx.x];
+        s_run[threadIdx.x] += add;
+      }
+      __syncthreads();
+    }
+  }
+  if (open && threadIdx.x == 0) {
+    uint32_t const next = cols[16 * kTreeBlocks + blockIdx.x];
+    o.length[s_open[0]] = (next == 0xffffffffu ? t.n : next) - s_open[1];
+  }
+}
+
+// The extra "parents" among the bottom-level nodes: those that hold more than
+// max_size points.
+__global__ void __launch_bounds__(64)
+  mark_extra_kernel(uint32_t const* __restrict__ key, uint32_t const* __restrict__ length,
+                    uint32_t const* __restrict__ offset, int last, uint32_t max_size,
+                    TreeMeta* __restrict__ meta)
+{
+  if (threadIdx.x != 0) return;
+  uint32_t const lo0 = meta->level_begin[last];
+  uint32_t const hi0 = static_cast<uint32_t>(meta->num_nodes);
+  for (uint32_t e = 0; e < meta->num_marked; ++e) {
+    uint32_t const mk = meta->marked_key[e];
+    uint32_t const at = lower_bound_u32(key, lo0, hi0, mk);
+    if (at < hi0 && key[at] == mk && length[at] > max_size) {
+      meta->marked_internal[e] = 1;
+      meta->marked_start[e]    = offset[at];
+      meta->marked_count[e]    = length[at];
+    }
+  }
+}
+
+// Flags them internal and drops their points from the leaves' offsets.
+__global__ void __launch_bounds__(256)
+  apply_extra_kernel(TreeMeta const* __restrict__ meta, int last, uint64_t m, TreeOut o)
+{
+  for (uint64_t i = static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < m;
+       i += static_cast<uint64_t>(gridDim.x) * blockDim.x) {
+    if (o.internal[i]) continue;
+    uint32_t const key = o.key[i], start = o.offset[i];
+    bool marked        = false;
+    uint32_t skipped   = 0;
+    for (uint32_t e = 0; e < meta->num_marked; ++e) {
+      if (!meta->marked_internal[e]) continue;
+      if (o.level[i] == last && meta->marked_key[e] == key) marked = true;
+      if (meta->marked_start[e] < start) skipped += meta->marked_count[e];
+    }
+    if (marked) {
+      o.internal[i] = 1;
+      o.length[i]   = 0;
+      o.offset[i]   = static_cast<uint32_t>(m);
+    } else {
+      o.offset[i] = start - skipped;
+    }
+  }
 }
 
 }  // namespace
@@ -360,47 +602,27 @@ static int64_t quadtree_on_points_impl(double const* x,
                                        un, key_bits, stream, counts0.get(), "point_sort");
   vals_tmp.release();
 
-  // Node capacity: level 0 holds <= 64 nodes; level l >= 1 holds <= 4 children
-  // of each internal node of level l-1 (internal nodes of a level are disjoint
-  // and hold > max_size points each), <= n, and <= 64 * 4^l.
-  uint64_t const internal_bound = un / (static_cast<uint64_t>(max_size) + 1);
-  uint64_t cap                  = 64;
-  for (int l = 1; l < std::max(d, 1); ++l) {
-    uint64_t c = std::min<uint64_t>(un, 4 * internal_bound);
-    if (2 * l + 6 < 62) c = std::min<uint64_t>(c, uint64_t{64} << (2 * l));
-    cap += c;
-  }
-  dbuf<uint32_t> nkey(cap), nstart(cap), ncount(cap), cfirst(cap), ccount(cap);
-  dbuf<uint8_t> nlevel(cap);
+  TreeShape const shape{sorted.keys, static_cast<uint32_t>(un), std::max(d, 1) - 1,
+                        static_cast<uint32_t>(max_size)};
+  // blocks of whole rounds, at most kTreeBlocks of them
+  uint64_t per = (un + kTreeBlocks - 1) / kTreeBlocks;
+  per          = std::max<uint64_t>(1, (per + kTreeStep - 1) / kTreeStep) * kTreeStep;
+  uint32_t const blocks = static_cast<uint32_t>((un + per - 1) / per);
+  dbuf<uint64_t> marks((un + kWave - 1) / kWave + 256 / kWave);
+  dbuf<uint32_t> cols(kTreeBlocks * kTreeCols);
   dbuf<TreeMeta> meta(1);
-  dbuf<uint4> split(cap);
-  dbuf<uint32_t> partials(kLevelBlocks);
-
   {
-  KernelTimer kt_levels("tree_levels", stream);
-  level0_kernel<<<1, 64, 0, stream>>>(sorted.keys, static_cast<uint32_t>(un), d, nkey.get(),
-                                      nstart.get(), ncount.get(), nlevel.get(), meta.get());
-  QPIP_LAUNCH_CHECK();
-  // Levels 0..d-2 may have children (level d-1 is the bottom).
-  for (int l = 0; l + 2 <= d; ++l) {
-    LevelArgs la{sorted.keys, nkey.get(), nstart.get(), ncount.get(), nlevel.get(),
-                 cfirst.get(), ccount.get(), split.get(), partials.get(), meta.get()->sizes,
-                 &meta.get()->overflow, cap, l};
-    UniformLevels rule{d, static_cast<uint32_t>(max_size)};
-    level_split_kernel<<<kLevelBlocks, 256, 0, stream>>>(la, rule);
+    KernelTimer kt("tree_count", stream);
+    tree_count_kernel<<<blocks, 256, 0, stream>>>(shape, static_cast<uint32_t>(per), marks.get(),
+                                                  cols.get());
     QPIP_LAUNCH_CHECK();
-    level_emit_kernel<<<kLevelBlocks, 256, 0, stream>>>(la, rule);
+    tree_scan_kernel<<<1, 1024, 0, stream>>>(shape, d, blocks, cols.get(), meta.get());
     QPIP_LAUNCH_CHECK();
-  }
-  post_levels_kernel<<<1, 64, 0, stream>>>(nkey.get(), nstart.get(), ncount.get(), d,
-                                           static_cast<uint32_t>(max_size), cap, meta.get());
-  QPIP_LAUNCH_CHECK();
   }
 
   TreeMeta h_meta;
   QPIP_HIP(hipMemcpyAsync(&h_meta, meta.get(), sizeof(TreeMeta), hipMemcpyDeviceToHost, stream));
   QPIP_HIP(hipStreamSynchronize(stream));
-  if (h_meta.overflow) throw device_error("quadtree node capacity exceeded (internal error)");
   uint64_t const m = h_meta.num_nodes;
 
   uint32_t* o_key      = oa.make<uint32_t>(m);
@@ -408,13 +630,20 @@ static int64_t quadtree_on_points_impl(double const* x,
   uint8_t* o_internal  = oa.make<uint8_t>(m);
   uint32_t* o_length   = oa.make<uint32_t>(m);
   uint32_t* o_offset   = oa.make<uint32_t>(m);
-  if (m > 0) {
-    KernelTimer kt("tree_finalize", stream);
-    finalize_kernel<<<grid_for(m, 256), 256, 0, stream>>>(
-      nkey.get(), nstart.get(), ncount.get(), nlevel.get(), cfirst.get(), ccount.get(),
-      meta.get(), d, static_cast<uint32_t>(max_size), m, o_key, o_level, o_internal, o_length,
-      o_offset);
+  {
+    KernelTimer kt("tree_emit", stream);
+    TreeOut const out{o_key, o_level, o_internal, o_length, o_offset};
+    fill_u32(o_length, m, 0u, stream);
+    tree_emit_kernel<<<blocks, 256, 0, stream>>>(shape, static_cast<uint32_t>(per), marks.get(),
+                                                 cols.get(), meta.get(), out);
     QPIP_LAUNCH_CHECK();
+    if (h_meta.num_marked > 0) {
+      mark_extra_kernel<<<1, 64, 0, stream>>>(o_key, o_length, o_offset, shape.last,
+                                              shape.max_size, meta.get());
+      QPIP_LAUNCH_CHECK();
+      apply_extra_kernel<<<grid_for(m, 256), 256, 0, stream>>>(meta.get(), shape.last, m, out);
+      QPIP_LAUNCH_CHECK();
+    }
   }
   // no wait here: the outputs are ready for work queued on `stream` after this call
   *point_indices = pi;

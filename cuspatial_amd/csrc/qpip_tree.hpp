@@ -1,5 +1,5 @@
-// Device code of the quadtree shared by the single-tree path and the batched
-// (many trees) path: Morton keys and the top-down level expansion.
+// Device code of the quadtree: the Morton keys of the single-tree and the batched
+// (many trees) path, and the batched path's top-down level expansion.
 #pragma once
 
 #include "qpip_scan.hpp"
@@ -87,24 +87,7 @@ struct LevelArgs {
   uint32_t* overflow;  // set when the node capacity is exceeded
   uint64_t cap;
   int level;
-  uint32_t const* samples = nullptr;  // K[j * kKeySample], or null: search K alone
-};
-
-// Split rule of one quadtree (every node has the same parameters): a node of
-// `level` may have children when level <= d - 2 and it holds more than max_size
-// points; its children's key prefixes start at bit 2 (d - 2 - level).
-struct UniformLevels {
-  int d;
-  uint32_t max_size;
-  __device__ __forceinline__ bool rule(uint64_t, int level, uint32_t& ms, int& sh,
-                                       uint64_t& prefix) const
-  {
-    ms     = max_size;
-    sh     = 2 * (d - 2 - level);
-    prefix = 0;
-    return level <= d - 2;
-  }
-  __device__ __forceinline__ void inherit(uint64_t, uint64_t) const {}
+  uint32_t const* samples;  // K[j * kKeySample]
 };
 
 __device__ __forceinline__ uint64_t level_begin(uint64_t const* sizes, int level)
@@ -173,44 +156,9 @@ __device__ __forceinline__ void wave_split(uint32_t const* __restrict__ K, uint3
   b3 = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(lo), 2 * P));
 }
 
-// Child boundaries with one thread: three interleaved binary searches.
-__device__ __forceinline__ void thread_split(uint32_t const* __restrict__ K, uint32_t s,
-                                             uint32_t e, uint32_t key, int sh, uint64_t prefix,
-                                             uint32_t& b1, uint32_t& b2, uint32_t& b3)
-{
-  uint64_t t[3];
-  uint32_t lo[3], hi[3];
-#pragma unroll
-  for (int q = 0; q < 3; ++q) {
-    t[q]  = prefix | ((static_cast<uint64_t>(key) * 4 + static_cast<uint64_t>(q + 1)) << sh);
-    lo[q] = s;
-    hi[q] = e;
-  }
-  while (lo[0] < hi[0] || lo[1] < hi[1] || lo[2] < hi[2]) {
-    uint32_t mid[3], v[3];
-#pragma unroll
-    for (int q = 0; q < 3; ++q) {
-      mid[q] = lo[q] + ((hi[q] - lo[q]) >> 1);
-      v[q]   = lo[q] < hi[q] ? K[mid[q]] : 0u;
-    }
-#pragma unroll
-    for (int q = 0; q < 3; ++q) {
-      if (lo[q] < hi[q]) {
-        if (static_cast<uint64_t>(v[q]) < t[q])
-          lo[q] = mid[q] + 1;
-        else
-          hi[q] = mid[q];
-      }
-    }
-  }
-  b1 = lo[0];
-  b2 = lo[1];
-  b3 = lo[2];
-}
-
-// thread_split over the key samples: three interleaved lower bounds on the
-// samples inside [s, e), then on the (at most 32) keys each one leaves.
-// Same results as thread_split: with a = ceil(s / 32), b = floor((e - 1) / 32)
+// Child boundaries with one thread over the key samples: three interleaved lower bounds
+// on the samples inside [s, e), then on the (at most 32) keys each one leaves.
+// With a = ceil(s / 32), b = floor((e - 1) / 32)
 // and j* the first sample in [a, b] at or above the target, the first key at or
 // above the target lies in [s, 32a] (j* = a), (32(j* - 1), 32 j*] (a < j* <= b)
 // or (32 b, e] (no sample above it).
@@ -326,10 +274,7 @@ __global__ void __launch_bounds__(256) level_split_kernel(LevelArgs a, Rule rule
       if (rule.rule(node, a.level, ms, sh, prefix) && c > ms) {
         uint32_t const s = a.nstart[node];
         uint32_t b1, b2, b3;
-        if (a.samples)
-          sampled_split(a.K, a.samples, s, s + c, a.nkey[node], sh, prefix, b1, b2, b3);
-        else
-          thread_split(a.K, s, s + c, a.nkey[node], sh, prefix, b1, b2, b3);
+        sampled_split(a.K, a.samples, s, s + c, a.nkey[node], sh, prefix, b1, b2, b3);
         sp = make_uint4(b1, b2, b3, nonempty(s, s + c, b1, b2, b3));
       }
       a.split[node] = sp;

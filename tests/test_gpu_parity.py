@@ -4,6 +4,7 @@ Bar: bit-identical quadtree columns, point_indices, bounding boxes, join pairs
 and point-in-polygon pairs (integer/index outputs and exact FP64 predicates).
 """
 
+import contextlib
 import ctypes
 
 import numpy as np
@@ -469,6 +470,35 @@ def test_float32_rejected(cs):
 
     with pytest.raises(TypeError, match="float64"):
         cs.Points(torch.zeros(3, dtype=torch.float32), torch.zeros(3, dtype=torch.float32))
+
+
+@pytest.mark.parametrize("d", [0, 1, 2, 7, 15])
+@pytest.mark.parametrize("n,ms", [(1, 1), (2, 1), (2047, 1), (2048, 2), (2049, 7), (16384, 64),
+                                  (16385, 63), (50000, 1), (50000, 16384), (50000, 60000)])
+def test_tree_starts_match_oracle(cs, oracle_mod, n, ms, d):
+    """The tree's node starts at the edges of its rounds (2,048 positions) and lists
+    (16,384), with max_size from 1 to more than the points, dense clusters, repeated
+    points, a grid's lines and a scale that puts coordinates at 2^d and above (the
+    extra root-level nodes). Every column exact."""
+    rng = np.random.default_rng(n * 31 + ms + d)
+    ext = 64.0
+    x, y = rng.uniform(0, ext, n), rng.uniform(0, ext, n)
+    k = n // 3
+    x[:k], y[:k] = 17.0 + rng.normal(0, 1e-3, k), 41.0 + rng.normal(0, 1e-3, k)
+    r = n // 4
+    x[k:k + r], y[k:k + r] = x[k], y[k]
+    x[-(n // 8 + 1):] = np.floor(x[-(n // 8 + 1):])
+    order = rng.permutation(n)
+    x, y = x[order], y[order]
+    for scale in (ext / (1 << d), 1e-9):
+        with pytest.warns(UserWarning) if scale == 1e-9 else contextlib.nullcontext():
+            pi, tree = cs.quadtree_on_points(cs.Points(x, y, device="cuda"), 0.0, ext, 0.0, ext,
+                                             scale, d, ms)
+        o = oracle_mod.quadtree_on_points(x, y, 0.0, ext, 0.0, ext, scale, d, ms)
+        assert np.array_equal(np_(pi), o[0])
+        for name, ref in zip(("key", "level", "is_internal_node", "length", "offset"), o[1:]):
+            assert np.array_equal(np_(tree[name]).astype(np.int64),
+                                  np.asarray(ref).astype(np.int64)), (name, scale)
 
 
 # ---------------------------------------------------------------------------
