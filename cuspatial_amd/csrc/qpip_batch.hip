@@ -385,22 +385,16 @@ struct TopSizeOp {
 };
 
 // Level 0 of the traversal: job j's virtual frontier i -> (i % T_j, i / T_j).
-struct BatchTopOp {
-  TreeView t;
-  BoxView bx;
-  JobGeometry g;
+struct BatchTopSource {
   JobTree const* trees;
   JobDev const* jobs;
   uint64_t const* top_off;
   uint32_t num_jobs;
-  JoinMeta* meta;
-  uint32_t* out_node;
-  uint32_t* out_bbox;
-  uint32_t* fr_node;
-  uint32_t* fr_bbox;
-  uint64_t cap_out, cap_fr;
+  JoinMeta const* meta;
 
-  __device__ void locate(uint64_t i, uint32_t& node, uint32_t& bbox) const
+  __device__ __forceinline__ uint64_t size() const { return meta->top_pairs; }
+  __device__ __forceinline__ bool root(TreeView const&, uint64_t i, uint32_t& node, uint32_t& bbox,
+                                       uint32_t& first, uint32_t& n) const
   {
     uint32_t lo = 0, hi = num_jobs - 1;  // last job with top_off <= i
     while (lo < hi) {
@@ -414,47 +408,11 @@ struct BatchTopOp {
     uint32_t const T     = trees[lo].num_top;
     node                 = trees[lo].top_first + static_cast<uint32_t>(local % T);
     bbox                 = jobs[lo].poly_begin + static_cast<uint32_t>(local / T);
-  }
-  __device__ uint64_t count(uint64_t i) const
-  {
-    uint32_t node, bbox;
-    locate(i, node, bbox);
-    int const c = classify(t, bx, g, node, bbox);
-    return c == 0 ? 1ull : (c == 1 ? (1ull << 32) : 0ull);
-  }
-  __device__ void emit(uint64_t i, uint64_t prefix) const
-  {
-    uint32_t node, bbox;
-    locate(i, node, bbox);
-    int const c = classify(t, bx, g, node, bbox);
-    if (c == 0) {
-      uint64_t const o = prefix & 0xFFFFFFFFull;
-      if (o < cap_out) {
-        out_node[o] = node;
-        out_bbox[o] = bbox;
-      } else {
-        atomicOr(&meta->overflow, 1u);
-      }
-    } else if (c == 1) {
-      uint64_t const f = prefix >> 32;
-      if (f < cap_fr) {
-        fr_node[f] = node;
-        fr_bbox[f] = bbox;
-      } else {
-        atomicOr(&meta->overflow, 1u);
-      }
-    }
+    first                = node;
+    n                    = 1;
+    return true;
   }
 };
-
-__global__ void __launch_bounds__(256)
-  gather_offsets_kernel(uint32_t const* __restrict__ out_node, uint32_t const* __restrict__ offset,
-                        uint64_t k, uint32_t* __restrict__ keys)
-{
-  for (uint64_t i = static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < k;
-       i += static_cast<uint64_t>(gridDim.x) * blockDim.x)
-    keys[i] = offset[out_node[i]];
-}
 
 __global__ void __launch_bounds__(256)
   permute_kernel(uint32_t const* __restrict__ perm, uint32_t const* __restrict__ out_node,
@@ -917,13 +875,16 @@ void run_group(std::vector<HostJob> const& hj, int64_t j0, int64_t j1, int64_t c
   dbuf<uint64_t> top_off(J);
   dbuf<JoinMeta> jmeta(1);
   dbuf<uint64_t> partials64(kScanBlocks + 1);
+  dbuf<StepCount> join_partials(kScanBlocks), join_counts;
   uint64_t cap_out = std::max<uint64_t>(uint64_t{1} << 20, 8 * npg);
   uint64_t cap_fr  = cap_out;
   JoinMeta h_meta{};
-  dbuf<uint32_t> out_node, out_bbox, fa_node, fa_bbox, fb_node, fb_bbox;
+  dbuf<uint32_t> out_node, out_bbox, ka, fa_node, fa_bbox, fb_node, fb_bbox;
   for (int attempt = 0;; ++attempt) {
     out_node.reset(cap_out);
     out_bbox.reset(cap_out);
+    ka.reset(cap_out);
+    join_counts.reset(cap_fr);
     fa_node.reset(cap_fr);
     fa_bbox.reset(cap_fr);
     fb_node.reset(cap_fr);
@@ -934,24 +895,12 @@ void run_group(std::vector<HostJob> const& hj, int64_t j0, int64_t j1, int64_t c
     count_scan_emit<TopSizeOp, uint64_t, uint64_t>(ts, nullptr, J, partials64.get(),
                                                    &dm->top_pairs, stream, scan_blocks_for(J),
                                                    "batch_join_setup");
-    BatchTopOp top{tv, bv, geom, trees.get(), jobs.get(), top_off.get(), J, dm, out_node.get(),
-                   out_bbox.get(), fa_node.get(), fa_bbox.get(), cap_out, cap_fr};
-    count_scan_emit<BatchTopOp, uint64_t, SplitTotal>(top, &dm->top_pairs, 0, partials64.get(),
-                                                      &dm->level[0], stream, kScanBlocks,
-                                                      "batch_join_level");
-    uint32_t* cur_node = fa_node.get();
-    uint32_t* cur_bbox = fa_bbox.get();
-    uint32_t* nxt_node = fb_node.get();
-    uint32_t* nxt_bbox = fb_bbox.get();
-    for (int lvl = 1; lvl < maxd; ++lvl) {
-      DescendOp<JobGeometry> op{tv, bv, geom, dm, cur_node, cur_bbox, out_node.get(),
-                                out_bbox.get(), nxt_node, nxt_bbox, cap_out, cap_fr, lvl};
-      count_scan_emit<DescendOp<JobGeometry>, uint64_t, SplitTotal>(
-        op, &dm->level[lvl - 1].quad, 0, partials64.get(), &dm->level[lvl], stream, kScanBlocks,
-        "batch_join_level");
-      std::swap(cur_node, nxt_node);
-      std::swap(cur_bbox, nxt_bbox);
-    }
+    BatchTopSource const top{trees.get(), jobs.get(), top_off.get(), J, dm};
+    JoinSink const sink{dm, out_node.get(), out_bbox.get(), ka.get(), nullptr, nullptr,
+                        join_counts.get(), cap_out, cap_fr, 0, 0};
+    launch_join(top, tv, bv, geom, sink, {fa_node.get(), fb_node.get()},
+                {fa_bbox.get(), fb_bbox.get()}, std::max(maxd, 1), join_partials.get(),
+                stream, "batch_join_level");
     QPIP_HIP(hipMemcpyAsync(&h_meta, dm, sizeof(JoinMeta), hipMemcpyDeviceToHost, stream));
     QPIP_HIP(hipStreamSynchronize(stream));
     if (h_meta.bad_index) throw logic_error("cuSpatial failure: forest child range out of range");
@@ -969,10 +918,7 @@ void run_group(std::vector<HostJob> const& hj, int64_t j0, int64_t j1, int64_t c
   for (int l = 0; l < std::max(maxd, 1); ++l) K += h_meta.level[l].leaf;
   if (K == 0) return;
   QPIP_EXPECTS(K < (uint64_t{1} << 32), "join produced more than 2^32 pairs");
-  dbuf<uint32_t> ka(K), kb(K), va(K), vb(K), pb(K), pq(K);
-  gather_offsets_kernel<<<grid_for(K, 256), 256, 0, stream>>>(out_node.get(), f_offset.get(), K,
-                                                              ka.get());
-  QPIP_LAUNCH_CHECK();
+  dbuf<uint32_t> kb(K), va(K), vb(K), pb(K), pq(K);
   SortResult ps = radix_sort_pairs(ka.get(), kb.get(), nullptr, va.get(), vb.get(), K,
                                    std::max(1, bits_for(n)), stream, nullptr, "batch_join_sort");
   permute_kernel<<<grid_for(K, 256), 256, 0, stream>>>(ps.values, out_node.get(), out_bbox.get(),
@@ -1162,6 +1108,7 @@ struct PlanGroup {
   dbuf<double> boxes;
   // join and pair sort (capacity-sized)
   dbuf<uint64_t> top_off, partials64;
+  dbuf<StepCount> join_partials, join_counts;
   dbuf<JoinMeta> jmeta;
   dbuf<uint32_t> out_node, out_bbox, fa_node, fa_bbox, fb_node, fb_bbox;
   dbuf<uint32_t> ka, kb, va, vb, pb, pq, pair_counts, pair_sums;
@@ -1236,6 +1183,7 @@ void plan_alloc(PlanGroup& g)
   g.out_node.reset(c.pairs);
   g.out_bbox.reset(c.pairs);
   g.fa_node.reset(c.frontier);
+  g.join_counts.reset(c.frontier);
   g.fa_bbox.reset(c.frontier);
   g.fb_node.reset(c.frontier);
   g.fb_bbox.reset(c.frontier);
@@ -1338,26 +1286,11 @@ void plan_enqueue(BatchPlan& P, PlanGroup& g, size_t gi, hipStream_t s)
   count_scan_emit<TopSizeOp, uint64_t, uint64_t>(ts, nullptr, g.J, g.partials64.get(),
                                                  &dm->top_pairs, s, scan_blocks_for(g.J),
                                                  "batch_join_setup");
-  BatchTopOp top{tv, bv, geom, g.trees.get(), g.jobs.get(), g.top_off.get(), g.J, dm,
-                 g.out_node.get(), g.out_bbox.get(), g.fa_node.get(), g.fa_bbox.get(),
-                 g.cap.pairs, g.cap.frontier};
-  count_scan_emit<BatchTopOp, uint64_t, SplitTotal>(top, &dm->top_pairs, 0, g.partials64.get(),
-                                                    &dm->level[0], s, kScanBlocks,
-                                                    "batch_join_level");
-  uint32_t* cur_node = g.fa_node.get();
-  uint32_t* cur_bbox = g.fa_bbox.get();
-  uint32_t* nxt_node = g.fb_node.get();
-  uint32_t* nxt_bbox = g.fb_bbox.get();
-  for (int lvl = 1; lvl < g.maxd; ++lvl) {
-    DescendOp<JobGeometry> op{tv, bv, geom, dm, cur_node, cur_bbox, g.out_node.get(),
-                              g.out_bbox.get(), nxt_node, nxt_bbox, g.cap.pairs, g.cap.frontier,
-                              lvl};
-    count_scan_emit<DescendOp<JobGeometry>, uint64_t, SplitTotal>(
-      op, &dm->level[lvl - 1].quad, 0, g.partials64.get(), &dm->level[lvl], s, kScanBlocks,
-      "batch_join_level");
-    std::swap(cur_node, nxt_node);
-    std::swap(cur_bbox, nxt_bbox);
-  }
+  BatchTopSource const top{g.trees.get(), g.jobs.get(), g.top_off.get(), g.J, dm};
+  JoinSink const sink{dm, g.out_node.get(), g.out_bbox.get(), nullptr, nullptr, nullptr,
+                      g.join_counts.get(), g.cap.pairs, g.cap.frontier, 0, 0};
+  launch_join(top, tv, bv, geom, sink, {g.fa_node.get(), g.fb_node.get()},
+              {g.fa_bbox.get(), g.fb_bbox.get()}, levels, g.join_partials.get(), s, "batch_join_level");
   plan_pairs_kernel<<<1, 64, 0, s>>>(dm, levels, g.cap.pairs, g.fmeta.get(), cnt, prev);
   QPIP_LAUNCH_CHECK();
   plan_gather_kernel<<<grid_for(g.cap.pairs, 256), 256, 0, s>>>(
@@ -1501,6 +1434,7 @@ void plan_group_setup(BatchPlan& P, PlanGroup& g, hipStream_t s)
   QPIP_HIP(hipStreamSynchronize(s));  // prefix is freed on return
   g.top_off.reset(g.J);
   g.partials64.reset(kScanBlocks + 1);
+  g.join_partials.reset(kScanBlocks);
   g.jmeta.reset(1);
   g.pip_partials.reset(kScanBlocks + 1);
   g.pip_totals.reset(2);

@@ -9,10 +9,8 @@
 // point position.
 //
 // Here the same traversal runs entirely on the device, one count/scan/emit per
-// level with the frontier length kept in device memory (the reference syncs the
-// host on every level for sizes, traversal.cuh:222). Each frontier element counts
-// its leaf and quad children in one packed 64-bit value, so a single scan gives
-// both output positions and the emission order is the reference's. The stable
+// kJoinStep levels (qpip_join.hpp) with the frontier length kept in device memory (the
+// reference syncs the host on every level for sizes, traversal.cuh:222). The stable
 // sort is the library's LSD radix sort over the bits of the largest leaf offset.
 // Frontier/output capacities are preallocated; on overflow the traversal is
 // rerun with the sizes the device recorded.
@@ -24,84 +22,61 @@ namespace qpip {
 
 namespace {
 
-// Level 0: the virtual frontier i -> (i % T, i / T), each pair classified once.
-struct TopOp {
-  TreeView t;
-  BoxView bx;
-  Params p;
-  JoinMeta* meta;
-  uint32_t* out_node;
-  uint32_t* out_bbox;
-  uint32_t* fr_node;
-  uint32_t* fr_bbox;
-  uint64_t cap_out, cap_fr;
-
-  __device__ uint64_t count(uint64_t i) const
+// Level 0: the virtual frontier i -> (i % T, i / T).
+struct TopSource {
+  JoinMeta const* meta;
+  __device__ __forceinline__ uint64_t size() const { return meta->top_pairs; }
+  __device__ __forceinline__ bool root(TreeView const&, uint64_t i, uint32_t& node, uint32_t& bbox,
+                                       uint32_t& first, uint32_t& n) const
   {
     uint32_t const T = meta->num_top;
-    int const c      = classify(t, bx, p, static_cast<uint32_t>(i % T), static_cast<uint32_t>(i / T));
-    return c == 0 ? 1ull : (c == 1 ? (1ull << 32) : 0ull);
-  }
-  __device__ void emit(uint64_t i, uint64_t prefix) const
-  {
-    uint32_t const T    = meta->num_top;
-    uint32_t const node = static_cast<uint32_t>(i % T);
-    uint32_t const bbox = static_cast<uint32_t>(i / T);
-    int const c         = classify(t, bx, p, node, bbox);
-    if (c == 0) {
-      uint64_t const o = prefix & 0xFFFFFFFFull;
-      if (o < cap_out) {
-        out_node[o] = node;
-        out_bbox[o] = bbox;
-      } else {
-        atomicOr(&meta->overflow, 1u);
-      }
-    } else if (c == 1) {
-      uint64_t const f = prefix >> 32;
-      if (f < cap_fr) {
-        fr_node[f] = node;
-        fr_bbox[f] = bbox;
-      } else {
-        atomicOr(&meta->overflow, 1u);
-      }
-    }
+    node             = static_cast<uint32_t>(i % T);
+    bbox             = static_cast<uint32_t>(i / T);
+    first            = node;
+    n                = 1;
+    return true;
   }
 };
 
-// T = count(level == 0) (quadtree_bbox_filtering.cuh:53-56) and the largest
-// leaf offset (for the sort's bit count).
-struct TopCountOp {
-  uint8_t const* level;
-  __device__ uint32_t count(uint64_t i) const { return level[i] == 0 ? 1u : 0u; }
-  __device__ void emit(uint64_t, uint32_t) const {}
-};
-
+// T = count(level == 0) (quadtree_bbox_filtering.cuh:53-56), T * B and the largest leaf
+// offset (for the sort's bit count), into a zeroed *meta. One atomic per block and
+// value; the last block to finish writes the product. (One atomic per wave on the
+// largest offset took 50 us for 1.2M nodes, next to four launches for the rest.)
 __global__ void __launch_bounds__(256)
-  leaf_offset_max_kernel(uint8_t const* __restrict__ internal, uint32_t const* __restrict__ offset,
-                         uint64_t m, JoinMeta* __restrict__ meta)
+  join_setup_kernel(uint8_t const* __restrict__ level, uint8_t const* __restrict__ internal,
+                    uint32_t const* __restrict__ offset, uint64_t m, uint64_t boxes,
+                    JoinMeta* __restrict__ meta)
 {
-  uint32_t mx = 0;
+  __shared__ uint32_t s_top[256 / kWave], s_max[256 / kWave];
+  uint32_t top = 0, mx = 0;
+#pragma unroll 4
   for (uint64_t i = static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < m;
-       i += static_cast<uint64_t>(gridDim.x) * blockDim.x)
-    if (!internal[i]) mx = max(mx, offset[i]);
+       i += static_cast<uint64_t>(gridDim.x) * blockDim.x) {
+    uint32_t const o = offset[i];
+    top += level[i] == 0 ? 1u : 0u;
+    if (!internal[i]) mx = max(mx, o);
+  }
+  top = wave_sum(top);
 #pragma unroll
-  for (int o = kWave / 2; o > 0; o >>= 1) mx = max(mx, static_cast<uint32_t>(__shfl_xor(mx, o, kWave)));
-  if (lane_id() == 0) atomicMax(&meta->max_leaf_offset, mx);
-}
-
-__global__ void setup_kernel(JoinMeta* meta, uint32_t const* num_top, uint64_t b)
-{
-  meta->num_top   = *num_top;
-  meta->top_pairs = static_cast<uint64_t>(*num_top) * b;
-}
-
-__global__ void __launch_bounds__(256)
-  gather_keys_kernel(uint32_t const* __restrict__ out_node, uint32_t const* __restrict__ offset,
-                     uint64_t k, uint32_t* __restrict__ keys)
-{
-  for (uint64_t i = static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < k;
-       i += static_cast<uint64_t>(gridDim.x) * blockDim.x)
-    keys[i] = offset[out_node[i]];
+  for (int o = kWave / 2; o > 0; o >>= 1)
+    mx = max(mx, static_cast<uint32_t>(__shfl_xor(mx, o, kWave)));
+  if (lane_id() == 0) {
+    s_top[threadIdx.x / kWave] = top;
+    s_max[threadIdx.x / kWave] = mx;
+  }
+  __syncthreads();
+  if (threadIdx.x != 0) return;
+  for (int w = 1; w < 256 / kWave; ++w) {
+    top += s_top[w];
+    mx = max(mx, s_max[w]);
+  }
+  if (top) atomicAdd(&meta->num_top, top);
+  if (mx) atomicMax(&meta->max_leaf_offset, mx);
+  __threadfence();
+  if (atomicAdd(&meta->tickets, 1u) + 1 == gridDim.x) {
+    __threadfence();
+    meta->top_pairs = static_cast<uint64_t>(atomicAdd(&meta->num_top, 0u)) * boxes;
+  }
 }
 
 __global__ void __launch_bounds__(256)
@@ -166,50 +141,34 @@ extern "C" int qpip_join_quadtree_and_bounding_boxes(const uint32_t* key,
     uint64_t const B = static_cast<uint64_t>(num_bboxes);
 
     dbuf<JoinMeta> meta(1);
-    dbuf<uint64_t> partials64(kScanBlocks + 1);
-    dbuf<uint32_t> partials32(kScanBlocks + 1);
-    dbuf<uint32_t> num_top(1);
+    dbuf<StepCount> partials(kScanBlocks), counts;
 
     uint64_t cap_out = std::max<uint64_t>(uint64_t{1} << 20, 8 * B);
     uint64_t cap_fr  = std::max<uint64_t>(uint64_t{1} << 20, 8 * B);
     JoinMeta h_meta{};
-    dbuf<uint32_t> out_node, out_bbox, fa_node, fa_bbox, fb_node, fb_bbox;
+    dbuf<uint32_t> out_node, out_bbox, ka, fa_node, fa_bbox, fb_node, fb_bbox;
     for (int attempt = 0;; ++attempt) {
       out_node.reset(cap_out);
       out_bbox.reset(cap_out);
+      ka.reset(cap_out);
+      counts.reset(cap_fr);
       fa_node.reset(cap_fr);
       fa_bbox.reset(cap_fr);
       fb_node.reset(cap_fr);
       fb_bbox.reset(cap_fr);
       QPIP_HIP(hipMemsetAsync(meta.get(), 0, sizeof(JoinMeta), stream));
-      count_scan_emit<TopCountOp, uint32_t, uint32_t>(TopCountOp{level}, nullptr, M,
-                                                      partials32.get(), num_top.get(), stream,
-                                                      scan_blocks_for(M), "join_setup");
-      setup_kernel<<<1, 1, 0, stream>>>(meta.get(), num_top.get(), B);
-      QPIP_LAUNCH_CHECK();
-      leaf_offset_max_kernel<<<grid_for(M, 256, 1024), 256, 0, stream>>>(is_internal_node, offset,
-                                                                         M, meta.get());
-      QPIP_LAUNCH_CHECK();
       JoinMeta* dm = meta.get();
-      TopOp top{tv, bv, prm, dm, out_node.get(), out_bbox.get(), fa_node.get(), fa_bbox.get(),
-                cap_out, cap_fr};
-      count_scan_emit<TopOp, uint64_t, SplitTotal>(top, &dm->top_pairs, 0, partials64.get(),
-                                                   &dm->level[0], stream, kScanBlocks,
-                                                   "join_level");
-      uint32_t* cur_node = fa_node.get();
-      uint32_t* cur_bbox = fa_bbox.get();
-      uint32_t* nxt_node = fb_node.get();
-      uint32_t* nxt_bbox = fb_bbox.get();
-      // quadtree_bbox_filtering.cuh:116-163: levels 1 .. max_depth-1
-      for (int lvl = 1; lvl < max_depth; ++lvl) {
-        DescendOp<Params> op{tv, bv, prm, dm, cur_node, cur_bbox, out_node.get(), out_bbox.get(),
-                             nxt_node, nxt_bbox, cap_out, cap_fr, lvl};
-        count_scan_emit<DescendOp<Params>, uint64_t, SplitTotal>(op, &dm->level[lvl - 1].quad, 0,
-                                                         partials64.get(), &dm->level[lvl], stream,
-                                                         kScanBlocks, "join_level");
-        std::swap(cur_node, nxt_node);
-        std::swap(cur_bbox, nxt_bbox);
+      {
+        KernelTimer kt("join_setup", stream);
+        join_setup_kernel<<<grid_for(M, 4 * 256, 256), 256, 0, stream>>>(level, is_internal_node,
+                                                                         offset, M, B, dm);
+        QPIP_LAUNCH_CHECK();
       }
+      // quadtree_bbox_filtering.cuh:116-163: levels 0 .. max_depth - 1
+      JoinSink const sink{dm, out_node.get(), out_bbox.get(), ka.get(), nullptr, nullptr,
+                          counts.get(), cap_out, cap_fr, 0, 0};
+      launch_join(TopSource{dm}, tv, bv, prm, sink, {fa_node.get(), fb_node.get()},
+                  {fa_bbox.get(), fb_bbox.get()}, max_depth, partials.get(), stream, "join_level");
       QPIP_HIP(hipMemcpyAsync(&h_meta, dm, sizeof(JoinMeta), hipMemcpyDeviceToHost, stream));
       QPIP_HIP(hipStreamSynchronize(stream));
       if (h_meta.bad_index)
@@ -231,9 +190,7 @@ extern "C" int qpip_join_quadtree_and_bounding_boxes(const uint32_t* key,
     QPIP_EXPECTS(K < (uint64_t{1} << 32), "join produced more than 2^32 pairs");
 
     // stable_sort_by_key(offset[leaf], (bbox, leaf)) (quadtree_bbox_filtering.cuh:152-166)
-    dbuf<uint32_t> ka(K), kb(K), va(K), vb(K);
-    gather_keys_kernel<<<grid_for(K, 256), 256, 0, stream>>>(out_node.get(), offset, K, ka.get());
-    QPIP_LAUNCH_CHECK();
+    dbuf<uint32_t> kb(K), va(K), vb(K);
     int bits = 1;
     while (bits < 32 && (h_meta.max_leaf_offset >> bits) != 0) ++bits;
     SortResult s = radix_sort_pairs(ka.get(), kb.get(), nullptr, va.get(), vb.get(), K, bits,
