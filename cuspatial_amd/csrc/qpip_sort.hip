@@ -18,6 +18,8 @@
 //             digit's run at its position.
 // The first pass's counts usually come from the producer of the keys (the keygen
 // kernel counts digit 0 while it writes the keys).
+// Few tiles: up to kSelfTiles the scatter blocks sum the earlier tiles' counts themselves
+// (no colscan launches), and up to one tile a single workgroup runs every pass in LDS.
 #include <algorithm>
 #include <string>
 #include <vector>
@@ -42,6 +44,9 @@ __global__ void fill_u32_kernel(uint32_t* __restrict__ p, uint64_t n, uint32_t v
 
 constexpr int kScanRows = 64;  // tiles per column-scan group
 constexpr int kBatch    = 8;   // loads in flight per thread in the column scans
+// Tiles up to which a scatter block sums all tiles' counts itself: at 128 its 16 rounds
+// of loads take about as long as the three colscan launches (8 us and their gaps).
+constexpr uint64_t kSelfTiles = 128;
 
 // Digit counts of one tile. `vec`: the keys are 16-byte aligned (full tiles are
 // then read as uint4).
@@ -172,16 +177,16 @@ __global__ void __launch_bounds__(kRadix)
   }
 }
 
-// Ranks one tile: keys/values in registers, per-wave digit counts in s_wcount_w,
+// Ranks one tile by digits of at most NB bits (`mask`): keys/values in registers, per-wave digit counts in s_wcount_w,
 // rank[j] = position of item j among equal digits within its wave (stable).
 template <int NB>
 __device__ __forceinline__ void rank_tile(uint32_t const* __restrict__ keys_in,
                                           uint32_t const* __restrict__ vals_in, uint64_t n,
-                                          uint64_t base, int shift, uint32_t (&key)[kSortItems],
+                                          uint64_t base, int shift, uint32_t mask,
+                                          uint32_t (&key)[kSortItems],
                                           uint32_t (&val)[kSortItems],
                                           uint32_t (&rank)[kSortItems], uint32_t* s_wcount_w)
 {
-  uint32_t const mask = (1u << NB) - 1u;
   int const lane      = lane_id();
   uint64_t const lt   = lanemask_lt();
 #pragma unroll
@@ -220,7 +225,9 @@ __device__ __forceinline__ uint64_t xcd_tile(uint64_t b, uint64_t tiles)
 // segment's first position is written there too (with `local_out`, in place of
 // the value itself); `key_samples`, when given, receives the key written at
 // every position that is a multiple of 32.
-template <int NB, bool SEG>
+// SELF: `offsets` holds the tiles' plain counts, and each block derives its own row of
+// first output positions from all of them.
+template <int NB, bool SEG, bool SELF = false>
 __global__ void __launch_bounds__(kSortThreads)
   radix_scatter_kernel(uint32_t const* __restrict__ keys_in,
                        uint32_t const* __restrict__ vals_in,  // null: identity
@@ -249,7 +256,23 @@ __global__ void __launch_bounds__(kSortThreads)
   int const lane      = lane_id();
   int const d         = threadIdx.x;  // kSortThreads == kRadix: one digit per thread
   uint64_t const tile = xcd_tile(blockIdx.x, gridDim.x);
-  s_global[d]         = offsets[tile * kRadix + d];
+  if constexpr (SELF) {
+    uint32_t before = 0, all = 0, sum;
+    for (uint32_t t = 0; t < gridDim.x; t += kBatch) {
+      uint32_t v[kBatch];
+#pragma unroll
+      for (int u = 0; u < kBatch; ++u)
+        v[u] = t + u < gridDim.x ? offsets[static_cast<uint64_t>(t + u) * kRadix + d] : 0u;
+#pragma unroll
+      for (int u = 0; u < kBatch; ++u) {
+        before += t + u < tile ? v[u] : 0u;
+        all += v[u];
+      }
+    }
+    s_global[d] = before + block_excl_scan<kSortThreads>(all, s_scan, &sum);
+  } else {
+    s_global[d] = offsets[tile * kRadix + d];
+  }
 #pragma unroll
   for (int ww = 0; ww < NW; ++ww) s_wcount[ww][d] = 0;
   __syncthreads();
@@ -266,7 +289,7 @@ __global__ void __launch_bounds__(kSortThreads)
   }
   uint64_t const base = tile_lo + static_cast<uint64_t>(w) * (kSortItems * kWave);
   uint32_t key[kSortItems], val[kSortItems], rank[kSortItems];
-  rank_tile<NB>(keys_in, vals_in, end, base, shift, key, val, rank, s_wcount[w]);
+  rank_tile<NB>(keys_in, vals_in, end, base, shift, mask, key, val, rank, s_wcount[w]);
   __syncthreads();
   // per digit: exclusive prefix over waves and the tile's first slot of the digit
   uint32_t count = 0;
@@ -307,6 +330,60 @@ __global__ void __launch_bounds__(kSortThreads)
       if (SEG && vals_local) vals_local[pos] = v - seg_begin;
       if (SEG && key_samples && (pos & 31u) == 0) key_samples[pos >> 5] = ko;
     }
+  }
+}
+
+// At most one tile of pairs, every pass in one workgroup: the pairs stay in LDS between
+// the passes. 1,000 pairs of 10 bits: 10 launches (two passes of five) before, one now.
+__global__ void __launch_bounds__(kSortThreads)
+  radix_single_kernel(uint32_t const* keys_in, uint32_t const* vals_in,  // null: identity
+                      uint32_t* keys_out, uint32_t* vals_out, uint32_t n, int bits)
+{
+  constexpr int NW = kSortThreads / kWave;
+  __shared__ uint32_t s_keys[kSortTile];
+  __shared__ uint32_t s_vals[kSortTile];
+  __shared__ uint32_t s_wcount[NW][kRadix];
+  __shared__ uint32_t s_scan[NW + 1];
+  int const w = threadIdx.x / kWave, lane = lane_id(), d = threadIdx.x;
+  uint32_t const base = static_cast<uint32_t>(w) * (kSortItems * kWave);
+  for (uint32_t i = threadIdx.x; i < n; i += kSortThreads) {
+    s_keys[i] = keys_in[i];
+    s_vals[i] = vals_in ? vals_in[i] : i;
+  }
+  for (int shift = 0; shift < bits; shift += kRadixBits) {
+    uint32_t const mask = bits - shift < kRadixBits ? (1u << (bits - shift)) - 1u : kRadix - 1u;
+#pragma unroll
+    for (int ww = 0; ww < NW; ++ww) s_wcount[ww][d] = 0;
+    __syncthreads();
+    uint32_t key[kSortItems], val[kSortItems], rank[kSortItems];
+    rank_tile<kRadixBits>(s_keys, s_vals, n, base, shift, mask, key, val, rank, s_wcount[w]);
+    __syncthreads();
+    // per digit: its first slot, then each wave's
+    uint32_t count = 0;
+#pragma unroll
+    for (int ww = 0; ww < NW; ++ww) count += s_wcount[ww][d];
+    uint32_t tot;
+    uint32_t run = block_excl_scan<kSortThreads>(count, s_scan, &tot);
+#pragma unroll
+    for (int ww = 0; ww < NW; ++ww) {
+      uint32_t const c = s_wcount[ww][d];
+      s_wcount[ww][d]  = run;
+      run += c;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < kSortItems; ++j) {
+      if (base + j * kWave + lane < n) {
+        uint32_t const loc = s_wcount[w][digit_of(key[j], shift, mask)] + rank[j];
+        s_keys[loc]        = key[j];
+        s_vals[loc]        = val[j];
+      }
+    }
+    __syncthreads();
+  }
+  for (uint32_t i = threadIdx.x; i < n; i += kSortThreads) {
+    keys_out[i] = s_keys[i];
+    vals_out[i] = s_vals[i];
   }
 }
 
@@ -424,6 +501,14 @@ SortResult radix_sort_pairs(uint32_t* keys_a,
   std::string const t_count   = std::string(tag) + "_count";
   std::string const t_scan    = std::string(tag) + "_colscan";
   std::string const t_scatter = std::string(tag) + "_scatter";
+  if (tiles == 1) {
+    KernelTimer kt(t_scatter.c_str(), stream);
+    radix_single_kernel<<<1, kSortThreads, 0, stream>>>(keys_a, values_in, keys_b, values_out,
+                                                        static_cast<uint32_t>(n), bits);
+    QPIP_LAUNCH_CHECK();
+    return {keys_b, values_out};
+  }
+  bool const self = tiles <= kSelfTiles;
 
   // the last pass writes values_out
   auto vdst_of = [&](int p) { return ((passes - 1 - p) % 2 == 0) ? values_out : values_tmp; };
@@ -449,7 +534,7 @@ SortResult radix_sort_pairs(uint32_t* keys_a,
         ksrc, n, shift, mask, vec, counts);
       QPIP_LAUNCH_CHECK();
     }
-    {
+    if (!self) {
       KernelTimer kt(t_scan.c_str(), stream);
       colscan_reduce_kernel<<<static_cast<unsigned>(groups), kRadix, 0, stream>>>(counts, tiles,
                                                                                sums);
@@ -462,10 +547,18 @@ SortResult radix_sort_pairs(uint32_t* keys_a,
     }
     {
       KernelTimer kt(t_scatter.c_str(), stream);
-#define QPIP_SCATTER(NB)                                                                      \
-  radix_scatter_kernel<NB, false><<<static_cast<unsigned>(tiles), kSortThreads, 0, stream>>>( \
-    ksrc, vsrc, kdst, vdst, n, shift, counts, nullptr, nullptr, false, nullptr, nullptr, false)
-      QPIP_DISPATCH_NB(nb, QPIP_SCATTER);
+#define QPIP_SCATTER(NB, SELF)                                            \
+  radix_scatter_kernel<NB, false, SELF>                                   \
+    <<<static_cast<unsigned>(tiles), kSortThreads, 0, stream>>>(          \
+      ksrc, vsrc, kdst, vdst, n, shift, counts, nullptr, nullptr, false, nullptr, nullptr, false)
+#define QPIP_SCATTER_SELF(NB) QPIP_SCATTER(NB, true)
+#define QPIP_SCATTER_SCAN(NB) QPIP_SCATTER(NB, false)
+      if (self)
+        QPIP_DISPATCH_NB(nb, QPIP_SCATTER_SELF)
+      else
+        QPIP_DISPATCH_NB(nb, QPIP_SCATTER_SCAN)
+#undef QPIP_SCATTER_SCAN
+#undef QPIP_SCATTER_SELF
 #undef QPIP_SCATTER
       QPIP_LAUNCH_CHECK();
     }

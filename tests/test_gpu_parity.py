@@ -501,6 +501,28 @@ def test_tree_starts_match_oracle(cs, oracle_mod, n, ms, d):
                                   np.asarray(ref).astype(np.int64)), (name, scale)
 
 
+@pytest.mark.parametrize("bits", [1, 8, 10, 17, 32])
+@pytest.mark.parametrize("n", [1, 63, 4095, 4096, 4097, 8192, 128 * 4096, 128 * 4096 + 1])
+def test_sort_pairs_stable_at_tile_edges(cs, n, bits):
+    """The radix sort at its edges: one workgroup up to a tile of 4,096 pairs, blocks
+    that sum the tiles' counts themselves up to 128 tiles, the column scans above.
+    Stable on the low bits, exact against numpy."""
+    import torch
+
+    from cuspatial_amd import _capi
+
+    rng = np.random.default_rng(n + bits)
+    k = rng.integers(0, 1 << bits, n, dtype=np.uint64)
+    k[: n // 3] = k[0]  # long runs of one key
+    v = rng.integers(0, 1 << 32, n, dtype=np.uint64)
+    kt = torch.as_tensor(k.astype(np.uint32).view(np.int32), device="cuda")
+    vt = torch.as_tensor(v.astype(np.uint32).view(np.int32), device="cuda")
+    _capi.sort_pairs(kt, vt, bits)
+    order = np.argsort(k, kind="stable")
+    assert np.array_equal(np_(kt).view(np.uint32), k[order].astype(np.uint32))
+    assert np.array_equal(np_(vt).view(np.uint32), v[order].astype(np.uint32))
+
+
 # ---------------------------------------------------------------------------
 # brute-force point-in-polygon (every point x every polygon; pairwise)
 # ---------------------------------------------------------------------------
