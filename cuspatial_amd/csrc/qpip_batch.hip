@@ -822,8 +822,7 @@ void run_group(std::vector<HostJob> const& hj, int64_t j0, int64_t j1, int64_t c
     }
   }
   ForestMeta hm;
-  QPIP_HIP(hipMemcpyAsync(&hm, fmeta.get(), sizeof(ForestMeta), hipMemcpyDeviceToHost, stream));
-  QPIP_HIP(hipStreamSynchronize(stream));
+  read_back({{&hm, fmeta.get(), sizeof(ForestMeta)}}, stream);
   if (hm.overflow) throw device_error("batched forest node capacity exceeded (internal error)");
   uint64_t M = 0;
   for (int l = 0; l < std::max(maxd, 1); ++l) M += hm.sizes[l];
@@ -901,8 +900,7 @@ void run_group(std::vector<HostJob> const& hj, int64_t j0, int64_t j1, int64_t c
     launch_join(top, tv, bv, geom, sink, {fa_node.get(), fb_node.get()},
                 {fa_bbox.get(), fb_bbox.get()}, std::max(maxd, 1), join_partials.get(),
                 stream, "batch_join_level");
-    QPIP_HIP(hipMemcpyAsync(&h_meta, dm, sizeof(JoinMeta), hipMemcpyDeviceToHost, stream));
-    QPIP_HIP(hipStreamSynchronize(stream));
+    read_back({{&h_meta, dm, sizeof(JoinMeta)}}, stream);
     if (h_meta.bad_index) throw logic_error("cuSpatial failure: forest child range out of range");
     if (!h_meta.overflow) break;
     uint64_t tot_out = 0, max_fr = h_meta.top_pairs;
@@ -957,9 +955,7 @@ void run_group(std::vector<HostJob> const& hj, int64_t j0, int64_t j1, int64_t c
   job_hit_offsets_kernel<<<(J + 255) / 256, 256, 0, stream>>>(ht, h, jobs.get(), J, first.get());
   QPIP_LAUNCH_CHECK();
   std::vector<uint64_t> hf(J);
-  QPIP_HIP(hipMemcpyAsync(hf.data(), first.get(), J * sizeof(uint64_t), hipMemcpyDeviceToHost,
-                          stream));
-  QPIP_HIP(hipStreamSynchronize(stream));
+  read_back({{hf.data(), first.get(), J * sizeof(uint64_t)}}, stream);
   for (uint32_t k = 0; k < J; ++k) job_hits[j0 + k] = (k + 1 < J ? hf[k + 1] : h) - hf[k];
 }
 
@@ -1787,11 +1783,9 @@ extern "C" int qpip_batch_plan_result(qpip_batch_plan* plan,
     std::vector<int64_t> first(static_cast<size_t>(P.num_jobs));
     // Copies on the caller's stream, never the legacy stream: another thread may be
     // capturing a plan, and a legacy-stream copy would have to wait on its stream.
-    QPIP_HIP(hipMemcpyAsync(hc.data(), P.counts.get(), G * sizeof(DeviceCounts),
-                            hipMemcpyDeviceToHost, rs));
-    QPIP_HIP(hipMemcpyAsync(first.data(), P.job_first.get(), first.size() * sizeof(int64_t),
-                            hipMemcpyDeviceToHost, rs));
-    QPIP_HIP(hipStreamSynchronize(rs));
+    read_back({{hc.data(), P.counts.get(), G * sizeof(DeviceCounts)},
+               {first.data(), P.job_first.get(), first.size() * sizeof(int64_t)}},
+              rs);
     uint32_t flags = 0;
     for (auto const& c : hc) flags |= c.flags;
     if (flags & 1u) throw logic_error("cuSpatial failure: forest child range or index out of range");

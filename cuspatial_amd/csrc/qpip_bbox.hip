@@ -182,8 +182,7 @@ extern "C" int qpip_polygon_bounding_boxes(const int32_t* poly_offsets,
       QPIP_LAUNCH_CHECK();
     }
     uint32_t h_flags[2];
-    QPIP_HIP(hipMemcpyAsync(h_flags, flags.get(), sizeof(h_flags), hipMemcpyDeviceToHost, stream));
-    QPIP_HIP(hipStreamSynchronize(stream));
+    read_back({{h_flags, flags.get(), sizeof(h_flags)}}, stream);
     if (h_flags[1])  // the outputs are released by `oa`
       throw logic_error("cuSpatial failure: polygon offset out of range of ring offsets");
     oa.keep();

@@ -7,6 +7,7 @@
 
 #include <cstddef>
 #include <cstdint>
+#include <initializer_list>
 #include <stdexcept>
 #include <string>
 #include <vector>
@@ -133,6 +134,18 @@ void pool_set_limit(size_t bytes);
 void pool_trim();
 size_t pool_bytes_in_use();
 void pool_stats(size_t* live, size_t* cached);
+
+// Copies small device results (sizes, flags: 4-byte aligned, whole words) to host
+// memory and waits for the stream: one kernel writes them into pinned host memory
+// (a block taken from a list that grows to the number of concurrent calls and is
+// given back by pool_trim). A hipMemcpyAsync into pageable memory stages and waits by
+// itself: 10 to 15 us of a call's host time each. Not for a stream that captures.
+struct ReadBack {
+  void* dst;
+  void const* src;
+  size_t bytes;
+};
+void read_back(std::initializer_list<ReadBack> parts, hipStream_t stream);
 
 class StreamScope {
  public:

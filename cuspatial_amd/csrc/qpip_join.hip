@@ -169,8 +169,7 @@ extern "C" int qpip_join_quadtree_and_bounding_boxes(const uint32_t* key,
                           counts.get(), cap_out, cap_fr, 0, 0};
       launch_join(TopSource{dm}, tv, bv, prm, sink, {fa_node.get(), fb_node.get()},
                   {fa_bbox.get(), fb_bbox.get()}, max_depth, partials.get(), stream, "join_level");
-      QPIP_HIP(hipMemcpyAsync(&h_meta, dm, sizeof(JoinMeta), hipMemcpyDeviceToHost, stream));
-      QPIP_HIP(hipStreamSynchronize(stream));
+      read_back({{&h_meta, dm, sizeof(JoinMeta)}}, stream);
       if (h_meta.bad_index)
         throw logic_error("cuSpatial failure: quadtree child range exceeds the number of nodes");
       if (!h_meta.overflow) break;

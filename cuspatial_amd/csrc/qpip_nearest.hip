@@ -550,10 +550,7 @@ extern "C" int qpip_quadtree_point_to_nearest_linestring(const uint32_t* linestr
       QPIP_LAUNCH_CHECK();
     };
     uint32_t h_bad = 0;
-    auto status = [&] {
-      QPIP_HIP(hipMemcpyAsync(&h_bad, bad.get(), sizeof(uint32_t), hipMemcpyDeviceToHost, stream));
-      QPIP_HIP(hipStreamSynchronize(stream));
-    };
+    auto status = [&] { read_back({{&h_bad, bad.get(), sizeof(uint32_t)}}, stream); };
     fill();
     // chunks of the paired leaves: a tree's leaves hold each point once
     uint64_t const cap = static_cast<uint64_t>(n) / kWave +

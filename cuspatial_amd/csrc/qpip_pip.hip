@@ -1484,9 +1484,7 @@ int quadtree_point_in_polygon_entry(const uint32_t* poly_index,
         masks.release();
         chunk_info.release();
         hit_start.release();
-        QPIP_HIP(hipMemcpyAsync(h_tot, totals.get(), sizeof(uint64_t), hipMemcpyDeviceToHost,
-                                stream));
-        QPIP_HIP(hipStreamSynchronize(stream));
+        read_back({{h_tot, totals.get(), sizeof(uint64_t)}}, stream);
         QPIP_EXPECTS(h_tot[0] < (uint64_t{1} << 31), "too many candidate points");
         chunk_cap = std::max<uint64_t>(h_tot[0], 1);
         exact     = true;
@@ -1513,9 +1511,7 @@ int quadtree_point_in_polygon_entry(const uint32_t* poly_index,
       count_scan_emit<HitScanOp, uint64_t, uint64_t>(hop, n_chunks.get(), 0, partials.get(),
                                                      totals.get() + 1, stream, kScanBlocks,
                                                      "pip_scan");
-      QPIP_HIP(hipMemcpyAsync(h_tot, totals.get(), sizeof(h_tot), hipMemcpyDeviceToHost, stream));
-      QPIP_HIP(hipMemcpyAsync(h_bad, bad.get(), sizeof(h_bad), hipMemcpyDeviceToHost, stream));
-      QPIP_HIP(hipStreamSynchronize(stream));
+      read_back({{h_tot, totals.get(), sizeof(h_tot)}, {h_bad, bad.get(), sizeof(h_bad)}}, stream);
       if (h_bad[0]) throw logic_error("cuSpatial failure: quadrant index out of range of the quadtree");
       if (h_bad[1] & 1u) throw logic_error("cuSpatial failure: point or polygon index out of range");
       if (!(h_bad[1] & 2u)) break;

@@ -98,8 +98,7 @@ extern "C" int qpip_compact_nonnegative(const int32_t* values,
                                                        total.get(), stream, scan_blocks_for(un),
                                                        "compact");
     uint32_t h = 0;
-    QPIP_HIP(hipMemcpyAsync(&h, total.get(), sizeof(h), hipMemcpyDeviceToHost, stream));
-    QPIP_HIP(hipStreamSynchronize(stream));
+    read_back({{&h, total.get(), sizeof(h)}}, stream);
     *count = static_cast<int64_t>(h);
   });
 }

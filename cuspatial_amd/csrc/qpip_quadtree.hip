@@ -621,8 +621,7 @@ static int64_t quadtree_on_points_impl(double const* x,
   }
 
   TreeMeta h_meta;
-  QPIP_HIP(hipMemcpyAsync(&h_meta, meta.get(), sizeof(TreeMeta), hipMemcpyDeviceToHost, stream));
-  QPIP_HIP(hipStreamSynchronize(stream));
+  read_back({{&h_meta, meta.get(), sizeof(TreeMeta)}}, stream);
   uint64_t const m = h_meta.num_nodes;
 
   uint32_t* o_key      = oa.make<uint32_t>(m);

@@ -321,8 +321,105 @@ CompletedScope::~CompletedScope() { t_scopes.pop_back(); }
 
 void pool_set_limit(size_t bytes) { g_limit = bytes; }
 
+namespace {
+
+constexpr size_t kMailboxBytes = 8192;
+
+struct Mailboxes {
+  std::mutex mu;
+  std::vector<void*> free;
+};
+
+Mailboxes& mailboxes()
+{
+  static Mailboxes* m = new Mailboxes;  // lives as long as any thread may call
+  return *m;
+}
+
+// A pinned block for one call; back in the list when the call ends. A call that throws
+// may leave a kernel in flight that still writes the block: it is not handed out again.
+class Mailbox {
+ public:
+  Mailbox()
+  {
+    Mailboxes& m = mailboxes();
+    {
+      std::lock_guard<std::mutex> g(m.mu);
+      if (!m.free.empty()) {
+        p_ = m.free.back();
+        m.free.pop_back();
+        return;
+      }
+    }
+    QPIP_HIP(hipHostMalloc(&p_, kMailboxBytes, hipHostMallocPortable | hipHostMallocMapped));
+  }
+  void done()
+  {
+    Mailboxes& m = mailboxes();
+    std::lock_guard<std::mutex> g(m.mu);
+    m.free.push_back(p_);
+  }
+  uint32_t* get() const { return static_cast<uint32_t*>(p_); }
+
+ private:
+  void* p_ = nullptr;
+};
+
+constexpr int kReadParts = 3;
+struct ReadParts {
+  uint32_t const* src[kReadParts];
+  uint32_t words[kReadParts];
+};
+
+__global__ void __launch_bounds__(256) read_back_kernel(ReadParts r, uint32_t* __restrict__ out)
+{
+  for (int k = 0; k < kReadParts; ++k) {
+    for (uint32_t i = threadIdx.x; i < r.words[k]; i += 256) out[i] = r.src[k][i];
+    out += r.words[k];
+  }
+}
+
+}  // namespace
+
+void read_back(std::initializer_list<ReadBack> parts, hipStream_t stream)
+{
+  size_t bytes = 0;
+  for (ReadBack const& p : parts) bytes += p.bytes;
+  if (bytes > kMailboxBytes || parts.size() > static_cast<size_t>(kReadParts)) {
+    for (ReadBack const& p : parts)
+      QPIP_HIP(hipMemcpyAsync(p.dst, p.src, p.bytes, hipMemcpyDeviceToHost, stream));
+    QPIP_HIP(hipStreamSynchronize(stream));
+    return;
+  }
+  Mailbox box;
+  ReadParts r{};
+  int k = 0;
+  for (ReadBack const& p : parts) {
+    r.src[k]   = static_cast<uint32_t const*>(p.src);
+    r.words[k] = static_cast<uint32_t>(p.bytes / sizeof(uint32_t));
+    ++k;
+  }
+  uint32_t* out = nullptr;
+  QPIP_HIP(hipHostGetDevicePointer(reinterpret_cast<void**>(&out), box.get(), 0));
+  read_back_kernel<<<1, 256, 0, stream>>>(r, out);
+  QPIP_LAUNCH_CHECK();
+  QPIP_HIP(hipStreamSynchronize(stream));
+  uint32_t const* in = box.get();
+  for (ReadBack const& p : parts) {
+    std::memcpy(p.dst, in, p.bytes);
+    in += p.bytes / sizeof(uint32_t);
+  }
+  box.done();
+}
+
 void pool_trim()
 {
+  {
+    Mailboxes& m = mailboxes();
+    std::lock_guard<std::mutex> g(m.mu);
+    for (void* p : m.free) (void)hipHostFree(p);
+    m.free.clear();
+  }
   DevicePool& p = pool_for_device(current_device());
   std::lock_guard<std::mutex> g(p.mu);
   release_cached(p);
