@@ -738,13 +738,20 @@ struct GroupResult {
   uint64_t hits = 0;
 };
 
+// Mean ring vertices per polygon of the whole polygon column.
+uint64_t mean_edges(int64_t num_poly_offsets, int64_t num_vertices)
+{
+  return num_poly_offsets > 1 ? static_cast<uint64_t>(num_vertices / (num_poly_offsets - 1)) : 0;
+}
+
 // Runs one group of jobs [j0, j1). Writes point_indices for the group's points into
 // out_pi (already offset) and returns the group's hits and per-job hit counts.
 void run_group(std::vector<HostJob> const& hj, int64_t j0, int64_t j1, int64_t const* jpo,
                int64_t const* jpoly, double const* points_xy, int32_t const* poly_offsets,
                int32_t const* ring_offsets, int64_t num_ring_offsets, double const* poly_x,
-               double const* poly_y, int64_t num_vertices, uint32_t* out_pi, GroupResult& res,
-               std::vector<uint64_t>& job_hits, hipStream_t stream)
+               double const* poly_y, int64_t num_vertices, uint64_t edges_per_poly,
+               uint32_t* out_pi, GroupResult& res, std::vector<uint64_t>& job_hits,
+               hipStream_t stream)
 {
   uint32_t const J   = static_cast<uint32_t>(j1 - j0);
   int64_t const P0   = jpo[j0], P1 = jpo[j1];
@@ -932,7 +939,7 @@ void run_group(std::vector<HostJob> const& hj, int64_t j0, int64_t j1, int64_t c
     points_xy + 2 * P0, static_cast<int64_t>(n), static_cast<int64_t>(n),
     reinterpret_cast<uint32_t const*>(poly_offsets + PO0), static_cast<int64_t>(npg) + 1,
     reinterpret_cast<uint32_t const*>(ring_offsets), num_ring_offsets, poly_x, poly_y,
-    num_vertices, num_vertices, nullptr, stream, &hp, &ht, &H, f_base.get());
+    num_vertices, num_vertices, nullptr, stream, &hp, &ht, &H, f_base.get(), edges_per_poly);
   if (rc != QPIP_SUCCESS) throw logic_error(qpip_last_error_message());
   struct Hits {
     uint32_t* p[2];
@@ -1111,7 +1118,7 @@ struct PlanGroup {
   // point-in-polygon (capacity-sized)
   dbuf<uint32_t> chunk_start, hit_poly, hit_pos;
   dbuf<uint64_t> pip_partials, pip_totals, masks, hit_start;
-  // the polygon-major PIP test's pair order (used when pip_polygon_group > 0)
+  // the polygon-major PIP test's pair order (used where the test takes it)
   dbuf<uint32_t> pm_count, pm_start, pm_cursor;
   dbuf<uint4> pm_order, pm_units;
   dbuf<uint64_t> pm_partials, pm_total, pm_num_units;
@@ -1131,6 +1138,7 @@ struct BatchPlan {
   int32_t const* poly_offsets = nullptr;
   int32_t const* ring_offsets = nullptr;
   int64_t num_ring_offsets = 0, num_vertices = 0;
+  uint32_t edges_per_poly = 0;
   double const *poly_x = nullptr, *poly_y = nullptr;
   dbuf<uint32_t> ring_edges;
   dbuf<LineEdge> lines;    // per edge: the PIP test's line form
@@ -1320,6 +1328,7 @@ void plan_enqueue(BatchPlan& P, PlanGroup& g, size_t gi, hipStream_t s)
   d.poly_x         = P.poly_x;
   d.poly_y         = P.poly_y;
   d.num_vertices   = static_cast<uint64_t>(P.num_vertices);
+  d.edges_per_poly = P.edges_per_poly;
   d.poly_box       = P.poly_box.get() + g.PO0;
   d.pairs_per_wave = g.pairs_per_wave;
   d.chunk_start    = g.chunk_start.get();
@@ -1518,6 +1527,7 @@ extern "C" int qpip_batched_quadtree_point_in_polygon(int64_t num_jobs,
       groups.emplace_back();
       run_group(hj, j0, j1, job_point_offsets, job_polygon_offsets, points_xy, poly_offsets,
                 ring_offsets, num_ring_offsets, poly_x, poly_y, num_poly_x,
+                mean_edges(num_poly_offsets, num_poly_x),
                 o_pi ? o_pi + job_point_offsets[j0] : nullptr, groups.back(), job_hits, stream);
     }
     uint64_t H = 0;
@@ -1614,6 +1624,8 @@ extern "C" int qpip_batch_plan_create(int64_t num_jobs,
     P->ring_offsets     = ring_offsets;
     P->num_ring_offsets = num_ring_offsets;
     P->num_vertices     = num_poly_x;
+    P->edges_per_poly   = static_cast<uint32_t>(
+      std::min<uint64_t>(mean_edges(num_poly_offsets, num_poly_x), 0xFFFFFFFFu));
     P->poly_x           = poly_x;
     P->poly_y           = poly_y;
     int64_t const rings = num_ring_offsets > 0 ? num_ring_offsets - 1 : 0;

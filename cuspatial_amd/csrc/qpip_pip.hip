@@ -118,6 +118,7 @@ struct PipArgs {
   double const* poly_y  = nullptr;
   uint64_t num_vertices = 0;
   uint32_t pm_group        = 0;
+  uint32_t edges_per_poly  = 0;  // mean ring vertices per polygon (the order's rule)
 };
 
 // Segments of at most max(m, pairs >> s) pairs (m = 2, s = 24 by default; both
@@ -131,6 +132,20 @@ inline uint32_t pairs_per_wave(uint64_t num_pairs)
   uint64_t const g = num_pairs >> tuning(Tuning::PipPairsShift);
   uint64_t const v = g < m ? m : g;
   return static_cast<uint32_t>(v > (1u << 30) ? (1u << 30) : v);
+}
+
+// Pairs per unit of the polygon-major test, 0 for the leaf-major one. A set
+// pip_polygon_group decides; otherwise polygon order is taken where a pair's cost is
+// its ring's edges rather than its leaf's points: long rings, polygons that meet few
+// leaves (so their boxes keep few of a leaf's points) and enough pairs to fill the
+// GPU. Measured, leaf against polygon order (us, order included): 256 jobs of 130-edge
+// stars with 2.3 pairs each 457 / 342, 500 such jobs 683 / 325, 30 jobs (9,000 pairs)
+// 71 / 74; 36-edge polygons with 7 pairs each 1012 / 1618, 20-edge stars 35 / 71.
+inline uint32_t polygon_group(uint64_t pairs, uint64_t polys, uint64_t edges_per_poly)
+{
+  int64_t const set = tuning(Tuning::PipPolygonGroup);
+  if (set > 0) return static_cast<uint32_t>(set);
+  return pairs >= (1u << 14) && edges_per_poly >= 64 && pairs <= 8 * polys ? 64 : 0;
 }
 
 // --- 3. test ------------------------------------------------------------------------
@@ -1048,7 +1063,7 @@ __global__ void __launch_bounds__(256)
 
 // Launches the test over pairs [0, pairs) in slices, with the tuned workgroup
 // size (2, 4 or 8 waves) and staging depth (64 or 128 edges): the leaf-major
-// kernel, or with pip_polygon_group > 0 (and `pm` given) the polygon-major one.
+// kernel, or where polygon_group() says so (and `pm` given) the polygon-major one.
 template <int W, int S>
 void launch_pip_test_ws(PipArgs const& a, uint64_t pairs, uint64_t* masks, uint2* chunk_info,
                         uint32_t* bad, bool pm, hipStream_t stream)
@@ -1080,7 +1095,7 @@ void launch_pip_test(PipArgs const& args, uint64_t pairs, uint64_t* masks, uint2
 {
   PipArgs a = args;
   if (tuning(Tuning::PipBoxFilter) == 0) a.poly_box = nullptr;
-  int64_t const group = tuning(Tuning::PipPolygonGroup);
+  uint32_t const group = polygon_group(pairs, a.num_polys, a.edges_per_poly);
   bool const pm = group > 0 && pmb != nullptr && a.num_polys > 0 &&
                   a.chunk_cap < (uint64_t{1} << 32);  // slots in 32 bits (PmPair)
   if (pm) {
@@ -1094,7 +1109,7 @@ void launch_pip_test(PipArgs const& args, uint64_t pairs, uint64_t* masks, uint2
     count_scan_emit<PmScanOp, uint64_t, uint64_t>(op, nullptr, a.num_polys, pmb->partials,
                                                   pmb->total, stream,
                                                   scan_blocks_for(a.num_polys), "pip_order_scan");
-    PmUnitOp uop{pmb->count, pmb->start, pmb->units, static_cast<uint32_t>(group)};
+    PmUnitOp uop{pmb->count, pmb->start, pmb->units, group};
     count_scan_emit<PmUnitOp, uint64_t, uint64_t>(uop, nullptr, a.num_polys, pmb->partials,
                                                   pmb->num_units, stream,
                                                   scan_blocks_for(a.num_polys), "pip_order_scan");
@@ -1105,7 +1120,7 @@ void launch_pip_test(PipArgs const& args, uint64_t pairs, uint64_t* masks, uint2
     a.pm_count     = pmb->count;
     a.pm_units     = pmb->units;
     a.pm_num_units = pmb->num_units;
-    a.pm_group     = static_cast<uint32_t>(group);
+    a.pm_group     = group;
   }
   KernelTimer kt("pip_test", stream);
   int64_t const w = tuning(Tuning::PipWavesPerBlock);
@@ -1344,6 +1359,7 @@ void launch_pip_device(PipDevice const& d, hipStream_t stream)
   args.poly_x       = d.poly_x;
   args.poly_y       = d.poly_y;
   args.num_vertices = d.num_vertices;
+  args.edges_per_poly = d.edges_per_poly;
   QPIP_EXPECTS(args.num_vertices == 0 || (args.poly_x && args.poly_y),
                "polygon vertices must not be null");
   PmBuffers const pmb{d.pm_count,    d.pm_start, d.pm_cursor, d.pm_order,
@@ -1397,7 +1413,8 @@ int quadtree_point_in_polygon_entry(const uint32_t* poly_index,
                                               uint32_t** polygon_index,
                                               uint32_t** point_index,
                                               int64_t* num_hits,
-                                              const uint32_t* point_base)
+                                              const uint32_t* point_base,
+                                              uint64_t edges_per_poly)
 {
   (void)key;
   (void)level;
@@ -1464,8 +1481,11 @@ int quadtree_point_in_polygon_entry(const uint32_t* poly_index,
     bool exact           = false;
     dbuf<uint64_t> masks, hit_start;
     dbuf<uint2> chunk_info;
-    // the polygon-major test's order (pip_polygon_group > 0)
-    bool const pm_on = tuning(Tuning::PipPolygonGroup) > 0 && num_polys > 0;
+    // the polygon-major test's order
+    uint64_t const edges = edges_per_poly > 0 ? edges_per_poly
+                           : num_polys > 0    ? static_cast<uint64_t>(num_poly_x) / num_polys
+                                              : 0;
+    bool const pm_on     = polygon_group(K, num_polys, edges) > 0 && num_polys > 0;
     dbuf<uint32_t> pm_count(pm_on ? num_polys : 1), pm_start(pm_on ? num_polys : 1),
       pm_cursor(pm_on ? num_polys : 1);
     dbuf<uint4> pm_order(pm_on ? K : 1), pm_units(pm_on ? K : 1);
@@ -1500,6 +1520,7 @@ int quadtree_point_in_polygon_entry(const uint32_t* poly_index,
       args.poly_x       = poly_x;
       args.poly_y       = poly_y;
       args.num_vertices = static_cast<uint64_t>(num_poly_x);
+      args.edges_per_poly = static_cast<uint32_t>(std::min<uint64_t>(edges, 0xFFFFFFFFu));
       launch_pip_test(args, K, masks.get(), chunk_info.get(), bad.get() + 1,
                       pm_on ? &pmb : nullptr, stream);
       // chunks past the capacity were not tested: the scan covers those that were
@@ -1584,7 +1605,7 @@ extern "C" int qpip_quadtree_point_in_polygon(const uint32_t* poly_index,
     poly_index, quad_index, num_pairs, key, level, is_internal_node, length, offset, num_nodes,
     point_indices, num_point_indices, x, y, nullptr, num_x, num_y, poly_offsets,
     num_poly_offsets, ring_offsets, num_ring_offsets, poly_x, poly_y, num_poly_x, num_poly_y, mr,
-    stream, polygon_index, point_index, num_hits, nullptr);
+    stream, polygon_index, point_index, num_hits, nullptr, 0);
 }
 
 extern "C" int qpip_quadtree_point_in_polygon_xy(const uint32_t* poly_index,
@@ -1618,7 +1639,7 @@ extern "C" int qpip_quadtree_point_in_polygon_xy(const uint32_t* poly_index,
     poly_index, quad_index, num_pairs, key, level, is_internal_node, length, offset, num_nodes,
     point_indices, num_point_indices, nullptr, nullptr, points_xy, num_points, num_points,
     poly_offsets, num_poly_offsets, ring_offsets, num_ring_offsets, poly_x, poly_y, num_poly_x,
-    num_poly_y, mr, stream, polygon_index, point_index, num_hits, nullptr);
+    num_poly_y, mr, stream, polygon_index, point_index, num_hits, nullptr, 0);
 }
 
 namespace {

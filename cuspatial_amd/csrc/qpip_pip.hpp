@@ -44,6 +44,7 @@ struct PipDevice {
   double const* poly_x  = nullptr;  // the vertices (the exact retest walks them)
   double const* poly_y  = nullptr;
   uint64_t num_vertices = 0;
+  uint32_t edges_per_poly = 0;  // mean ring vertices per polygon
   PolyBox const* poly_box;  // per polygon (null: the test filters no points)
   uint32_t pairs_per_wave;
   // workspace
@@ -88,7 +89,8 @@ void launch_pip_device(PipDevice const& d, hipStream_t stream);
 // The quadtree PIP join over host-visible sizes (qpip_quadtree_point_in_polygon and
 // its _xy form; x/y or xy). With point_base non-null, point_indices are local to
 // each node's job and point_base[node] is that job's first point (the batched
-// eager call); the C entry points pass null.
+// eager call); the C entry points pass null. edges_per_poly: the mean ring vertices per
+// polygon where the vertices given are those of more polygons than these (0: count).
 int quadtree_point_in_polygon_entry(const uint32_t* poly_index, const uint32_t* quad_index,
                                     int64_t num_pairs, const uint32_t* key, const uint8_t* level,
                                     const uint8_t* is_internal_node, const uint32_t* length,
@@ -101,7 +103,8 @@ int quadtree_point_in_polygon_entry(const uint32_t* poly_index, const uint32_t* 
                                     const double* poly_y, int64_t num_poly_x, int64_t num_poly_y,
                                     const qpip_resource* mr, void* stream,
                                     uint32_t** polygon_index, uint32_t** point_index,
-                                    int64_t* num_hits, const uint32_t* point_base);
+                                    int64_t* num_hits, const uint32_t* point_base,
+                                    uint64_t edges_per_poly);
 
 // The test kernel's pairs-per-wave segment length for a join of num_pairs pairs
 // (the runtime tuning parameters pip_min_pairs_per_wave, pip_pairs_shift).

@@ -96,8 +96,10 @@ QPIP_API void qpip_memory_info(size_t* live_bytes, size_t* cached_bytes);
  *   pip_box_filter          1: that test skips points outside a polygon's vertex
  *                           box and packs the rest into fewer lanes; 0: it tests
  *                           every candidate point (default 1)
- *   pip_polygon_group       0: the test walks the pairs leaf by leaf (default);
- *                           n > 0: it groups them by polygon, one wave taking up
+ *   pip_polygon_group       0: the test's order is chosen by the join's shape
+ *                           (default): leaf by leaf, or by polygon where rings are
+ *                           long and meet few leaves;
+ *                           n > 0: it groups the pairs by polygon, one wave taking up
  *                           to n pairs of one polygon and packing their kept
  *                           points from several leaves into full waves
  * Results do not depend on them, only the time. Errors: unknown name, value out

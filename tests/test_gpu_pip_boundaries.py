@@ -15,6 +15,7 @@ equal the brute-force bitmask's (GPU and oracle).
 import numpy as np
 import pytest
 
+from conftest import star_polygons
 from test_gpu_parity import assert_same, run_gpu, run_oracle
 
 pytestmark = pytest.mark.gpu
@@ -306,3 +307,32 @@ def test_long_rings_few_points_match_oracle(cs, oracle_mod, stage, group, box):
         o = run_oracle(oracle_mod, x, y, bbox, 48.0 / (1 << d), d, max_size, polys)
         assert_same(g, o)
         assert len(o["polygon_index"]) > 0
+
+
+@pytest.mark.parametrize("kmin,n,fewer", [(63, 9000, 0), (70, 9000, 0), (70, 2500, 0),
+                                          (70, 9000, 1)])
+def test_order_chosen_by_shape_matches_oracle(cs, oracle_mod, kmin, n, fewer):
+    """The rule that takes the polygon-major order by itself (mean ring length from 64,
+    2^14 pairs, at most eight pairs per polygon), on both sides of each line: rings a
+    little shorter and longer, fewer pairs, larger polygons with more pairs each. Hits
+    exact against the oracle, in its order."""
+    rng = np.random.default_rng(kmin + n + fewer)
+    ext = 1000.0
+    size = (750, 30.0, 60.0) if fewer else (n, 4.0, 9.0)
+    part, ring, vx, vy = star_polygons(rng, size[0], ext, *size[1:], kmin=kmin, kmax=kmin + 2)
+    x, y = rng.uniform(0, ext, 60000), rng.uniform(0, ext, 60000)
+    k = 500
+    x[:k], y[:k] = vx[:k], vy[:k]
+    d, ms, scale = 6, 64, ext / 64
+    pts, P = cs.Points(x, y, device="cuda"), cs.Polygons(part, ring, vx, vy, device="cuda")
+    pi, tree = cs.quadtree_on_points(pts, 0.0, ext, 0.0, ext, scale, d, ms)
+    bb = cs.polygon_bounding_boxes(P)
+    pairs = cs.join_quadtree_and_bounding_boxes(tree, bb, 0.0, ext, 0.0, ext, scale, d)
+    hits = cs.quadtree_point_in_polygon(pairs, tree, pi, pts, P)
+    t = tuple(v.cpu().numpy() for v in tree.values())
+    pp, pt = oracle_mod.quadtree_point_in_polygon(
+        tuple(v.cpu().numpy() for v in pairs.values()), t, pi.cpu().numpy(), x, y, part, ring, vx,
+        vy)
+    assert len(pp) > 1000
+    assert np.array_equal(hits["polygon_index"].cpu().numpy().astype(np.int64), pp.astype(np.int64))
+    assert np.array_equal(hits["point_index"].cpu().numpy().astype(np.int64), pt.astype(np.int64))
