@@ -89,9 +89,7 @@ struct GridView {
 __device__ __forceinline__ uint32_t grid_coord(double v, double v0, double inv_cell, uint32_t dim)
 {
   double const t = floor((v - v0) * inv_cell);
-  if (!(t >= 0.0)) return 0u;
-  if (t >= static_cast<double>(dim - 1)) return dim - 1;
-  return static_cast<uint32_t>(t);
+  return static_cast<uint32_t>(fmin(fmax(t, 0.0), static_cast<double>(dim - 1)));  // NaN: 0
 }
 
 struct Loc {
@@ -175,6 +173,14 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint16_t u16x8 __attribute__((ext_vector_type(8)));
 
 constexpr int kKT = 32;  // K per v_mfma_f32_16x16x32_bf16
+
+// A wave's LDS writes before, its reads after (and the other way round).
+__device__ __forceinline__ void wave_lds_sync()
+{
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
 
 // D = A B + C on one 16x16x32 bf16 tile (gfx950). Lane l supplies
 // A[l % 16][8 (l / 16) + j] and B[8 (l / 16) + j][l % 16] (j = 0..7) and holds
@@ -633,9 +639,7 @@ __global__ void __launch_bounds__(kMlpWaves * kWave, 1) mlp_kernel(MlpArgs a)
 #pragma unroll
         for (int mt = 0; mt < kEmb / 16; ++mt)
           *reinterpret_cast<f32x4*>(row0 + (16 * t + r) * kDxPitch + 16 * mt + 4 * g) = dx[t][mt];
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      wave_lds_sync();
 #pragma unroll
       for (int t = 0; t < kMlpCols; ++t)
 #pragma unroll 4
@@ -735,6 +739,7 @@ struct PolyView {
   EdgeB const* edges_b;
   uint32_t const* ring_edges;
   struct Record const* records;
+  struct RingSlot const* slots;
 };
 
 // Per polygon with exactly one ring: its effective edges [e0, e0 + ne) and the y
@@ -746,24 +751,76 @@ struct alignas(16) Record {
   double y0;
 };
 
-__global__ void __launch_bounds__(256) records_kernel(PolyView P, Record* __restrict__ out)
+// A polygon of one short ring in single precision, in one 128-byte line: vertices
+// relative to (cx, cy), the first the edges' first `b`, then each edge's `a`, and
+// the largest magnitude among them. 20,000 cells of 6 edges: 2.6 MB, which one L2
+// holds, against 4.5 MB of edges and 0.3 MB of records for the exact test.
+// ne == kMultiRing: no slot (several rings, more than kSlotEdges edges, coordinates
+// that are not finite, an extent outside [2^-60, 2^60]).
+constexpr uint32_t kSlotEdges = 13;
+struct alignas(128) RingSlot {
+  float cx, cy, m;
+  uint32_t ne;
+  float2 v[kSlotEdges + 1];
+};
+
+__device__ __forceinline__ void fill_slot(PolyView const& P, Record const& rec, RingSlot& out)
+{
+  RingSlot s;
+  s.cx = s.cy = s.m = 0.f;
+  s.ne = kMultiRing;
+#pragma unroll
+  for (uint32_t i = 0; i <= kSlotEdges; ++i) s.v[i] = float2{0.f, 0.f};
+  if (rec.ne <= kSlotEdges) {
+    Edge const* E = P.edges + rec.e0;
+    double2 w[kSlotEdges + 1];
+    double mnx = __builtin_inf(), mxx = -mnx, mny = mnx, mxy = -mnx;
+    uint32_t const nv = rec.ne ? rec.ne + 1 : 0u;
+#pragma unroll
+    for (uint32_t i = 0; i <= kSlotEdges; ++i)
+      if (i < nv) {
+        w[i] = i ? double2{E[i - 1].ax, E[i - 1].ay}
+                 : double2{P.edges_b[rec.e0].bx, P.edges_b[rec.e0].by};
+        mnx = fmin(mnx, w[i].x), mxx = fmax(mxx, w[i].x);
+        mny = fmin(mny, w[i].y), mxy = fmax(mxy, w[i].y);
+      }
+    s.cx   = static_cast<float>(0.5 * mnx + 0.5 * mxx);
+    s.cy   = static_cast<float>(0.5 * mny + 0.5 * mxy);
+    bool ok = true;
+#pragma unroll
+    for (uint32_t i = 0; i <= kSlotEdges; ++i)
+      if (i < nv) {
+        s.v[i] = float2{static_cast<float>(w[i].x - static_cast<double>(s.cx)),
+                        static_cast<float>(w[i].y - static_cast<double>(s.cy))};
+        float const m = fmaxf(fabsf(s.v[i].x), fabsf(s.v[i].y));
+        ok            = ok && fabsf(s.v[i].x) <= 0x1p60f && fabsf(s.v[i].y) <= 0x1p60f;
+        s.m           = fmaxf(s.m, m);
+      }
+    s.m *= 1.f + 0x1p-20f;  // above every vertex's own magnitude, not its rounded one
+    if (rec.ne == 0 || (ok && s.m >= 0x1p-60f)) s.ne = rec.ne;
+  }
+  out = s;
+}
+
+__global__ void __launch_bounds__(64)
+  records_kernel(PolyView P, Record* __restrict__ out, RingSlot* __restrict__ slots)
 {
   for (int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < P.num_polys;
-       i += static_cast<int64_t>(gridDim.x) * blockDim.x)
-    [&] {
-      uint32_t const r0 = P.poly_offsets[i];
-      uint32_t r1       = P.poly_offsets[i + 1];
-      if (r1 > P.num_rings) r1 = static_cast<uint32_t>(P.num_rings);
-      Record rec{0u, kMultiRing, 0.0};
-      if (r1 == r0 + 1) {
-        rec.e0 = P.ring_offsets[r0];
-        rec.ne = P.ring_edges[r0];
-        rec.y0 = rec.ne ? P.edges_b[rec.e0].by : 0.0;
-      } else if (r1 <= r0) {
-        rec.ne = 0;  // no rings: never contains a point
-      }
-      out[i] = rec;
-    }();
+       i += static_cast<int64_t>(gridDim.x) * blockDim.x) {
+    uint32_t const r0 = P.poly_offsets[i];
+    uint32_t r1       = P.poly_offsets[i + 1];
+    if (r1 > P.num_rings) r1 = static_cast<uint32_t>(P.num_rings);
+    Record rec{0u, kMultiRing, 0.0};
+    if (r1 == r0 + 1) {
+      rec.e0 = P.ring_offsets[r0];
+      rec.ne = P.ring_edges[r0];
+      rec.y0 = rec.ne ? P.edges_b[rec.e0].by : 0.0;
+    } else if (r1 <= r0) {
+      rec.ne = 0;  // no rings: never contains a point
+    }
+    out[i] = rec;
+    fill_slot(P, rec, slots[i]);
+  }
 }
 
 struct LocateArgs {
@@ -844,12 +901,67 @@ __device__ __forceinline__ void exact_test(PolyView const& P, uint32_t poly, dou
   near_out   = near;
 }
 
+// The test on a polygon's single-precision slot: false where it cannot vouch for the
+// exact test's outcome. With s the point's and the vertices' largest magnitude about
+// the slot's centre, a vertex relative to the point is known to within 2^-23 s (its
+// rounding, the point's and the subtraction's, 2^-24 of at most s, s and 2 s, the
+// first two never both at their largest), so an edge's lhs - rhs, two products of such,
+// to within 2^-20 s^2 with their own rounding. Where every vertex's y is off the
+// point's by more than 2^-21 s and every edge's |lhs - rhs| is above 2^-19 s^2, all signs
+// are the exact test's, whose own error is 2^-48 of the same products, and no edge is
+// within its collinearity filter (near). NaN and infinite points never pass.
+__device__ __forceinline__ bool slot_test(RingSlot const& S, double px, double py, bool& inside)
+{
+  float4 const* q = reinterpret_cast<float4 const*>(&S);
+  // the header and eight vertices (up to seven edges) in one round trip
+  float4 const h = q[0];
+  float4 a[4]    = {q[1], q[2], q[3], q[4]};
+  uint32_t const ne = __float_as_uint(h.w);
+  inside            = false;
+  if (ne > kSlotEdges) return false;
+  if (ne == 0) return true;
+  float const dx = static_cast<float>(px - static_cast<double>(h.x));
+  float const dy = static_cast<float>(py - static_cast<double>(h.y));
+  float const s  = fabsf(dx) + fabsf(dy) + h.z;  // NaN if either is
+  float bx = a[0].x - dx, by = a[0].y - dy;
+  float my = fabsf(by), mt = INFINITY;
+  uint32_t flip = 0;
+  auto edge = [&](float vx, float vy) {
+    float const ux = vx - dx, uy = vy - dy;
+    float const t  = __builtin_fmaf(bx, uy, -(ux * by));
+    my             = fminf(my, fabsf(uy));
+    mt             = fminf(mt, fabsf(t));
+    // toggles where the y signs differ and t's sign is the edge's end's
+    flip ^= (__float_as_uint(uy) ^ __float_as_uint(by)) &
+            ~(__float_as_uint(t) ^ __float_as_uint(uy));
+    bx = ux, by = uy;
+  };
+  edge(a[0].z, a[0].w);
+#pragma unroll
+  for (uint32_t k = 1; k < 4; ++k) {
+    if (2 * k <= ne) edge(a[k].x, a[k].y);
+    if (2 * k + 1 <= ne) edge(a[k].z, a[k].w);
+  }
+  for (uint32_t k = 4; 2 * k <= ne; ++k) {
+    float4 const w = q[1 + k];
+    edge(w.x, w.y);
+    if (2 * k + 1 <= ne) edge(w.z, w.w);
+  }
+  inside = (flip >> 31) != 0u;
+  return my > 0x1p-21f * s && mt > 0x1p-19f * (s * s);
+}
+
 __device__ __forceinline__ bf16x8 load_frag(uint16_t const* lds, int frag, int lane)
 {
   return *reinterpret_cast<bf16x8 const*>(lds +
                                           (static_cast<int64_t>(frag) * kWave + lane) * kFragElems);
 }
 
+// The next round's coordinates are loaded before layer 2 and its cells' embeddings and
+// candidate counts before layer 3, into the registers that the layers in between have
+// freed: the chain point -> cell -> embedding, two misses long, then runs under the MFMAs
+// (20,000,000 points: 1337 -> 1105 us; the MFMAs alone are 490 us of it, the bf16
+// conversions, features and the choice of the slots about as many VALU cycles).
 // Two waves per SIMD (at most 256 registers, which also keeps the accumulators in
 // VGPRs: no AGPR copies before the bf16 conversions), as many as two workgroups'
 // LDS allows: one wave's feature and conversion work overlaps the other's MFMAs.
@@ -893,30 +1005,52 @@ __global__ void __launch_bounds__(kLocWaves * kWave, 2) rank_kernel(LocateArgs a
   uint16_t const* W2s = w_lds + kW1Frags * kWave * kFragElems;
   uint16_t const* W3s = w_lds + (kW1Frags + kW2Frags) * kWave * kFragElems;
 
-  for (int64_t base = (static_cast<int64_t>(blockIdx.x) * kLocWaves + wave) * kWave; base < a.n;
-       base += waves * kWave) {
-    uint32_t cell[kLocTiles];
-    bf16x8 X[kLocTiles][kIn / kKT];
+  int64_t base = (static_cast<int64_t>(blockIdx.x) * kLocWaves + wave) * kWave;
+  if (base >= a.n) return;
+  // the round's points, lane r of each group holding row r of every tile
+  auto load_points = [&](int64_t from, double2 (&p)[kLocTiles]) {
 #pragma unroll
     for (int t = 0; t < kLocTiles; ++t) {
-      int64_t const p = base + 16 * t + r;
-      bool const in   = p < a.n;
-      Loc const L     = locate_cell(a.g, in ? a.xy[2 * p] : 0.0, in ? a.xy[2 * p + 1] : 0.0);
-      cell[t]         = L.cell;
+      int64_t i = from + 16 * t + r;
+      if (i >= a.n) i = a.n - 1;  // a row past the end: any point, its order is not written
+      p[t] = double2{a.xy[2 * i], a.xy[2 * i + 1]};
+    }
+  };
+  bf16x8 X[kLocTiles][kIn / kKT];
+  float u[kLocTiles], v[kLocTiles];
+  int count;  // candidates at this lane's own point (tile g, row r)
+  // their cells; the embeddings and the count are on their way afterwards
+  auto load_cells = [&](double2 const (&p)[kLocTiles]) {
+    uint32_t own = 0;
+#pragma unroll
+    for (int t = 0; t < kLocTiles; ++t) {
+      Loc const L = locate_cell(a.g, p[t].x, p[t].y);
+      u[t] = L.u, v[t] = L.v;
+      if (g == t) own = L.cell;
       uint16_t const* e = a.pb + a.lay.e + static_cast<int64_t>(L.cell) * kEmb;
 #pragma unroll
       for (int c = 0; c < kEmb / kKT; ++c)
         X[t][c] = *reinterpret_cast<bf16x8 const*>(e + kKT * c + 8 * g);
+    }
+    count = a.g.count[own];
+  };
+  double2 pts[kLocTiles];
+  load_points(base, pts);
+  load_cells(pts);
+  for (; base < a.n; base += waves * kWave) {
+#pragma unroll
+    for (int t = 0; t < kLocTiles; ++t) {
       // features 64 + 8g + j: frequencies 2g (j < 4) and 2g + 1 (j >= 4)
       float f0[4], f1[4];
-      fourier4(L.u, L.v, 2 * g, f0);
-      fourier4(L.u, L.v, 2 * g + 1, f1);
+      fourier4(u[t], v[t], 2 * g, f0);
+      fourier4(u[t], v[t], 2 * g + 1, f1);
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         X[t][kEmb / kKT][j]     = bf(f0[j]);
         X[t][kEmb / kKT][j + 4] = bf(f1[j]);
       }
     }
+    int const cnt = count;
     // layer 1: output tile mt holds rows 16 mt + 4g + j; tiles 2c and 2c + 1 form
     // layer 2's K tile c (chained_col)
     f32x4 H[kLocTiles][kHid / 16];
@@ -946,6 +1080,7 @@ __global__ void __launch_bounds__(kLocWaves * kWave, 2) rank_kernel(LocateArgs a
                     relu2(h[2 * c + 1][2], h[2 * c + 1][3])};
       return __builtin_bit_cast(bf16x8, w);
     };
+    load_points(base + waves * kWave, pts);  // the next round's (X is free from here)
     // layer 2
     f32x4 H2[kLocTiles][kHid / 16];
     {
@@ -968,6 +1103,7 @@ __global__ void __launch_bounds__(kLocWaves * kWave, 2) rank_kernel(LocateArgs a
         }
       }
     }
+    load_cells(pts);
     // layer 3: logits, then transpose through LDS (lane l -> point base + l)
     {
       f32x4 acc[kLocTiles];
@@ -986,24 +1122,15 @@ __global__ void __launch_bounds__(kLocWaves * kWave, 2) rank_kernel(LocateArgs a
 #pragma unroll
         for (int j = 0; j < 4; ++j) lg[(16 * t + r) * kLogitPitch + 4 * g + j] = acc[t][j];
     }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    wave_lds_sync();
     float z[kCand];
 #pragma unroll
     for (int s = 0; s < kCand; ++s) z[s] = lg[l * kLogitPitch + s];
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    wave_lds_sync();
 
     // this lane's point is tile g, row r: base + 16 g + r = base + l
     int64_t const p = base + l;
     if (p >= a.n) continue;
-    uint32_t c = cell[0];
-#pragma unroll
-    for (int t = 1; t < kLocTiles; ++t)
-      if (g == t) c = cell[t];
-    int const cnt   = a.g.count[c];
     int const limit = cnt > kCand ? 0 : (cnt < a.max_tests ? cnt : a.max_tests);
     // The three best slots by decreasing logit (NaN lowest, near-ties to the lower
     // slot): each slot's key is the logit's order-preserving bits with the low 4
@@ -1031,57 +1158,116 @@ __global__ void __launch_bounds__(kLocWaves * kWave, 2) rank_kernel(LocateArgs a
   }
 }
 
-// Exact tests in predicted order, one lane per point.
-__global__ void __launch_bounds__(256) verify_kernel(LocateArgs a)
+// Exact tests in predicted order, one lane per point. A wave takes `chunks` chunks of
+// 64 points: each point's first candidate at once, the points it does not settle
+// through a queue in LDS, so that second and later tests run in full waves too (the
+// slowest of 64 points needs three or four). Bound by the scattered reads: a cell's
+// count and candidate, and a polygon's line per test. 20,000,000 points, 20,000 cells
+// of about 6 edges, 65,536 grid cells: 1658 us with a lane running its point's tests
+// one after the other over 32-byte edges, 840 us so; 8 and 16 chunks: 850 and 890.
+constexpr int kVerWaves     = 4;
+constexpr uint32_t kVerMost = 4;  // chunks of a wave at most
+
+struct Pending {  // a point in the queue
+  uint32_t at;    // index in the wave's points | tests << 16 | count << 24
+  uint32_t cell;
+  uint32_t slots;  // order's three slots | the unranked slots as a mask << 16
+};
+
+__global__ void __launch_bounds__(kVerWaves * kWave, 7)
+  verify_kernel(LocateArgs a, uint32_t chunks)
 {
-  int64_t const p = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (p >= a.n) return;
-  double const x  = a.xy[2 * p];
-  double const y  = a.xy[2 * p + 1];
-  uint32_t const order = a.order[p];  // issued with the point, before the cell lookup
-  uint32_t const c = locate_cell(a.g, x, y).cell;
-  int const cnt    = a.g.count[c];
-  int32_t result   = -1;
-  uint8_t flags    = 0;
-  int tests        = 0;
-  if (cnt > kCand) {
-    flags = 1;  // overflowed cell: quadtree path
-  } else {
-    uint32_t const ranked = order >> 12;
-    int const limit       = cnt < a.max_tests ? cnt : a.max_tests;
-    // one candidate: true when the search is over (a hit, or an error)
-    auto test = [&](int s) {
-      ++tests;
-      int32_t const poly = a.g.cand[static_cast<int64_t>(c) * kCand + s];
-      if (poly < 0 || poly >= a.P.num_polys) {
-        flags |= 1;
-        return true;
+  __shared__ Pending s_queue[kVerWaves][2 * kWave];
+  int const lane      = lane_id();
+  Pending* const q    = s_queue[threadIdx.x / kWave];
+  int64_t const first = (static_cast<int64_t>(blockIdx.x) * kVerWaves + threadIdx.x / kWave) *
+                        static_cast<int64_t>(chunks) * kWave;
+  uint32_t queued = 0;  // uniform
+
+  // the point's outcome
+  auto write = [&](int64_t p, int32_t result, uint32_t tests, uint32_t flags) {
+    if (!(result >= 0 && tests == 1)) flags |= 2u;  // first prediction was not the answer
+    a.out_poly[p]  = (flags & 1u) ? -2 : result;
+    a.out_tests[p] = static_cast<uint8_t>(tests);
+    a.out_flags[p] = static_cast<uint8_t>(flags);
+  };
+
+  for (uint32_t k = 0;;) {
+    // 64 queued points, or the next chunk, or the rest of the queue
+    int64_t const next = first + static_cast<int64_t>(k) * kWave;
+    bool const fresh   = queued < static_cast<uint32_t>(kWave) && k < chunks && next < a.n;
+    if (!fresh && queued == 0) break;
+    bool active;
+    int64_t p = 0;
+    double x = 0.0, y = 0.0;
+    Pending e{};
+    if (fresh) {
+      p      = next + lane;
+      active = p < a.n;
+      if (active) {
+        x = a.xy[2 * p], y = a.xy[2 * p + 1];
+        uint32_t const order = a.order[p];  // issued with the point, before the cell lookup
+        e.cell               = locate_cell(a.g, x, y).cell;
+        uint32_t const cnt   = a.g.count[e.cell];
+        if (cnt - 1u >= static_cast<uint32_t>(kCand)) {  // none, or overflowed: quadtree path
+          write(p, -1, 0, cnt ? 1u : 0u);
+          active = false;
+        } else {
+          uint32_t rest = (1u << cnt) - 1u;
+          for (uint32_t i = 0; i < order >> 12; ++i) rest &= ~(1u << ((order >> (4 * i)) & 15u));
+          e.at    = (k * kWave + static_cast<uint32_t>(lane)) | (cnt << 24);
+          e.slots = order | (rest << 16);
+        }
       }
-      bool inside, near;
-      exact_test(a.P, static_cast<uint32_t>(poly), x, y, inside, near);
-      if (!inside) return false;
-      if (near)
-        flags |= 1;
-      else
-        result = poly;
-      return true;
-    };
-    bool done = false;
-    // the ranked slots, then the others in list order
-    for (uint32_t i = 0; i < ranked && !done && tests < limit; ++i)
-      done = test(static_cast<int>((order >> (4 * i)) & 15u));
-    for (int q = 0; q < cnt && !done && tests < limit; ++q) {
-      bool ranked_q = false;
-      for (uint32_t i = 0; i < ranked; ++i)
-        ranked_q |= ((order >> (4 * i)) & 15u) == static_cast<uint32_t>(q);
-      if (!ranked_q) done = test(q);
+      ++k;
+    } else {
+      uint32_t const take = queued < static_cast<uint32_t>(kWave) ? queued : kWave;
+      queued -= take;
+      active = static_cast<uint32_t>(lane) < take;
+      wave_lds_sync();
+      if (active) {
+        e = q[queued + static_cast<uint32_t>(lane)];
+        p = first + (e.at & 0xffffu);
+        x = a.xy[2 * p], y = a.xy[2 * p + 1];
+      }
+      wave_lds_sync();
     }
-    if (result < 0 && !(flags & 1) && tests < cnt) flags |= 1;  // stopped at max_tests
-    if (!(result >= 0 && tests == 1)) flags |= 2;  // first prediction was not the answer
+    // one candidate of each point
+    bool more = false;
+    if (active) {
+      uint32_t tests        = (e.at >> 16) & 0xffu;
+      uint32_t const cnt    = e.at >> 24;
+      uint32_t const ranked = (e.slots >> 12) & 15u;
+      uint32_t slot;
+      if (tests < ranked) {
+        slot = (e.slots >> (4 * tests)) & 15u;
+      } else {
+        uint32_t const rest = e.slots >> 16;
+        slot                = static_cast<uint32_t>(__ffs(static_cast<int>(rest))) - 1u;
+        e.slots             = (e.slots & 0xffffu) | ((rest & (rest - 1u)) << 16);
+      }
+      ++tests;
+      int32_t const poly = a.g.cand[static_cast<int64_t>(e.cell) * kCand + slot];
+      if (poly < 0 || poly >= a.P.num_polys) {
+        write(p, -1, tests, 1u);
+      } else {
+        bool inside, near = false;
+        if (!slot_test(a.P.slots[poly], x, y, inside))
+          exact_test(a.P, static_cast<uint32_t>(poly), x, y, inside, near);
+        if (inside) {
+          write(p, near ? -1 : poly, tests, near ? 1u : 0u);
+        } else if (tests < cnt && tests < static_cast<uint32_t>(a.max_tests)) {
+          more = true;
+          e.at = (e.at & 0xff00ffffu) | (tests << 16);
+        } else {
+          write(p, -1, tests, tests < cnt ? 1u : 0u);  // stopped at max_tests, or no polygon
+        }
+      }
+    }
+    uint64_t const m = ballot(more);
+    if (more) q[queued + static_cast<uint32_t>(__popcll(m & lanemask_lt()))] = e;
+    queued += static_cast<uint32_t>(__popcll(m));
   }
-  a.out_poly[p]  = (flags & 1) ? -2 : result;
-  a.out_tests[p] = static_cast<uint8_t>(tests);
-  a.out_flags[p] = flags;
 }
 
 // ---------------------------------------------------------------------------------
@@ -1306,10 +1492,12 @@ extern "C" int qpip_ranker_locate(const qpip_ranker* model,
     a.out_tests = out_tests;
     a.out_flags = out_flags;
     dbuf<Record> records(std::max<int64_t>(polys, 1));
+    dbuf<RingSlot> slots(std::max<int64_t>(polys, 1));
     a.P.records = records.get();
+    a.P.slots   = slots.get();
     if (polys > 0) {
-      records_kernel<<<grid_for(static_cast<uint64_t>(polys), 256), 256, 0, stream>>>(
-        a.P, records.get());
+      records_kernel<<<grid_for(static_cast<uint64_t>(polys), 64), 64, 0, stream>>>(
+        a.P, records.get(), slots.get());
       QPIP_LAUNCH_CHECK();
     }
     dbuf<uint16_t> order(num_points);
@@ -1327,7 +1515,13 @@ extern "C" int qpip_ranker_locate(const qpip_ranker* model,
     }
     {
       KernelTimer kt("ranker_verify", stream);
-      verify_kernel<<<grid_for(static_cast<uint64_t>(num_points), 256, 1u << 30), 256, 0, stream>>>(a);
+      // more chunks per wave only where every wave slot of the GPU (32 per CU) has one:
+      // 10,000 points are one chunk for each of 157 waves, and a second chunk would
+      // only lengthen their chain of loads
+      uint64_t const chunks =
+        std::clamp<uint64_t>(groups / (uint64_t(32) * cus), 1, kVerMost);
+      verify_kernel<<<grid_for(groups, kVerWaves * chunks, 1u << 30), kVerWaves * kWave, 0,
+                      stream>>>(a, static_cast<uint32_t>(chunks));
       QPIP_LAUNCH_CHECK();
     }
   });

@@ -539,8 +539,8 @@ class LearnedLocator:
             P.x.numel(), xy.data_ptr(), n, int(max_tests), out.data_ptr(), tests.data_ptr(),
             flags.data_ptr(), _capi.stream_handle(dev)))
         t1 = time.perf_counter()
-        fb, _ = _capi.compact_nonnegative(
-            torch.where(out == -2, 0, -1).to(torch.int32), with_values=False)
+        # -2 - out is 0 at the points left to the quadtree path (-2), negative elsewhere
+        fb, _ = _capi.compact_nonnegative(torch.rsub(out, -2), with_values=False)
         extra = (torch.zeros(0, dtype=torch.int64, device=dev),
                  torch.zeros(0, dtype=torch.int64, device=dev))
         if fb.numel():

@@ -257,6 +257,53 @@ def test_locator_partition_with_holes(env):
     assert torch.equal(poly, want_poly) and torch.equal(pt, want_pt)
 
 
+@pytest.mark.parametrize("edges, exponent, n",
+                         [(4, 0, 1), (4, 0, 2000), (12, 0, 4097), (13, 0, 5000), (14, 0, 5000),
+                          (20, 0, 2000), (9, -70, 3000), (9, 61, 3000), (6, 0, 1_300_003)])
+def test_locator_short_rings_equal_plain_join(env, edges, exponent, n):
+    """Sheared unit cells whose bottom and top sides carry extra vertices (4 to 20
+    edges: up to 13 have the single-precision form), scaled by powers of two inside
+    and outside that form's range; a third of the points lie on vertices, on sides or
+    level with vertices. Every coordinate is exact. The pairs are the plain join's
+    (bit-identical); the longest list takes several chunks per wave."""
+    torch, cs, ranker, rk, _ = env
+    k, size = 12, 2.0**exponent
+    extra = edges - 4
+    bottom = np.arange(extra // 2 + 2) / 16.0
+    bottom[-1] = 1.0
+    top = (np.arange(extra - extra // 2 + 2) / 16.0)[::-1].copy()
+    top[0] = 1.0
+    cx = np.concatenate([bottom, top, [0.0]])
+    cy = np.concatenate([np.zeros(len(bottom)), np.ones(len(top)), [0.0]])
+    ox, oy = np.meshgrid(np.arange(k, dtype=float), np.arange(k, dtype=float))
+    px = (ox.reshape(-1, 1) + cx).reshape(-1)
+    py = (oy.reshape(-1, 1) + cy).reshape(-1) + px / 2.0
+    P = cs.Polygons(np.arange(k * k + 1, dtype=np.int32),
+                    np.arange(k * k + 1, dtype=np.int32) * len(cx), px * size, py * size,
+                    device="cuda")
+    rng = np.random.default_rng(edges + n)
+    ext = 1.5 * k
+    x, y = rng.uniform(0, ext, n), rng.uniform(0, ext, n)
+    t = np.arange(0, n, 3)
+    v = rng.integers(0, len(px), len(t))
+    kind = rng.integers(0, 3, len(t))
+    x[t] = np.where(kind == 2, x[t], px[v] + np.where(kind == 1, 0.0078125, 0.0))
+    y[t] = py[v] + np.where(kind == 1, 0.00390625, 0.0)
+    xy = torch.as_tensor(np.stack([x, y], 1).reshape(-1) * size, device="cuda")
+    grid = ranker.CandidateGrid.build(P, 0.0, 0.0, ext * size, 16)
+    bbox = (0.0, ext * size, 0.0, ext * size)
+    # a tree of depth 6 joins no leaf above its size there: none is above the last one
+    leaf = 64 if n <= 5000 else n
+    loc = ranker.LearnedLocator(P, grid, ranker.Ranker(grid.num_cells, seed=3), bbox,
+                                ext * size / 64, 6, leaf, check_partition=False)
+    want = exact_pairs(env, P, xy, bbox, 6, leaf)
+    for most in (16, 2):
+        res = loc.locate(cs.Points.from_points_xy(xy), max_tests=most)
+        got = res.pairs()
+        assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1]), most
+        assert int(res.tests.max()) <= most
+
+
 def test_fused_ranking_matches_gemm_logits(env):
     """The locator's fused MLP (rank_kernel, 16x16x32 MFMA, weights chained in
     registers) ranks like the training path's logits (qpip_ranker_logits, checked
