@@ -179,8 +179,16 @@ inline uint32_t polygon_group(uint64_t pairs, uint64_t polys, uint64_t edges_per
 // and every point is suspect) and n at [2^-70, 2^400] (outside, the line form's
 // c' is NaN), so no product overflows.
 //
-// Lane state is kept as wave-uniform 64-bit masks (one bit per lane and point
-// slot), so the loop's bookkeeping is a handful of scalar ops per edge.
+// An edge costs a subtraction, two fmas, half a minimum3 and two bit operations per
+// point slot: a comparison into a scalar mask takes as long as a fma and a half, so
+// the loop makes none. The sign bit of py - ay is "ay > py" (the difference of two
+// unequal doubles is never zero, and py is never -0, which the callers see to), a
+// lane's parity is the sign bit of an accumulated word, and |t| > tol is decided once per ring on the smallest high word of |t|: read
+// as a float it orders as |t| does, a NaN stays one through minimum, and a high word
+// above tol's is a value above tol. A |t| within 2^-20 above tol is marked too.
+// 2,000,003 points, 31 polygons of 4 to 256 vertices: 620 -> 522 us with nothing else
+// changed (bitmask kernel); the joins' tests, bound by the points' gathers, take what
+// they took.
 // Ring staging: a wave copies up to S line forms of the ring into its own LDS
 // slot with one coalesced vector load per lane (one memory latency per batch),
 // then walks them with broadcast LDS reads. Walking them from global memory took
@@ -194,12 +202,13 @@ constexpr int kStageEdges = kWave;  // the default depth, and the bitmask kernel
 // A wave's staged batch of line forms (LineEdge, built with the edge table).
 template <int S>
 struct PipStage {
-  LineEdge e[S];
+  LineEdge e[S + 1];  // e[0]: the vertex before the batch, for lane groups (its ay only)
 };
 
 // Point slots a wave holds at a time: lane l of slot u is point u * 64 + l of
 // the wave's current group (two slots keep the per-slot masks in few scalar
-// registers at eight waves per SIMD).
+// registers at seven waves per SIMD: a join of 31 million points runs in 4579 us, 4655
+// with eight, where vector registers spill).
 constexpr int kSlots = 2;
 
 // Largest |coordinate| of the wave's points in slots [0, nu) (NaN ignored).
@@ -219,13 +228,12 @@ __device__ __forceinline__ double wave_max_abs(double const (&px)[kSlots],
 // points, lane l holding point l % (64 / G) of copy g = l / (64 / G), and step e
 // gives copy g the ring's edge e * G + g: the G copies read G adjacent line forms.
 // A crossing toggles on the two ends of its own edge only: y1 from its first
-// vertex, y0 from the vertex before it, which is the previous edge's first vertex
-// and so copy g - 1's y1 of the same step (64 / G lanes down the ballot), or, for
-// copy 0, the last copy's y1 of the step before. The ring's parity is the XOR of
+// vertex, y0 from the vertex before it, the line form before (for a batch's first
+// edge the batch before's last vertex, kept ahead of the batch). The ring's parity is the XOR of
 // the copies' parities (the suspect marks their OR), so a flush of few points
 // takes G times fewer edge steps. The ring's last batch is padded to a multiple
 // of G with edges that neither toggle (their vertex repeats the ring's last one)
-// nor mark (t = +inf for finite points; for a point that is not finite t is NaN,
+// nor mark (t = 2^500 for finite points; for a point that is not finite t is NaN,
 // a mark, as on every real edge).
 // The reference's test of one point against rings [r0, r1) of a polygon
 // (is_point_in_polygon.cuh:46-100), on the vertices: a ring's first edge ends at
@@ -297,7 +305,14 @@ __device__ __forceinline__ RingHint ring_hint(PipArgs const& a, uint32_t poly)
   return h;
 }
 
-template <int U, int S = kStageEdges>
+__device__ __forceinline__ uint32_t high_word(double v)
+{
+  return static_cast<uint32_t>(static_cast<uint64_t>(__double_as_longlong(v)) >> 32);
+}
+__device__ __forceinline__ float high_as_float(double v) { return __uint_as_float(high_word(v)); }
+
+// R: edges per round of the loops, whose LDS reads are in flight together.
+template <int U, int S = kStageEdges, int R = 2>
 __device__ __forceinline__ void test_polygon(PipArgs const& a, uint32_t poly,
                                              double const (&px)[kSlots],
                                              double const (&py)[kSlots],
@@ -307,8 +322,12 @@ __device__ __forceinline__ void test_polygon(PipArgs const& a, uint32_t poly,
                                              RingHint const* hint = nullptr)
 {
   uint64_t inside_m[U], suspect_m[U];
+  uint32_t flip[U];  // sign bit: the lane's parity
 #pragma unroll
-  for (int u = 0; u < U; ++u) inside_m[u] = suspect_m[u] = 0;
+  for (int u = 0; u < U; ++u) {
+    suspect_m[u] = 0;
+    flip[u]      = 0;
+  }
   uint32_t r0 = 0, r1 = 0;
   if (poly >= a.num_polys) {
     err = true;
@@ -334,38 +353,34 @@ __device__ __forceinline__ void test_polygon(PipArgs const& a, uint32_t poly,
     // y0 of the first edge is its `b` (the ring's last vertex); afterwards the
     // previous edge's `a` (is_point_in_polygon.cuh:339, :375-376).
     double const by0 = hinted ? hint->by0 : ring_last_y(a, r);
-    uint64_t y0[U];
+    float const ftol = high_as_float(tol);
+    uint32_t w0[U];  // sign bit: the previous vertex is above the point
+    float near[U];   // the smallest |t|, by its high word
 #pragma unroll
-    for (int u = 0; u < U; ++u) y0[u] = ballot(by0 > py[u]);
+    for (int u = 0; u < U; ++u) {
+      w0[u]   = high_word(py[u] - by0);
+      near[u] = __builtin_inff();
+    }
     // The reference toggles on (y1 != y0) && ((lhs < rhs) != y1); the line form is
     // oriented so that t < 0 is (lhs < rhs) != y1 wherever the edge straddles.
     auto edge = [&](LineEdge const& ed) {
 #pragma unroll
       for (int u = 0; u < U; ++u) {
         double const t    = fma(px[u], ed.rise, fma(-py[u], ed.run, ed.c));
-        uint64_t const y1 = ballot(ed.ay > py[u]);
-        uint64_t const cr = ballot(t < 0.0);
-        suspect_m[u] |= ballot(!(fabs(t) > tol));
-        inside_m[u] ^= (y1 ^ y0[u]) & cr;
-        y0[u] = y1;
+        uint32_t const w1 = high_word(py[u] - ed.ay);
+        flip[u] ^= (w1 ^ w0[u]) & high_word(t);
+        near[u] = __builtin_elementwise_minimum(near[u], fabsf(high_as_float(t)));
+        w0[u]   = w1;
       }
     };
     if (U == 1 && lg != 0) {
       uint32_t const G  = 1u << lg;
-      uint32_t const Q  = static_cast<uint32_t>(kWave) >> lg;  // lanes per copy
       uint32_t const gq = static_cast<uint32_t>(lane) >> (6 - lg);
-      // y1 of the previous step; before edge 0 every copy holds the ring's b vertex
-      uint64_t y1p = ballot(by0 > py[0]);
-      // one step: copy g takes edge e + g; the vertex before it is the previous
-      // copy's edge (Q lanes down), or for copy 0 the last copy's previous step
-      auto step = [&](LineEdge const& ed) {
-        double const t    = fma(px[0], ed.rise, fma(-py[0], ed.run, ed.c));
-        uint64_t const y1 = ballot(ed.ay > py[0]);
-        uint64_t const cr = ballot(t < 0.0);
-        suspect_m[0] |= ballot(!(fabs(t) > tol));
-        uint64_t const y0 = (y1 << Q) | (y1p >> (kWave - Q));
-        inside_m[0] ^= (y1 ^ y0) & cr;
-        y1p = y1;
+      // one step: copy g takes edge e + g, `ed`, after the vertex of the form before it
+      auto step = [&](LineEdge const* ed) {
+        double const t = fma(px[0], ed->rise, fma(-py[0], ed->run, ed->c));
+        flip[0] ^= (high_word(py[0] - ed->ay) ^ high_word(py[0] - ed[-1].ay)) & high_word(t);
+        near[0] = __builtin_elementwise_minimum(near[0], fabsf(high_as_float(t)));
       };
       for (uint32_t base = 0; base < ne; base += S) {
         uint32_t const n   = ne - base < S ? ne - base : S;
@@ -376,20 +391,21 @@ __device__ __forceinline__ void test_polygon(PipArgs const& a, uint32_t poly,
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 #pragma unroll
         for (int i = 0; i < S; i += kWave)
-          if (static_cast<uint32_t>(i + lane) < n) stage->e[i + lane] = L[base + i + lane];
+          if (static_cast<uint32_t>(i + lane) < n) stage->e[1 + i + lane] = L[base + i + lane];
+        if (lane == 0) stage->e[0].ay = base ? L[base - 1].ay : by0;
         if (static_cast<uint32_t>(lane) < np - n)
-          stage->e[n + lane] = LineEdge{ylast, 0.0, 0.0, __builtin_inf()};
+          stage->e[1 + n + lane] = LineEdge{ylast, 0.0, 0.0, 0x1p500};
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        LineEdge const* E = &stage->e[gq];
+        LineEdge const* E = &stage->e[1 + gq];
         uint32_t e        = 0;
-        for (; e + 2 * G <= np; e += 2 * G) {
-          step(E[e]);
-          step(E[e + G]);
-        }
-        if (e < np) step(E[e]);
+        for (; e + R * G <= np; e += R * G)
+#pragma unroll
+          for (int i = 0; i < R; ++i) step(E + e + i * G);
+        for (; e < np; e += G) step(E + e);
       }
+      suspect_m[0] |= ballot(!(near[0] > ftol));
       continue;
     }
     for (uint32_t base = 0; base < ne; base += S) {
@@ -401,19 +417,22 @@ __device__ __forceinline__ void test_polygon(PipArgs const& a, uint32_t poly,
       __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 #pragma unroll
       for (int i = 0; i < S; i += kWave)
-        if (static_cast<uint32_t>(i + lane) < n) stage->e[i + lane] = L[base + i + lane];
+        if (static_cast<uint32_t>(i + lane) < n) stage->e[1 + i + lane] = L[base + i + lane];
       __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
       __builtin_amdgcn_wave_barrier();
       __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
       uint32_t e = 0;
       // unrolled so that the loop's scalar bookkeeping is amortised
-      for (; e + 2 <= n; e += 2) {
-        edge(stage->e[e]);
-        edge(stage->e[e + 1]);
-      }
-      if (e < n) edge(stage->e[e]);
+      for (; e + R <= n; e += R)
+#pragma unroll
+        for (int i = 0; i < R; ++i) edge(stage->e[1 + e + i]);
+      for (; e < n; ++e) edge(stage->e[1 + e]);
     }
+#pragma unroll
+    for (int u = 0; u < U; ++u) suspect_m[u] |= ballot(!(near[u] > ftol));
   }
+#pragma unroll
+  for (int u = 0; u < U; ++u) inside_m[u] = ballot((flip[u] >> 31) != 0u);
   if (U == 1 && lg != 0) {
     // the copies' parities and marks onto the first copy's lanes
     for (uint32_t sh = kWave / 2; sh >= (static_cast<uint32_t>(kWave) >> lg); sh >>= 1) {
@@ -540,7 +559,7 @@ __device__ __forceinline__ uint64_t xcd_block(uint64_t b, uint64_t grid, uint32_
 }
 
 template <int W, int S>  // W waves per workgroup, S edges per staged batch
-__global__ void __launch_bounds__(W * kWave) __attribute__((amdgpu_waves_per_eu(8)))
+__global__ void __launch_bounds__(W * kWave) __attribute__((amdgpu_waves_per_eu(7)))
   pip_test_kernel(PipArgs a, uint64_t base, uint32_t xcd_run, uint64_t* __restrict__ masks,
                   uint2* __restrict__ chunk_info, uint32_t* __restrict__ bad)
 {
@@ -606,6 +625,7 @@ __global__ void __launch_bounds__(W * kWave) __attribute__((amdgpu_waves_per_eu(
           }
         }
       }
+      py[u] += 0.0;  // -0 as +0 (test_polygon)
       valid_m[u] = ballot(valid);
     }
     double const pmax = wave_max_abs(px, py, nu);
@@ -791,6 +811,7 @@ __device__ __forceinline__ void pm_unit(PipArgs const& a, uint32_t i, uint32_t p
       qx[0]            = __shfl(qx[0], src, kWave);
       qy[0]            = __shfl(qy[0], src, kWave);
     }
+    qy[0] += 0.0;  // -0 as +0 (test_polygon)
     test_polygon<1, S>(a, poly, qx, qy, test_m, m, hit_m, err, stage, lg, &rh);
     if ((hit_m[0] >> lane) & 1ull)
       atomicOr(reinterpret_cast<unsigned long long*>(&masks[qtag >> 6]), 1ull << (qtag & 63u));
@@ -967,11 +988,11 @@ __device__ __forceinline__ void pm_unit(PipArgs const& a, uint32_t i, uint32_t p
 // One wave per unit of the unit list, in the XCD-run workgroup order (a
 // polygon's units are adjacent in the list, so its edges are fetched by one XCD);
 // the grid covers the most units the pairs can form, and waves past the count
-// return at once. No occupancy bound: held to the 7 or 8 waves per SIMD its LDS
-// would admit, the compiler spills vector registers to scratch; unbounded it
-// keeps 5 or 6 waves without spills, which measured faster.
+// return at once. Held to six waves per SIMD: 3,000 jobs in batches of 500 run in
+// 15.49 ms with six, 15.64 with the five the compiler would keep, 15.71 and 16.72 with
+// seven and eight, where it spills vector registers to scratch.
 template <int W, int S>
-__global__ void __launch_bounds__(W * kWave)
+__global__ void __launch_bounds__(W * kWave) __attribute__((amdgpu_waves_per_eu(6)))
   pip_test_pm_kernel(PipArgs a, uint64_t base, uint32_t xcd_run, uint64_t* __restrict__ masks,
                      uint2* __restrict__ chunk_info, uint32_t* __restrict__ bad)
 {
@@ -1176,14 +1197,16 @@ __device__ __forceinline__ void load_point(PipArgs const& a, uint64_t i, double&
 // What a polygon's test reads first (its box, ring range and first ring's entries)
 // is loaded once per workgroup, one polygon per thread, instead of as a chain of
 // dependent loads by every wave and polygon.
-// Bound by the edge steps (five FP64 instructions each, 40 cycles of a SIMD). 2,000,003
-// points, 31 polygons of 4 to 256 vertices, boxes of about a tenth of the square: every
-// point over every edge (two slots of 64 points) took 2020 us, this 620 us. Loading the
-// next polygon's first batch a polygon ahead with eight edges' LDS reads in flight
-// took 595 us for twice the vector registers, and is not done.
-constexpr int kBmChunks = 8;    // 64-point chunks per wave at most
+// Bound by the edge steps. 2,000,003 points, 31 polygons of 4 to 256 vertices, boxes of
+// about a tenth of the square: every point over every edge (two slots of 64 points)
+// took 2020 us, this 490 us (620 with a comparison per decision in the edge step). Two
+// edges' LDS reads in flight instead of four cost 17 us; eight change nothing.
+// Six chunks: fuller flushes than four or five (45 us), and 12 waves per CU, three on
+// each SIMD, where seven and eight chunks leave room for ten (22 us).
+constexpr int kBmChunks = 6;    // 64-point chunks per wave at most
 constexpr int kBmWaves  = 2;    // waves per workgroup
 constexpr int kBmStage  = 128;  // edges per staged batch
+constexpr int kBmRound  = 4;    // edges whose LDS reads are in flight together
 constexpr int kBmPolys  = 31;
 
 struct BmPoly {
@@ -1235,7 +1258,7 @@ __global__ void __launch_bounds__(kBmWaves * kWave)
     double px = 0.0, py = 0.0;
     if (i < n) load_point(a, i, px, py);
     pmax                   = fmax(pmax, fmax(fabs(px), fabs(py)));
-    s.p[c * kWave + lane]    = make_double2(px, py);
+    s.p[c * kWave + lane]    = make_double2(px, py + 0.0);  // -0 as +0 (test_polygon)
     s.bits[c * kWave + lane] = 0;
   }
 #pragma unroll
@@ -1267,7 +1290,7 @@ __global__ void __launch_bounds__(kBmWaves * kWave)
       double px[kSlots] = {pt.x, 0.0}, py[kSlots] = {pt.y, 0.0};
       uint64_t hit_m[kSlots] = {0, 0};
       uint64_t const test_m[kSlots] = {q >= kWave ? ~0ull : ((1ull << q) - 1ull), 0};
-      test_polygon<1, kBmStage>(a, j, px, py, test_m, pmax, hit_m, err, &s.stage, 6u - g, &rh);
+      test_polygon<1, kBmStage, kBmRound>(a, j, px, py, test_m, pmax, hit_m, err, &s.stage, 6u - g, &rh);
       if ((hit_m[0] >> lane) & 1ull) s.bits[slot] |= 1u << j;
     };
     for (uint32_t c = 0; c < nc; ++c) {

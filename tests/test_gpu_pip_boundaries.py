@@ -336,3 +336,45 @@ def test_order_chosen_by_shape_matches_oracle(cs, oracle_mod, kmin, n, fewer):
     assert len(pp) > 1000
     assert np.array_equal(hits["polygon_index"].cpu().numpy().astype(np.int64), pp.astype(np.int64))
     assert np.array_equal(hits["point_index"].cpu().numpy().astype(np.int64), pt.astype(np.int64))
+
+
+@pytest.mark.parametrize("edges", [3, 8, 63, 64, 65, 129])
+def test_signed_zeros_match_oracle(cs, oracle_mod, edges):
+    """Polygons with vertices at y = +0 and y = -0 and points at both, of ring lengths
+    around a staged batch: leaf-major, polygon-major (lane groups and full waves) and
+    bitmask tests, exact against the oracle."""
+    from cuspatial_amd import autotune
+
+    rng = np.random.default_rng(edges)
+    part, ring, vx, vy = [0], [0], [], []
+    for j in range(9):
+        a = 2 * np.pi * np.arange(edges) / edges
+        r = rng.uniform(2.0, 8.0, edges)
+        xs, ys = rng.uniform(-6, 6) + r * np.cos(a), r * np.sin(a)
+        at = rng.integers(0, edges, max(1, edges // 4))
+        ys[at] = np.where(rng.uniform(size=len(at)) < 0.5, 0.0, -0.0)
+        vx.extend(list(xs) + [xs[0]])
+        vy.extend(list(ys) + [ys[0]])
+        ring.append(len(vx))
+        part.append(j + 1)
+    polys = (np.array(part, np.int32), np.array(ring, np.int32), np.array(vx), np.array(vy))
+    n = 5000
+    x, y = rng.uniform(-16, 16, n), rng.uniform(-16, 16, n)
+    y[: n // 2] = np.where(rng.uniform(size=n // 2) < 0.5, 0.0, -0.0)
+    v = rng.integers(0, len(vx), 300)
+    x[:300] = polys[2][v]
+    x[300:400] = np.where(rng.uniform(size=100) < 0.5, 0.0, -0.0)
+    bbox = (-16.0, 16.0, -16.0, 16.0)
+    saved = autotune.current()
+    for stage, group in ((64, 0), (128, 0), (64, 16), (128, 64)):
+        try:
+            autotune.apply({"pip_stage_edges": stage, "pip_polygon_group": group})
+            g = run_gpu(cs, x, y, bbox, 2.0, 4, 24, polys)
+        finally:
+            autotune.apply(saved)
+        o = run_oracle(oracle_mod, x, y, bbox, 2.0, 4, 24, polys)
+        assert_same(g, o)
+    ref = oracle_mod.point_in_polygon_bitmask(x, y, *polys)
+    got = cs.point_in_polygon_bitmask(cs.Points(x, y, device="cuda"),
+                                      cs.Polygons(*polys, device="cuda"))
+    assert np.array_equal(got.cpu().numpy().astype(np.int64), ref.astype(np.int64))
