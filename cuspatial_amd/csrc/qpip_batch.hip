@@ -25,6 +25,7 @@
 //   * hits and point_indices are translated back to job-local indices.
 // A group's jobs never interact: every search is confined to its job's key range.
 #include <algorithm>
+#include <array>
 #include <memory>
 #include <vector>
 
@@ -627,11 +628,14 @@ std::vector<JobDev> job_descs(std::vector<HostJob> const& hj, int64_t j0, int64_
 
 // Upper bound of the forest's node count for jobs [j0, j1): 64 level-0 nodes per
 // job, then per level at most 4 children per internal node of the level above
-// (at most points / (max_size + 1) of them) and at most 4^level nodes.
+// (at most points / (max_size + 1) of them) and at most 64 * 4^level nodes. `most`
+// gets the bound of each level.
 uint64_t forest_capacity(std::vector<HostJob> const& hj, int64_t j0, int64_t j1,
-                         int64_t const* jpo)
+                         int64_t const* jpo, std::array<uint64_t, kMaxLevelsBatch>& most)
 {
-  uint64_t cap = 64ull * static_cast<uint64_t>(j1 - j0);
+  most.fill(0);
+  most[0]      = 64ull * static_cast<uint64_t>(j1 - j0);
+  uint64_t cap = most[0];
   for (int64_t j = j0; j < j1; ++j) {
     uint64_t const nj = static_cast<uint64_t>(jpo[j + 1] - jpo[j]);
     uint64_t const ib = nj / (static_cast<uint64_t>(hj[j].max_size) + 1);
@@ -639,6 +643,7 @@ uint64_t forest_capacity(std::vector<HostJob> const& hj, int64_t j0, int64_t j1,
       uint64_t c = std::min<uint64_t>(nj, 4 * ib);
       if (2 * l + 6 < 62) c = std::min<uint64_t>(c, uint64_t{64} << (2 * l));
       cap += c;
+      most[l] += c;
     }
   }
   QPIP_EXPECTS(cap < (uint64_t{1} << 32), "batched forest too large");
@@ -799,7 +804,8 @@ void run_group(std::vector<HostJob> const& hj, int64_t j0, int64_t j1, int64_t c
   vals_tmp.release();
 
   // 3. forest levels
-  uint64_t const cap = forest_capacity(hj, j0, j1, jpo);
+  std::array<uint64_t, kMaxLevelsBatch> most;  // nodes per level
+  uint64_t const cap = forest_capacity(hj, j0, j1, jpo, most);
   dbuf<uint32_t> nkey(cap), nstart(cap), ncount(cap), cfirst(cap), ccount(cap), njob(cap);
   dbuf<uint8_t> nlevel(cap);
   dbuf<uint4> split(cap), staging(static_cast<size_t>(J) * 64);
@@ -822,9 +828,9 @@ void run_group(std::vector<HostJob> const& hj, int64_t j0, int64_t j1, int64_t c
       LevelArgs la{sorted.keys, nkey.get(), nstart.get(), ncount.get(), nlevel.get(),
                    cfirst.get(), ccount.get(), split.get(), partials.get(), fmeta.get()->sizes,
                    &fmeta.get()->overflow, cap, l, samples.get()};
-      level_split_kernel<<<kLevelBlocks, 256, 0, stream>>>(la, rule);
+      level_split_kernel<<<level_blocks(most[l]), 256, 0, stream>>>(la, rule);
       QPIP_LAUNCH_CHECK();
-      level_emit_kernel<<<kLevelBlocks, 256, 0, stream>>>(la, rule);
+      level_emit_kernel<<<level_blocks(most[l]), 256, 0, stream>>>(la, rule);
       QPIP_LAUNCH_CHECK();
     }
   }
@@ -1093,6 +1099,7 @@ struct PlanGroup {
   uint64_t n = 0, npg = 0;
   int key_bits = 1, maxd = 0;
   uint64_t node_cap = 0;
+  std::array<uint64_t, kMaxLevelsBatch> level_most{};  // nodes per level at most
   bool tree = false, join = false;  // stages that run (host-known)
   PlanCaps cap;
   dbuf<JobDev> jobs;
@@ -1253,9 +1260,9 @@ void plan_enqueue(BatchPlan& P, PlanGroup& g, size_t gi, hipStream_t s)
                    g.cfirst.get(), g.ccount.get(), g.split.get(), g.partials.get(),
                    g.fmeta.get()->sizes, &g.fmeta.get()->overflow, g.node_cap, l,
                    g.samples.get()};
-      level_split_kernel<<<kLevelBlocks, 256, 0, s>>>(la, rule);
+      level_split_kernel<<<level_blocks(g.level_most[l]), 256, 0, s>>>(la, rule);
       QPIP_LAUNCH_CHECK();
-      level_emit_kernel<<<kLevelBlocks, 256, 0, s>>>(la, rule);
+      level_emit_kernel<<<level_blocks(g.level_most[l]), 256, 0, s>>>(la, rule);
       QPIP_LAUNCH_CHECK();
     }
   }
@@ -1401,7 +1408,7 @@ void plan_group_setup(BatchPlan& P, PlanGroup& g, hipStream_t s)
   g.vals_tmp.reset(g.n);
   g.samples.reset((g.n + 31) / 32);
   g.counts0.reset(g.num_stiles * kRadix);
-  g.node_cap = forest_capacity(hj, g.j0, g.j1, jpo);
+  g.node_cap = forest_capacity(hj, g.j0, g.j1, jpo, g.level_most);
   uint64_t const cap = g.node_cap;
   g.nkey.reset(cap);
   g.nstart.reset(cap);
