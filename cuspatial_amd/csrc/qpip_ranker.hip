@@ -14,7 +14,8 @@
 // bf16 operands, fp32 accumulation, on MFMA (v_mfma_f32_16x16x32_bf16, and
 // v_mfma_f32_16x16x16_bf16 where the contraction is over the 16 slots). The
 // locator tests the candidates in the order of their logits with the exact FP64
-// point-in-polygon test of the quadtree path (same edge table, same arithmetic)
+// point-in-polygon test of the quadtree path (same edge table, same arithmetic; for
+// short rings a single-precision form first, whose outcome counts where it is certain)
 // and stops at the first polygon that contains the point away from its edges.
 // Points whose only hit is close to an edge, or whose cell lists more than 16
 // candidates, or that have no hit after max_tests tests, are marked for the
