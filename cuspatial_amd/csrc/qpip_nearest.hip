@@ -283,13 +283,18 @@ struct RunChunkOp {
 //
 // With M the largest float32 coordinate met (points and vertices), every float32
 // distance is within 2^-19 M of the exact one (rounded ends, direction, projection and
-// difference: at most 31 roundings of 2^-24 M) and the reference's double result
-// within 2^-25 M (the cancellation of d0 - r), so E = 2^-17 M + 1e-14 bounds both: a
-// linestring whose distance is more than 2 E below every other's is the reference's
-// nearest (and no other one's distance is zero). Its distance is then computed as the
-// reference does. Otherwise (two linestrings that near, a zero distance, a linestring
-// without segments, coordinates that are not finite or above 1e15) the lane folds over
-// the run's pairs.
+// difference: at most 31 roundings of 2^-24 M), and so is the reference's double result
+// (within 2^-23 M: the cancellation of d0 - r) except where
+//  * the point lies on a segment: d0 - r may round below zero, and the distance is NaN;
+//  * a segment's length^2 and its d3^2 underflow to 0: r = 0 / 0, and fmin drops the
+//    segment, so the distance comes out larger.
+// E = 2^-17 M + 1e-14 bounds both kinds of rounding. Where one float32 distance is more
+// than 2 E below every other, no other linestring comes out as near, as zero or as NaN
+// (the first exception needs a distance below 2^-23 M, the second only adds to one). If
+// the reference's distance to that linestring is then within E of the float32 one it is
+// the answer. Otherwise (an exception above, two linestrings that near, a zero distance,
+// a linestring without segments, coordinates that are not finite or above 1e15) the lane
+// folds over the run's pairs, as the reference does.
 //
 // Bound by the float32 instructions. 1e6 points, 20,000 linestrings of 2 to 32
 // vertices (about 15 per leaf of 61 points): one wave per pair, each segment a chain of
@@ -459,7 +464,7 @@ __global__ void __launch_bounds__(kNearWaves * kWave)
   if (own && decided) {
     best_ls = a.pair_ls[l1];
     best_d  = own_linestring_distance(a, best_ls, px, py);
-    decided = best_d != 0.0;
+    decided = best_d > 0.0 && fabs(best_d - static_cast<double>(sqrtf(m1))) <= E;  // not NaN
   }
   if (own && !decided) fold_run(a, rs, rs + R, px, py, best_ls, best_d, err);
   if (own) {

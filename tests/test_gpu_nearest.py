@@ -150,6 +150,64 @@ def test_chunks_and_undecided_points_match_oracle(cs, oracle_mod, case, n, ms):
     assert np.array_equal(np_(res["distance"]).view(np.int64), od.view(np.int64))
 
 
+def leaf_fold(cs, oracle_mod, x, y, offs, lx, ly, bbox):
+    """Every linestring against the one leaf of all points, on the GPU and in the oracle:
+    indices, and distances bit for bit (a NaN is one on both sides)."""
+    import torch
+
+    pts, L = cs.Points(x, y, device="cuda"), cs.Linestrings(offs, lx, ly, device="cuda")
+    pi, tree = cs.quadtree_on_points(pts, *bbox, bbox[1] - bbox[0], 1, len(x))
+    t = tuple(np_(tree[c]) for c in ("key", "level", "is_internal_node", "length", "offset"))
+    assert t[3].tolist() == [len(x)]
+    pl = np.arange(len(offs) - 1, dtype=np.uint32)
+    pq = np.zeros(len(pl), np.uint32)
+    pairs = {c: torch.as_tensor(v.astype(np.int64), device="cuda")
+             for c, v in (("a", pl), ("b", pq))}
+    res = cs.quadtree_point_to_nearest_linestring(pairs, tree, pi, pts, L)
+    opt, ols, od = oracle_mod.quadtree_point_to_nearest_linestring(
+        (pl, pq), t, np_(pi), x, y, offs, lx, ly)
+    assert np.array_equal(np_(res["point_index"]), opt)
+    assert np.array_equal(np_(res["linestring_index"]), ols)
+    d = np_(res["distance"])
+    assert np.array_equal(np.isnan(d), np.isnan(od))
+    ok = ~np.isnan(od)
+    assert np.array_equal(d[ok].view(np.int64), od[ok].view(np.int64))
+    return ols, od
+
+
+@pytest.mark.parametrize("at", [0, 1, 2])
+@pytest.mark.parametrize("n", [20, 2000])
+def test_points_on_a_segment_match_oracle(cs, oracle_mod, n, at):
+    """Points a + t (b - a) of a sloped segment: d0 - r rounds below zero at some of them,
+    the distance to their own linestring is NaN and the fold goes on to the next pair.
+    That linestring first, in the middle and last of its run."""
+    rng = np.random.default_rng(n + at)
+    b = (97.3, 61.7)
+    t = rng.uniform(0.02, 0.98, n)
+    x, y = t * b[0], t * b[1]
+    far = [((0.0, 99.0), (100.0, 100.0)), ((99.0, 0.0), (100.0, 30.0))]
+    lines = far[:at] + [((0.0, 0.0), b)] + far[at:]
+    v = np.array(lines).reshape(-1, 2)
+    offs = np.arange(0, 2 * len(lines) + 1, 2).astype(np.int32)
+    ols, od = leaf_fold(cs, oracle_mod, x, y, offs, v[:, 0].copy(), v[:, 1].copy(),
+                        (0.0, 100.0, 0.0, 100.0))
+    # the scene meets the case: some points lose their own linestring, or keep its NaN
+    lost = np.isnan(od) if at == 2 else ols != at
+    assert 0 < lost.sum() < n
+
+
+@pytest.mark.parametrize("first", [True, False])
+def test_underflowing_segment_matches_oracle(cs, oracle_mod, first):
+    """A linestring of one segment whose squared length and projection underflow: the
+    reference drops the segment, so the point's nearest is the other, farther one."""
+    tiny, other = ((0.0, 0.0), (1e-163, 0.0)), ((3.0, 3.0), (4.0, 3.0))
+    v = np.array([tiny, other] if first else [other, tiny]).reshape(-1, 2)
+    ols, od = leaf_fold(cs, oracle_mod, np.array([0.5]), np.array([0.1]),
+                        np.array([0, 2, 4], np.int32), v[:, 0].copy(), v[:, 1].copy(),
+                        (0.0, 4.0, 0.0, 4.0))
+    assert ols[0] == (1 if first else 0) and 3.8 < od[0] < 3.9
+
+
 def test_empty_and_errors(cs):
     import torch
 
