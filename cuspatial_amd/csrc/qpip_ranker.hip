@@ -1187,7 +1187,8 @@ __global__ void __launch_bounds__(kVerWaves * kWave, 7)
 
   // the point's outcome
   auto write = [&](int64_t p, int32_t result, uint32_t tests, uint32_t flags) {
-    if (!(result >= 0 && tests == 1)) flags |= 2u;  // first prediction was not the answer
+    // the first prediction was not the answer (an overflowed cell makes none: 1, no test)
+    if (!(result >= 0 && tests == 1) && !(tests == 0 && flags == 1u)) flags |= 2u;
     a.out_poly[p]  = (flags & 1u) ? -2 : result;
     a.out_tests[p] = static_cast<uint8_t>(tests);
     a.out_flags[p] = static_cast<uint8_t>(flags);

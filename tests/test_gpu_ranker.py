@@ -304,6 +304,34 @@ def test_locator_short_rings_equal_plain_join(env, edges, exponent, n):
         assert int(res.tests.max()) <= most
 
 
+def test_flags_of_points_without_a_prediction(env):
+    """Points of a cell with too many candidates are left to the quadtree path without a
+    test or a prediction (flags 1), and those of a cell without candidates have no answer
+    (flags 2); the other points' tests and flags do not change."""
+    torch, cs, ranker, rk, _ = env
+    _, P, grid, xy, x, y = voronoi(env, 20000, 150, 9, 16)
+    model = ranker.Ranker(grid.num_cells, seed=3)
+    bbox = (0.0, 1e5, 0.0, 1e5)
+
+    def locate(g):
+        loc = ranker.LearnedLocator(P, g, model, bbox, 1e5 / 1024, 10, 64, check_partition=False)
+        return loc.locate(cs.Points.from_points_xy(xy))
+
+    plain = locate(grid)
+    counts = grid.counts.clone()
+    counts[0::3] = ranker.OVERFLOW
+    counts[1::3] = 0
+    res = locate(ranker.CandidateGrid(grid.x0, grid.y0, grid.cell, grid.dim, grid.candidates,
+                                      counts))
+    kind = grid.cells_of(xy) % 3
+    over, none, rest = kind == 0, kind == 1, kind == 2
+    assert min(over.sum(), none.sum(), rest.sum()) > 1000
+    assert (res.flags[over] == 1).all() and (res.flags[none] == 2).all()
+    assert (res.tests[over | none] == 0).all()
+    assert torch.equal(res.flags[rest], plain.flags[rest])
+    assert torch.equal(res.tests[rest], plain.tests[rest])
+
+
 def test_fused_ranking_matches_gemm_logits(env):
     """The locator's fused MLP (rank_kernel, 16x16x32 MFMA, weights chained in
     registers) ranks like the training path's logits (qpip_ranker_logits, checked
