@@ -380,6 +380,8 @@ def point_in_polygon(points: Points, polygons: Polygons):
     # Byte plane k holds bits 8k .. 8k + 7 of every point; eight points' bytes per
     # word, one shift and one mask turn a plane into its eight columns of 0 / 1 bytes.
     n = bits.numel()
+    if n == 0:
+        return Table((j, bits.to(torch.bool)) for j in range(len(polygons)))
     planes = torch.empty((4, (n + 255) // 256 * 256), dtype=torch.uint8, device=bits.device)
     planes[:, :n] = bits.view(torch.uint8).view(n, 4).t()
     shifts = torch.arange(8, device=bits.device)

@@ -225,6 +225,23 @@ def test_brute_force_pip_empty(capi):
     assert _brute(capi, True, npo=1) == (capi.QPIP_SUCCESS, 0, None)
 
 
+@pytest.mark.parametrize("polygons", [1, 9, 31])
+def test_point_in_polygon_without_points(capi, polygons):
+    """No points: one empty bool column per polygon."""
+    import numpy as np
+    import torch
+
+    import cuspatial_amd as cs
+
+    part = np.arange(polygons + 1, dtype=np.int32)
+    ring = (4 * part).astype(np.int32)
+    v = np.tile([0.0, 1.0, 1.0, 0.0], polygons)
+    points = cs.Points(np.zeros(0), np.zeros(0), device="cpu")
+    out = cs.point_in_polygon(points, cs.Polygons(part, ring, v, v, device="cpu"))
+    assert out.columns == list(range(polygons))
+    assert all(c.dtype == torch.bool and c.shape == (0,) for c in out.values())
+
+
 def test_noalloc_pip_preconditions_and_limits(capi):
     """qpip_point_in_polygon_noalloc: the bitmask entry point's checks, then its
     scratch limits (262,144 vertices, 65,536 rings), all decided before any device
