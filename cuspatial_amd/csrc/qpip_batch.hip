@@ -911,8 +911,8 @@ void run_group(std::vector<HostJob> const& hj, int64_t j0, int64_t j1, int64_t c
     JoinSink const sink{dm, out_node.get(), out_bbox.get(), ka.get(), nullptr, nullptr,
                         join_counts.get(), cap_out, cap_fr, 0, 0};
     launch_join(top, tv, bv, geom, sink, {fa_node.get(), fb_node.get()},
-                {fa_bbox.get(), fb_bbox.get()}, std::max(maxd, 1), join_partials.get(),
-                stream, "batch_join_level");
+                {fa_bbox.get(), fb_bbox.get()}, std::max(maxd, 1), join_shape(M, npg),
+                join_partials.get(), stream, "batch_join_level");
     read_back({{&h_meta, dm, sizeof(JoinMeta)}}, stream);
     if (h_meta.bad_index) throw logic_error("cuSpatial failure: forest child range out of range");
     if (!h_meta.overflow) break;
@@ -1300,8 +1300,11 @@ void plan_enqueue(BatchPlan& P, PlanGroup& g, size_t gi, hipStream_t s)
   BatchTopSource const top{g.trees.get(), g.jobs.get(), g.top_off.get(), g.J, dm};
   JoinSink const sink{dm, g.out_node.get(), g.out_bbox.get(), nullptr, nullptr, nullptr,
                       g.join_counts.get(), g.cap.pairs, g.cap.frontier, 0, 0};
+  // a tree's nodes are about 4/3 of its widest level's, which level_most bounds
+  uint64_t const widest = *std::max_element(g.level_most.begin(), g.level_most.end());
   launch_join(top, tv, bv, geom, sink, {g.fa_node.get(), g.fb_node.get()},
-              {g.fa_bbox.get(), g.fb_bbox.get()}, levels, g.join_partials.get(), s, "batch_join_level");
+              {g.fa_bbox.get(), g.fb_bbox.get()}, levels, join_shape(widest + widest / 3, g.npg),
+              g.join_partials.get(), s, "batch_join_level");
   plan_pairs_kernel<<<1, 64, 0, s>>>(dm, levels, g.cap.pairs, g.fmeta.get(), cnt, prev);
   QPIP_LAUNCH_CHECK();
   plan_gather_kernel<<<grid_for(g.cap.pairs, 256), 256, 0, s>>>(

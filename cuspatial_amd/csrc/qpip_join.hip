@@ -8,8 +8,8 @@
 // children in order, and finally stable-sorts the leaf pairs by the leaf's first
 // point position.
 //
-// Here the same traversal runs entirely on the device, one count/scan/emit per
-// kJoinStep levels (qpip_join.hpp) with the frontier length kept in device memory (the
+// Here the same traversal runs entirely on the device, one count/scan/emit per step
+// of one to three levels (qpip_join.hpp) with the frontier length kept in device memory (the
 // reference syncs the host on every level for sizes, traversal.cuh:222). The stable
 // sort is the library's LSD radix sort over the bits of the largest leaf offset.
 // Frontier/output capacities are preallocated; on overflow the traversal is
@@ -168,7 +168,8 @@ extern "C" int qpip_join_quadtree_and_bounding_boxes(const uint32_t* key,
       JoinSink const sink{dm, out_node.get(), out_bbox.get(), ka.get(), nullptr, nullptr,
                           counts.get(), cap_out, cap_fr, 0, 0};
       launch_join(TopSource{dm}, tv, bv, prm, sink, {fa_node.get(), fb_node.get()},
-                  {fa_bbox.get(), fb_bbox.get()}, max_depth, partials.get(), stream, "join_level");
+                  {fa_bbox.get(), fb_bbox.get()}, max_depth, join_shape(M, B), partials.get(), stream,
+                  "join_level");
       read_back({{&h_meta, dm, sizeof(JoinMeta)}}, stream);
       if (h_meta.bad_index)
         throw logic_error("cuSpatial failure: quadtree child range exceeds the number of nodes");

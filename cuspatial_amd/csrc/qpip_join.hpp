@@ -108,14 +108,12 @@ __device__ __forceinline__ uint64_t level_out_base(JoinMeta const* meta, int lvl
 // The traversal (quadtree_bbox_filtering.cuh:53-166, traversal.cuh:63-145) is breadth
 // first: each (quad node, box) element of a frontier is replaced by its children that
 // meet the box, leaves go to the output and quads to the next frontier, both in element
-// order. A step here takes kJoinStep levels at once: an element's thread descends its
-// subtree that far, counting its leaves per level and the quads below; after one scan
-// of the four counts each level's leaves and the next frontier are written in the same
-// order as level by level (within a level, path order is element order). Two launches
-// per step instead of per level: the launches and their fixed part (7 to 16 us a level
-// for a few thousand elements) were most of a join's time. Three levels: at most 21
-// quads per element are expanded in turn by one thread, about as long as three
-// levels' launches take.
+// order. A step here takes up to kJoinStep levels at once: an element's thread descends
+// its subtree that far, counting its leaves per level and the quads below; after one
+// scan of the four counts each level's leaves and the next frontier are written in the
+// same order as level by level (within a level, path order is element order). Two
+// launches per step instead of per level, for quads that one thread expands in turn (at
+// most 21 per element at three levels, 5 at two); join_shape says how many levels.
 constexpr int kJoinStep = 3;
 
 // Counts of one element: leaves of the step's levels 0 and 1, of level 2 and quads.
@@ -328,20 +326,47 @@ struct FrontierSource {
   }
 };
 
+// Levels per step and blocks of the grid, by the tree's nodes and the boxes. Measured
+// with 3, 2 and 1 levels per step (us of all steps' kernels):
+//   * no more nodes than boxes, so few of a step's nodes meet a box and the launches
+//     count: one request of 20,000 points and 50,000 boxes 621 / 644 / 711 (whole call);
+//   * more nodes, where a thread's quads in turn cost more than launches: 84 nodes and
+//     200 boxes 27 / 25 / 43, 21,844 and 1,000 85 / 77 / 89, 1.22 million and 50,000 (of
+//     36 edges) 260 / 216 / 246, and with boxes that cover the domain 5,456 nodes and 10
+//     boxes 109 / 66 / 72, 113,432 and 20,000 257 / 186 / 214, 639,000 and 5,000
+//     312 / 228 / 236;
+//   * from 2^20 nodes and 64 per box the frontiers fill the GPU at every level: 1.21
+//     million and 100 boxes 868 / 583 / 551, 1.4 million and 20,000 719 / 764 / 687, 2.18
+//     million and 20,000 1959 / 1188 / 954 (1002 with the children classified twice).
+// The grid has a block per 64 boxes or 512 nodes, at most kScanBlocks and 64 at least: a
+// box meets a few nodes of a level, or it covers many and their number is the nodes'.
+// 1.21 million nodes and 100 boxes at three levels per step: 1367 us with 65 blocks (the
+// boxes alone), 874 with this many or 1024; 84 nodes and 200 boxes 27 against 31.
+struct JoinShape {
+  int levels;
+  unsigned blocks;
+};
+
+inline JoinShape join_shape(uint64_t nodes, uint64_t boxes)
+{
+  uint64_t const want   = 64 + (boxes + nodes / 8) / 64;
+  unsigned const blocks = static_cast<unsigned>(want < kScanBlocks ? want : kScanBlocks);
+  if (nodes <= boxes) return {kJoinStep, blocks};
+  return {nodes >= (uint64_t{1} << 20) && nodes / 64 >= boxes ? 1 : 2, blocks};
+}
+
 // The whole traversal of `depth` levels from the top elements; fr[2] are the frontiers'
-// node and box arrays, used in turn. The grid has a block per 64 boxes, at most
-// kScanBlocks (and 64 at least): a box meets a few nodes of a level.
+// node and box arrays, used in turn.
 template <class Top, class Geom>
 void launch_join(Top const& top, TreeView const& t, BoxView const& bx, Geom const& g, JoinSink s,
                  uint32_t* const (&fr_node)[2], uint32_t* const (&fr_bbox)[2], int depth,
-                 StepCount* partials, hipStream_t stream, char const* timer)
+                 JoinShape shape, StepCount* partials, hipStream_t stream, char const* timer)
 {
-  uint64_t const want   = 64 + bx.b / 64;
-  unsigned const blocks = static_cast<unsigned>(want < kScanBlocks ? want : kScanBlocks);
-  for (int lvl = 0, step = 0; lvl < depth; lvl += kJoinStep, ++step) {
+  unsigned const blocks = shape.blocks;
+  for (int lvl = 0, step = 0; lvl < depth; lvl += shape.levels, ++step) {
     KernelTimer kt(timer, stream);
     s.lvl     = lvl;
-    s.levels  = depth - lvl < kJoinStep ? depth - lvl : kJoinStep;
+    s.levels  = depth - lvl < shape.levels ? depth - lvl : shape.levels;
     s.fr_node = fr_node[step % 2];
     s.fr_bbox = fr_bbox[step % 2];
     if (lvl == 0) {

@@ -389,6 +389,36 @@ def test_gaussian_holes_full_size_properties(cs, oracle_mod):
 # ---------------------------------------------------------------------------
 # boundary behaviour
 # ---------------------------------------------------------------------------
+@pytest.mark.parametrize("n,d,ms,zones,nodes", [
+    (20000, 6, 256, 900, (100, 900)),             # no more nodes than boxes: three levels a step
+    (60000, 8, 8, 40, (5000, 1 << 20)),           # more: two
+    (1300000, 11, 1, 30, (1 << 20, 1 << 32)),     # from 2^20 and 64 per box: one
+    (1300000, 11, 1, 40000, (1 << 20, 1 << 32)),  # ... unless there are fewer per box
+])
+def test_join_steps_match_oracle(cs, oracle_mod, n, d, ms, zones, nodes):
+    """The join's levels per step and grid (join_shape): a partition of the square into
+    zones, whose boxes meet many nodes, on both sides of each line. The oracle's pairs."""
+    rng = np.random.default_rng(n + zones)
+    ext = 1024.0
+    pts = cs.Points(rng.uniform(0, ext, n), rng.uniform(0, ext, n))
+    _, tree = cs.quadtree_on_points(pts, 0.0, ext, 0.0, ext, ext / 2**d, d, ms)
+    assert nodes[0] <= len(tree) < nodes[1]
+    # columns of uneven widths, each cut into rows
+    cols = max(1, int(np.sqrt(zones)))
+    x = np.concatenate([[0.0], np.sort(rng.uniform(0, ext, cols - 1)), [ext]])
+    rows = zones // cols
+    y = np.linspace(0.0, ext, rows + 1)
+    boxes = [np.repeat(x[:-1], rows), np.tile(y[:-1], cols), np.repeat(x[1:], rows),
+             np.tile(y[1:], cols)]
+    pairs = cs.join_quadtree_and_bounding_boxes(tree, boxes, 0.0, ext, 0.0, ext, ext / 2**d, d)
+    t = tuple(np_(tree[c]) for c in ("key", "level", "is_internal_node", "length", "offset"))
+    ob, oq = oracle_mod.join_quadtree_and_bounding_boxes(t, boxes, 0.0, ext, 0.0, ext,
+                                                         ext / 2**d, d)
+    assert len(ob) > len(boxes[0])
+    assert np.array_equal(np_(pairs["bbox_offset"]), ob)
+    assert np.array_equal(np_(pairs["quad_offset"]), oq)
+
+
 def test_deterministic(cs):
     x, y, polys = scene(41, 300000)
     a = run_gpu(cs, x, y, (0.0, 100.0, 0.0, 100.0), 100 / 2**10, 10, 50, polys)
