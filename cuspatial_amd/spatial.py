@@ -377,18 +377,25 @@ def point_in_polygon(points: Points, polygons: Polygons):
     if len(polygons) == 0:
         return Table()
     bits = _brute_force(points, polygons, pairwise=False)
+    n, P = bits.numel(), len(polygons)
+    if n == 0 or P == 1:  # one polygon: the bits are its column
+        return Table((j, bits.to(torch.bool)) for j in range(P))
     # Byte plane k holds bits 8k .. 8k + 7 of every point; eight points' bytes per
-    # word, one shift and one mask turn a plane into its eight columns of 0 / 1 bytes.
-    n = bits.numel()
-    if n == 0:
-        return Table((j, bits.to(torch.bool)) for j in range(len(polygons)))
-    planes = torch.empty((4, (n + 255) // 256 * 256), dtype=torch.uint8, device=bits.device)
-    planes[:, :n] = bits.view(torch.uint8).view(n, 4).t()
-    shifts = torch.arange(8, device=bits.device)
-    words = planes.view(torch.int64)[:, None, :] >> shifts[None, :, None]
-    words &= 0x0101010101010101
-    table = words.view(32, -1).view(torch.bool)
-    return Table((j, table[j, :n]) for j in range(len(polygons)))
+    # word, a shift and a mask turn a plane into its columns of 0 / 1 bytes.
+    row = (n + 255) // 256 * 256
+    planes = torch.empty(((P + 7) // 8, row), dtype=torch.uint8, device=bits.device)
+    planes[:, :n] = bits.view(torch.uint8).view(n, 4).t()[:planes.shape[0]]
+    planes = planes.view(torch.int64)[:, None]
+    shifts = torch.arange(8, device=bits.device)[:, None]
+    table = torch.empty((P, row // 8), dtype=torch.int64, device=bits.device)
+    full = P // 8  # planes whose eight columns are all there, then the last plane's
+    if full:
+        torch.bitwise_right_shift(planes[:full], shifts, out=table[:8 * full].view(full, 8, -1))
+    if P % 8:
+        torch.bitwise_right_shift(planes[full], shifts[:P % 8], out=table[8 * full:])
+    table &= 0x0101010101010101
+    table = table.view(torch.bool)
+    return Table((j, table[j, :n]) for j in range(P))
 
 
 def point_in_polygon_bitmask(points: Points, polygons: Polygons) -> torch.Tensor:
