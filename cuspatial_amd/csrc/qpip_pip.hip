@@ -1188,6 +1188,51 @@ __device__ __forceinline__ void load_point(PipArgs const& a, uint64_t i, double&
   }
 }
 
+// Few edges in all: one wave takes 128 points (two per lane) over every polygon's edges.
+// Neither boxes (a launch less) nor queue.
+__global__ void __launch_bounds__(256)
+  pip_bitmask_direct_kernel(PipArgs a, uint64_t n, int32_t* __restrict__ out)
+{
+  __shared__ PipStage<kStageEdges> s_stage[256 / kWave];
+  PipStage<kStageEdges>* const stage = &s_stage[threadIdx.x / kWave];
+  uint64_t const p0 = (static_cast<uint64_t>(blockIdx.x) * (256 / kWave) + threadIdx.x / kWave) *
+                      (kSlots * kWave);
+  if (p0 >= n) return;
+  int const lane      = lane_id();
+  uint64_t const left = (n - p0 + kWave - 1) / kWave;
+  uint32_t const nu   = left < kSlots ? static_cast<uint32_t>(left) : kSlots;
+  double px[kSlots], py[kSlots];
+  uint64_t valid_m[kSlots];
+  uint32_t bits[kSlots];
+#pragma unroll
+  for (int u = 0; u < kSlots; ++u) {
+    uint64_t const i = p0 + static_cast<uint64_t>(u) * kWave + lane;
+    bool const valid = i < n;
+    px[u] = py[u] = 0.0;
+    if (valid) load_point(a, i, px[u], py[u]);
+    py[u] += 0.0;  // -0 as +0 (test_polygon)
+    valid_m[u] = ballot(valid);
+    bits[u]    = 0;
+  }
+  double const pmax = wave_max_abs(px, py, nu);
+  bool err          = false;
+  for (uint32_t j = 0; j < a.num_polys; ++j) {
+    uint64_t hit_m[kSlots] = {0, 0};
+    if (nu == 1)
+      test_polygon<1>(a, j, px, py, valid_m, pmax, hit_m, err, stage);
+    else
+      test_polygon<2>(a, j, px, py, valid_m, pmax, hit_m, err, stage);
+#pragma unroll
+    for (int u = 0; u < kSlots; ++u)
+      bits[u] |= static_cast<uint32_t>((hit_m[u] >> lane) & 1ull) << j;
+  }
+#pragma unroll
+  for (int u = 0; u < kSlots; ++u) {
+    uint64_t const i = p0 + static_cast<uint64_t>(u) * kWave + lane;
+    if (i < n) out[i] = static_cast<int32_t>(bits[u]);
+  }
+}
+
 // One wave holds up to kBmChunks chunks of 64 points in LDS and takes the polygons one
 // after the other: the points inside the polygon's vertex box (box_excludes, with the
 // wave's largest coordinate in place of the point's own: a wider margin, so it keeps
@@ -1325,12 +1370,31 @@ __global__ void __launch_bounds__(kBmWaves * kWave)
   }
 }
 
-// Enqueues the test of n points against a.num_polys <= 31 polygons. Chunks per wave:
-// as many as leave 4,096 waves (four per SIMD), since the more points a wave holds
-// the fuller its queue's flushes are.
+// Whether the test takes the polygons' boxes and queue: where the polygons have more
+// vertices on average than a point's box test and its share of a flush cost. Every edge
+// against box and queue (us, whole call): 4e6 points, 57 vertices of 8 polygons 84 / 94,
+// 221 of 31 252 / 276, 355 of 31 331 / 290, 59 of one 64 / 44; 2.5e6 points, 110 of 16
+// 100 / 113, 169 of 16 121 / 119, 284 of 16 167 / 133. Below 2^20 points a wave holds one
+// or two chunks, whose flushes are less full: 3e5 points, 348 of 31 58 / 96, 408 of 16
+// 54 / 62, 1125 of 31 114 / 104; 1e5 points, 320 of 16 38 / 39, 593 of 31 61 / 56.
+inline bool bitmask_boxes(uint64_t n, int64_t polys, int64_t vertices)
+{
+  return vertices > (n < (uint64_t{1} << 20) ? 16 : 10) * polys + 8;
+}
+
+// Enqueues the test of n points against a.num_polys <= 31 polygons: box filter and queue
+// where the polygons have boxes, else every edge. Chunks per wave there: as many as leave 4,096 waves (four per SIMD), since the
+// more points a wave holds the fuller its queue's flushes are.
 void launch_bitmask(PipArgs const& a, uint64_t n, int32_t* out, hipStream_t stream)
 {
   KernelTimer kt("pip_bitmask", stream);
+  if (!a.poly_box) {
+    pip_bitmask_direct_kernel<<<static_cast<unsigned>((n + 4 * kSlots * kWave - 1) /
+                                                      (4 * kSlots * kWave)),
+                                256, 0, stream>>>(a, n, out);
+    QPIP_LAUNCH_CHECK();
+    return;
+  }
   uint64_t const all = (n + kWave - 1) / kWave;
   uint32_t const chunks =
     static_cast<uint32_t>(std::min<uint64_t>(kBmChunks, std::max<uint64_t>(1, all / 4096)));
@@ -1713,18 +1777,21 @@ int point_in_polygon_entry(const double* x,
     dbuf<uint32_t> ring_edges(std::max<uint64_t>(num_rings, 1));
     dbuf<LineEdge> lines(pairwise ? 1 : std::max<int64_t>(num_poly_x, 1));
     dbuf<double> ring_amax(pairwise ? 1 : std::max<uint64_t>(num_rings, 1));
-    dbuf<PolyBox> ring_box(pairwise ? 1 : std::max<uint64_t>(num_rings, 1));
-    dbuf<PolyBox> poly_box(pairwise ? 1 : std::max<int64_t>(num_polys, 1));
+    bool const boxes = !pairwise && num_polys > 0 && bitmask_boxes(n, num_polys, num_poly_x);
+    dbuf<PolyBox> ring_box, poly_box;
+    if (boxes) {
+      ring_box.reset(std::max<uint64_t>(num_rings, 1));
+      poly_box.reset(num_polys);
+    }
     if (num_rings > 0) {
       KernelTimer kt("pip_edges", stream);
       build_edges_kernel<<<grid_for(num_rings, 256 / kWave), 256, 0, stream>>>(
         reinterpret_cast<uint32_t const*>(ring_offsets), static_cast<int64_t>(num_rings), poly_x,
         poly_y, num_poly_x, nullptr, nullptr, ring_edges.get(),
-        pairwise ? nullptr : lines.get(), pairwise ? nullptr : ring_amax.get(),
-        pairwise ? nullptr : ring_box.get());
+        pairwise ? nullptr : lines.get(), pairwise ? nullptr : ring_amax.get(), ring_box.get());
       QPIP_LAUNCH_CHECK();
     }
-    if (!pairwise && num_polys > 0) {
+    if (boxes) {
       poly_box_kernel<<<1, 256, 0, stream>>>(
         reinterpret_cast<uint32_t const*>(poly_offsets), static_cast<uint64_t>(num_polys),
         num_rings, ring_box.get(), poly_box.get());
@@ -1898,8 +1965,10 @@ extern "C" int qpip_point_in_polygon_noalloc(const double* x,
     uint32_t* const ring_edges = reinterpret_cast<uint32_t*>(base + kNoAllocRingsOff);
     LineEdge* const lines      = reinterpret_cast<LineEdge*>(base + kNoAllocLinesOff);
     double* const ring_amax    = reinterpret_cast<double*>(base + kNoAllocAmaxOff);
-    PolyBox* const ring_box    = reinterpret_cast<PolyBox*>(base + kNoAllocBoxOff);
-    PolyBox* const poly_box    = reinterpret_cast<PolyBox*>(base + kNoAllocPolyOff);
+    uint64_t const n           = static_cast<uint64_t>(num_x);
+    bool const boxes           = num_polys > 0 && bitmask_boxes(n, num_polys, num_poly_x);
+    PolyBox* const ring_box = boxes ? reinterpret_cast<PolyBox*>(base + kNoAllocBoxOff) : nullptr;
+    PolyBox* const poly_box = boxes ? reinterpret_cast<PolyBox*>(base + kNoAllocPolyOff) : nullptr;
     // Every ring's entry and every edge a ring keeps are written below before the
     // test reads them; the test reads nothing else of the scratch, so nothing a
     // previous call left there needs clearing.
@@ -1909,13 +1978,12 @@ extern "C" int qpip_point_in_polygon_noalloc(const double* x,
         poly_y, num_poly_x, nullptr, nullptr, ring_edges, lines, ring_amax, ring_box);
       QPIP_LAUNCH_CHECK();
     }
-    if (num_polys > 0) {
+    if (boxes) {
       poly_box_kernel<<<1, 256, 0, stream>>>(
         reinterpret_cast<uint32_t const*>(poly_offsets), static_cast<uint64_t>(num_polys),
         num_rings, ring_box, poly_box);
       QPIP_LAUNCH_CHECK();
     }
-    uint64_t const n = static_cast<uint64_t>(num_x);
     PipArgs a{};
     a.num_points   = n;
     a.x            = x;

@@ -633,6 +633,42 @@ def test_bitmask_box_filter_and_queue(cs, oracle_mod, n):
         assert len(tbl[j]) == n and np.array_equal(np_(tbl[j]), ((ref >> j) & 1).astype(bool))
 
 
+@pytest.mark.parametrize("n", [1, 64, 65, 128, 129, 600001, 1048577])
+@pytest.mark.parametrize("polygons", [1, 5, 31])
+def test_bitmask_of_few_vertices_and_the_line(cs, oracle_mod, n, polygons):
+    """The bitmask test without boxes at the edges of its 128-point waves, and the line in
+    vertices (10 or 16 per polygon and 8) at which the box filter takes over: one vertex
+    less, at it and one more. Points on vertices, NaN, infinite and huge. Exact."""
+    rng = np.random.default_rng(n + polygons)
+    line = (10 if n >= 1 << 20 else 16) * polygons + 8
+    x, y = rng.uniform(-5, 105, n), rng.uniform(-5, 105, n)
+    for m, v in enumerate((np.nan, np.inf, -np.inf, 1e130, -1e200)):
+        if 2 * m + 1 < n:
+            x[2 * m], y[2 * m + 1] = v, v
+    for total in (4 * polygons, line - 1, line, line + 1):
+        counts = np.full(polygons, total // polygons) + (np.arange(polygons) < total % polygons)
+        part, ring, vx, vy = [0], [0], [], []
+        for c in counts:
+            a = np.sort(rng.uniform(0, 2 * np.pi, c - 1))
+            r = rng.uniform(5, 40, c - 1)
+            at = rng.uniform(0, 100, 2)
+            vx += list(at[0] + r * np.cos(a)) + [at[0] + r[0] * np.cos(a[0])]
+            vy += list(at[1] + r * np.sin(a)) + [at[1] + r[0] * np.sin(a[0])]
+            ring.append(len(vx))
+            part.append(len(part))
+        assert len(vx) == total
+        vx, vy = np.array(vx), np.array(vy)
+        k = min(n // 3, total)
+        if k:
+            x[n - k:], y[n - k:] = vx[:k], vy[:k]
+        ref = oracle_mod.point_in_polygon_bitmask(x, y, np.array(part, np.int32),
+                                                  np.array(ring, np.int32), vx, vy)
+        got = cs.point_in_polygon_bitmask(
+            cs.Points(x, y, device="cuda"),
+            cs.Polygons(np.array(part, np.int32), np.array(ring, np.int32), vx, vy, device="cuda"))
+        assert np.array_equal(np_(got).astype(np.int64), ref.astype(np.int64)), total
+
+
 @pytest.mark.parametrize("seed,n", [(61, 1), (62, 5000), (63, 200001)])
 def test_pairwise_point_in_polygon_random(cs, oracle_mod, seed, n):
     rng = np.random.default_rng(seed)
