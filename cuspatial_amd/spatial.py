@@ -387,11 +387,13 @@ def point_in_polygon(points: Points, polygons: Polygons):
     planes[:, :n] = bits.view(torch.uint8).view(n, 4).t()[:planes.shape[0]]
     planes = planes.view(torch.int64)[:, None]
     shifts = torch.arange(8, device=bits.device)[:, None]
-    table = torch.empty((P, row // 8), dtype=torch.int64, device=bits.device)
-    full = P // 8  # planes whose eight columns are all there, then the last plane's
+    # the last plane's columns with the others' where that is two spare ones at most,
+    # else in a launch of their own
+    full = (P + 2) // 8
+    table = torch.empty((max(P, 8 * full), row // 8), dtype=torch.int64, device=bits.device)
     if full:
         torch.bitwise_right_shift(planes[:full], shifts, out=table[:8 * full].view(full, 8, -1))
-    if P % 8:
+    if P > 8 * full:
         torch.bitwise_right_shift(planes[full], shifts[:P % 8], out=table[8 * full:])
     table &= 0x0101010101010101
     table = table.view(torch.bool)

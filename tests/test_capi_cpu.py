@@ -242,11 +242,11 @@ def test_point_in_polygon_without_points(capi, polygons):
     assert all(c.dtype == torch.bool and c.shape == (0,) for c in out.values())
 
 
-@pytest.mark.parametrize("polygons", [1, 2, 3, 8, 9, 16, 31])
+@pytest.mark.parametrize("polygons", [1, 2, 5, 6, 7, 8, 9, 16, 31])
 @pytest.mark.parametrize("points", [1, 255, 257, 5000])
 def test_point_in_polygon_table(capi, monkeypatch, points, polygons):
     """The table's columns are the bitmask's bits, and what they keep alive is a byte per
-    point and polygon that there is (rows of whole 256 bytes)."""
+    point and polygon that there is, or two more (rows of whole 256 bytes)."""
     import torch
 
     from cuspatial_amd import spatial
@@ -258,7 +258,7 @@ def test_point_in_polygon_table(capi, monkeypatch, points, polygons):
     assert out.columns == list(range(polygons))
     for j, column in out.items():
         assert torch.equal(column, ((bits >> j) & 1).to(torch.bool)) and column.is_contiguous()
-        assert column.untyped_storage().nbytes() <= polygons * (points + 255)
+        assert column.untyped_storage().nbytes() <= (polygons + 2) * (points + 255)
 
 
 def test_noalloc_pip_preconditions_and_limits(capi):
