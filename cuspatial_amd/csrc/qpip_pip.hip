@@ -134,8 +134,8 @@ inline uint32_t pairs_per_wave(uint64_t num_pairs)
   return static_cast<uint32_t>(v > (1u << 30) ? (1u << 30) : v);
 }
 
-// Pairs per unit of the polygon-major test, 0 for the leaf-major one. A set
-// pip_polygon_group decides; otherwise polygon order is taken where a pair's cost is
+// Pairs per unit of the polygon-major test, 0 for the leaf-major one. A pip_polygon_group
+// that is not 0 decides (-1: leaf-major); otherwise polygon order is taken where a pair's cost is
 // its ring's edges rather than its leaf's points: long rings, polygons that meet few
 // leaves (so their boxes keep few of a leaf's points) and enough pairs to fill the
 // GPU. Measured, leaf against polygon order (us, order included): 256 jobs of 130-edge
@@ -144,7 +144,7 @@ inline uint32_t pairs_per_wave(uint64_t num_pairs)
 inline uint32_t polygon_group(uint64_t pairs, uint64_t polys, uint64_t edges_per_poly)
 {
   int64_t const set = tuning(Tuning::PipPolygonGroup);
-  if (set > 0) return static_cast<uint32_t>(set);
+  if (set != 0) return set > 0 ? static_cast<uint32_t>(set) : 0u;
   return pairs >= (1u << 14) && edges_per_poly >= 64 && pairs <= 8 * polys ? 64 : 0;
 }
 

@@ -98,7 +98,7 @@ QPIP_API void qpip_memory_info(size_t* live_bytes, size_t* cached_bytes);
  *                           every candidate point (default 1)
  *   pip_polygon_group       0: the test's order is chosen by the join's shape
  *                           (default): leaf by leaf, or by polygon where rings are
- *                           long and meet few leaves;
+ *                           long and meet few leaves; -1: leaf by leaf;
  *                           n > 0: it groups the pairs by polygon, one wave taking up
  *                           to n pairs of one polygon and packing their kept
  *                           points from several leaves into full waves

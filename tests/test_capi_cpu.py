@@ -391,6 +391,12 @@ def test_tuning_parameters(capi):
     assert autotune.get("pip_xcd_run") == 16
     assert autotune.get("pip_box_filter") == 1
     assert autotune.get("pip_polygon_group") == 0
+    autotune.set("pip_polygon_group", -1)  # leaf by leaf, whatever the shape
+    assert autotune.get("pip_polygon_group") == -1
+    autotune.set("pip_polygon_group", 0)
+    assert -1 in autotune.PARAMETERS["pip_polygon_group"][0]
+    with pytest.raises(RuntimeError, match="out of range"):
+        autotune.set("pip_polygon_group", -2)
     with pytest.raises(RuntimeError, match="out of range"):
         autotune.set("pip_box_filter", 2)
     with pytest.raises(RuntimeError, match="out of range"):

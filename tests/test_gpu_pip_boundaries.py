@@ -309,33 +309,62 @@ def test_long_rings_few_points_match_oracle(cs, oracle_mod, stage, group, box):
         assert len(o["polygon_index"]) > 0
 
 
+def order_scene(seed, polygons, kmin, rmin, rmax):
+    """60,000 points (some on vertices) against star polygons of kmin to kmin + 2 edges."""
+    rng = np.random.default_rng(seed)
+    ext = 1000.0
+    part, ring, vx, vy = star_polygons(rng, polygons, ext, rmin, rmax, kmin=kmin, kmax=kmin + 2)
+    x, y = rng.uniform(0, ext, 60000), rng.uniform(0, ext, 60000)
+    x[:500], y[:500] = vx[:500], vy[:500]
+    return (x, y), (part, ring, vx, vy), (0.0, ext, 0.0, ext)
+
+
+def join_of_scene(cs, points, polys, bbox):
+    """The join's columns and tree of 64 x 64 deepest cells, ready for the test."""
+    pts, P = cs.Points(*points, device="cuda"), cs.Polygons(*polys, device="cuda")
+    scale = bbox[1] / 64
+    pi, tree = cs.quadtree_on_points(pts, *bbox, scale, 6, 64)
+    bb = cs.polygon_bounding_boxes(P)
+    return cs.join_quadtree_and_bounding_boxes(tree, bb, *bbox, scale, 6), tree, pi, pts, P
+
+
+def timed_order(cs, args):
+    """The hits and whether the test sorted the pairs by polygon (its timer ran)."""
+    from cuspatial_amd import _capi
+
+    _capi.profile_reset()
+    _capi.profile_enable(True)
+    try:
+        hits = cs.quadtree_point_in_polygon(*args)
+    finally:
+        _capi.profile_enable(False)
+    report = _capi.profile_report()
+    return hits, "pip_order" in report
+
+
 @pytest.mark.parametrize("kmin,n,fewer", [(63, 9000, 0), (70, 9000, 0), (70, 2500, 0),
                                           (70, 9000, 1)])
 def test_order_chosen_by_shape_matches_oracle(cs, oracle_mod, kmin, n, fewer):
     """The rule that takes the polygon-major order by itself (mean ring length from 64,
     2^14 pairs, at most eight pairs per polygon), on both sides of each line: rings a
     little shorter and longer, fewer pairs, larger polygons with more pairs each. Hits
-    exact against the oracle, in its order."""
-    rng = np.random.default_rng(kmin + n + fewer)
-    ext = 1000.0
+    exact against the oracle, in its order; a set order is the one that runs."""
+    from cuspatial_amd import autotune
+
     size = (750, 30.0, 60.0) if fewer else (n, 4.0, 9.0)
-    part, ring, vx, vy = star_polygons(rng, size[0], ext, *size[1:], kmin=kmin, kmax=kmin + 2)
-    x, y = rng.uniform(0, ext, 60000), rng.uniform(0, ext, 60000)
-    k = 500
-    x[:k], y[:k] = vx[:k], vy[:k]
-    d, ms, scale = 6, 64, ext / 64
-    pts, P = cs.Points(x, y, device="cuda"), cs.Polygons(part, ring, vx, vy, device="cuda")
-    pi, tree = cs.quadtree_on_points(pts, 0.0, ext, 0.0, ext, scale, d, ms)
-    bb = cs.polygon_bounding_boxes(P)
-    pairs = cs.join_quadtree_and_bounding_boxes(tree, bb, 0.0, ext, 0.0, ext, scale, d)
-    hits = cs.quadtree_point_in_polygon(pairs, tree, pi, pts, P)
+    points, polys, bbox = order_scene(kmin + n + fewer, size[0], kmin, *size[1:])
+    args = join_of_scene(cs, points, polys, bbox)
+    pairs, tree, pi = args[:3]
     t = tuple(v.cpu().numpy() for v in tree.values())
     pp, pt = oracle_mod.quadtree_point_in_polygon(
-        tuple(v.cpu().numpy() for v in pairs.values()), t, pi.cpu().numpy(), x, y, part, ring, vx,
-        vy)
+        tuple(v.cpu().numpy() for v in pairs.values()), t, pi.cpu().numpy(), *points, *polys)
     assert len(pp) > 1000
-    assert np.array_equal(hits["polygon_index"].cpu().numpy().astype(np.int64), pp.astype(np.int64))
-    assert np.array_equal(hits["point_index"].cpu().numpy().astype(np.int64), pt.astype(np.int64))
+    for group in (0, -1, 64):
+        with autotune.applied({"pip_polygon_group": group}):
+            hits, ordered = timed_order(cs, args)
+        assert group == 0 or ordered == (group > 0), (group, len(pairs))
+        for c, ref in (("polygon_index", pp), ("point_index", pt)):
+            assert np.array_equal(hits[c].cpu().numpy().astype(np.int64), ref.astype(np.int64))
 
 
 @pytest.mark.parametrize("edges", [3, 8, 63, 64, 65, 129])
