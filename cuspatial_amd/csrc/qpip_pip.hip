@@ -136,16 +136,27 @@ inline uint32_t pairs_per_wave(uint64_t num_pairs)
 
 // Pairs per unit of the polygon-major test, 0 for the leaf-major one. A pip_polygon_group
 // that is not 0 decides (-1: leaf-major); otherwise polygon order is taken where a pair's cost is
-// its ring's edges rather than its leaf's points: long rings, polygons that meet few
-// leaves (so their boxes keep few of a leaf's points) and enough pairs to fill the
-// GPU. Measured, leaf against polygon order (us, order included): 256 jobs of 130-edge
-// stars with 2.3 pairs each 457 / 342, 500 such jobs 683 / 325, 30 jobs (9,000 pairs)
-// 71 / 74; 36-edge polygons with 7 pairs each 1012 / 1618, 20-edge stars 35 / 71.
+// its ring's edges rather than its leaf's points (long rings, polygons that meet few
+// leaves, so that their boxes keep few of a leaf's points) and there are polygons for
+// waves and pairs enough to be worth the sort. Measured, leaf against polygon order (us,
+// order included), leaves of 61 points and of 244, polygons x edges, pairs of each:
+//   12,000 x 64, 3.4   87 /   90    209 /  240     12,000 x 130, 3.4  140 / 103   346 /  271
+//   30,000 x 64, 1.8  112 /  105    263 /  303      6,000 x 130, 3.4   82 /  79   197 /  165
+//   30,000 x 64, 5.9  351 /  269   1759 / 1611      6,000 x 64,  5.9   80 /  98   192 /  245
+//   60,000 x 64, 3.4  388 /  262   1972 / 1627     30,000 x 130, 1.9  177 / 118   432 /  314
+//    3,000 x 200, 1.9   54 /   61    129 /   87      1,500 x 400, 6.2  124 / 150   316 /  383
+// and 256 jobs of 130-edge stars with 2.3 pairs each 457 / 342, 36-edge polygons with 7
+// pairs each 1012 / 1618. What is gained grows with the polygons and with the square of
+// the edges, which is how the lines are drawn: of 560 shapes measured none that takes
+// polygon order loses more than 3%.
 inline uint32_t polygon_group(uint64_t pairs, uint64_t polys, uint64_t edges_per_poly)
 {
   int64_t const set = tuning(Tuning::PipPolygonGroup);
   if (set != 0) return set > 0 ? static_cast<uint32_t>(set) : 0u;
-  return pairs >= (1u << 14) && edges_per_poly >= 64 && pairs <= 8 * polys ? 64 : 0;
+  uint64_t const e  = edges_per_poly < 4096 ? edges_per_poly : 4096;
+  bool const enough = polys >= 4096 && polys * e * e >= (3u << 25) &&
+                      pairs * e * e >= (1u << 28);
+  return enough && edges_per_poly >= 64 && pairs <= 8 * polys ? 64 : 0;
 }
 
 // --- 3. test ------------------------------------------------------------------------

@@ -342,27 +342,33 @@ def timed_order(cs, args):
     return hits, "pip_order" in report
 
 
-@pytest.mark.parametrize("kmin,n,fewer", [(63, 9000, 0), (70, 9000, 0), (70, 2500, 0),
-                                          (70, 9000, 1)])
-def test_order_chosen_by_shape_matches_oracle(cs, oracle_mod, kmin, n, fewer):
-    """The rule that takes the polygon-major order by itself (mean ring length from 64,
-    2^14 pairs, at most eight pairs per polygon), on both sides of each line: rings a
-    little shorter and longer, fewer pairs, larger polygons with more pairs each. Hits
-    exact against the oracle, in its order; a set order is the one that runs."""
+@pytest.mark.parametrize("kmin,n,radius,by_polygon", [
+    (130, 12000, 6.0, True),
+    (130, 5000, 6.0, False),    # polygons * edges^2 below 3 * 2^25
+    (160, 4000, 8.0, False),    # ... above, but fewer than 4096 polygons
+    (160, 4200, 8.0, True),
+    (110, 12000, 0.5, False),   # pairs * edges^2 below 2^28
+    (60, 32000, 6.0, False),    # below 64 edges
+    (64, 32000, 6.0, True),
+    (130, 6500, 24.0, False),   # more than eight pairs per polygon
+])
+def test_order_chosen_by_shape_matches_oracle(cs, oracle_mod, kmin, n, radius, by_polygon):
+    """The rule that takes the polygon-major order by itself (polygon_group), on both sides
+    of each of its lines. Hits exact against the oracle, in its order; a set order is the
+    one that runs."""
     from cuspatial_amd import autotune
 
-    size = (750, 30.0, 60.0) if fewer else (n, 4.0, 9.0)
-    points, polys, bbox = order_scene(kmin + n + fewer, size[0], kmin, *size[1:])
+    points, polys, bbox = order_scene(kmin + n, n, kmin, 0.9 * radius, 1.1 * radius)
     args = join_of_scene(cs, points, polys, bbox)
     pairs, tree, pi = args[:3]
     t = tuple(v.cpu().numpy() for v in tree.values())
     pp, pt = oracle_mod.quadtree_point_in_polygon(
         tuple(v.cpu().numpy() for v in pairs.values()), t, pi.cpu().numpy(), *points, *polys)
-    assert len(pp) > 1000
+    assert len(pp) > 500
     for group in (0, -1, 64):
         with autotune.applied({"pip_polygon_group": group}):
             hits, ordered = timed_order(cs, args)
-        assert group == 0 or ordered == (group > 0), (group, len(pairs))
+        assert ordered == (by_polygon if group == 0 else group > 0), (group, len(pairs))
         for c, ref in (("polygon_index", pp), ("point_index", pt)):
             assert np.array_equal(hits[c].cpu().numpy().astype(np.int64), ref.astype(np.int64))
 
