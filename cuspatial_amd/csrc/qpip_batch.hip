@@ -1131,6 +1131,7 @@ struct PlanGroup {
   dbuf<uint64_t> pm_partials, pm_total, pm_num_units;
   dbuf<uint2> chunk_info;
   uint32_t pairs_per_wave = 16;
+  uint64_t pairs = 0;  // the sizing run's count (the capacity until there is one)
 };
 
 }  // namespace
@@ -1340,6 +1341,7 @@ void plan_enqueue(BatchPlan& P, PlanGroup& g, size_t gi, hipStream_t s)
   d.num_vertices   = static_cast<uint64_t>(P.num_vertices);
   d.edges_per_poly = P.edges_per_poly;
   d.poly_box       = P.poly_box.get() + g.PO0;
+  d.pairs          = g.pairs;
   d.pairs_per_wave = g.pairs_per_wave;
   d.chunk_start    = g.chunk_start.get();
   d.partials       = g.pip_partials.get();
@@ -1683,7 +1685,8 @@ extern "C" int qpip_batch_plan_create(int64_t num_jobs,
       for (auto& g : P->groups) {
         if (!g->join) continue;
         plan_alloc(*g);
-        g->pairs_per_wave = pip_pairs_per_wave(g->cap.pairs);
+        g->pairs          = g->cap.pairs;
+        g->pairs_per_wave = pip_pairs_per_wave(g->pairs);
         H += g->cap.hits;
       }
       P->hit_cap = H;
@@ -1743,7 +1746,10 @@ extern "C" int qpip_batch_plan_create(int64_t num_jobs,
     }
     alloc_all();
     for (size_t gi = 0; gi < G; ++gi)
-      if (P->groups[gi]->join) P->groups[gi]->pairs_per_wave = pip_pairs_per_wave(measured[gi].pairs);
+      if (PlanGroup& g = *P->groups[gi]; g.join) {
+        g.pairs          = measured[gi].pairs;
+        g.pairs_per_wave = pip_pairs_per_wave(g.pairs);
+      }
     QPIP_HIP(hipStreamSynchronize(s));
 
     // capture the whole sequence once

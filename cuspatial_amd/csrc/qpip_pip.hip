@@ -118,7 +118,8 @@ struct PipArgs {
   double const* poly_y  = nullptr;
   uint64_t num_vertices = 0;
   uint32_t pm_group        = 0;
-  uint32_t edges_per_poly  = 0;  // mean ring vertices per polygon (the order's rule)
+  uint32_t edges_per_poly  = 0;  // the order's rule: mean ring vertices per polygon,
+  uint64_t expected_pairs  = 0;  // and the pairs to expect
 };
 
 // Segments of at most max(m, pairs >> s) pairs (m = 2, s = 24 by default; both
@@ -1127,7 +1128,7 @@ void launch_pip_test(PipArgs const& args, uint64_t pairs, uint64_t* masks, uint2
 {
   PipArgs a = args;
   if (tuning(Tuning::PipBoxFilter) == 0) a.poly_box = nullptr;
-  uint32_t const group = polygon_group(pairs, a.num_polys, a.edges_per_poly);
+  uint32_t const group = polygon_group(a.expected_pairs, a.num_polys, a.edges_per_poly);
   bool const pm = group > 0 && pmb != nullptr && a.num_polys > 0 &&
                   a.chunk_cap < (uint64_t{1} << 32);  // slots in 32 bits (PmPair)
   if (pm) {
@@ -1458,6 +1459,7 @@ void launch_pip_device(PipDevice const& d, hipStream_t stream)
   args.poly_y       = d.poly_y;
   args.num_vertices = d.num_vertices;
   args.edges_per_poly = d.edges_per_poly;
+  args.expected_pairs = d.pairs;
   QPIP_EXPECTS(args.num_vertices == 0 || (args.poly_x && args.poly_y),
                "polygon vertices must not be null");
   PmBuffers const pmb{d.pm_count,    d.pm_start, d.pm_cursor, d.pm_order,
@@ -1619,6 +1621,7 @@ int quadtree_point_in_polygon_entry(const uint32_t* poly_index,
       args.poly_y       = poly_y;
       args.num_vertices = static_cast<uint64_t>(num_poly_x);
       args.edges_per_poly = static_cast<uint32_t>(std::min<uint64_t>(edges, 0xFFFFFFFFu));
+      args.expected_pairs = K;
       launch_pip_test(args, K, masks.get(), chunk_info.get(), bad.get() + 1,
                       pm_on ? &pmb : nullptr, stream);
       // chunks past the capacity were not tested: the scan covers those that were

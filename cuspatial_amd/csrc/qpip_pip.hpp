@@ -45,6 +45,7 @@ struct PipDevice {
   double const* poly_y  = nullptr;
   uint64_t num_vertices = 0;
   uint32_t edges_per_poly = 0;  // mean ring vertices per polygon
+  uint64_t pairs          = 0;  // pairs to expect (pair_cap has headroom): the order's rule
   PolyBox const* poly_box;  // per polygon (null: the test filters no points)
   uint32_t pairs_per_wave;
   // workspace

@@ -147,6 +147,30 @@ def test_plan_capacity_exceeded_is_reported(cs):
     plan2.close()
 
 
+@pytest.mark.parametrize("polygons,headroom", [(200, 1.25), (200, 8.0), (600, 1.25)])
+def test_plan_in_the_order_of_its_shape_matches_eager(cs, polygons, headroom):
+    """Plans whose PIP test takes the order by shape: jobs of long rings whose pairs are
+    below the rule's line while the plan's room for them is above it, and above it."""
+    from cuspatial_amd import _capi, datasets
+
+    w = datasets.batched_jobs(seed=polygons, num_jobs=40, min_points=500, max_points=2000,
+                              min_polygons=polygons, max_polygons=polygons + 50, min_vertices=100,
+                              max_vertices=200, ext=1e4)
+    xy, P = device_inputs(cs, w)
+    _capi.profile_reset()
+    _capi.profile_enable(True)
+    try:
+        want = eager(cs, w, xy, P)
+    finally:
+        _capi.profile_enable(False)
+    assert ("pip_order" in _capi.profile_report()) == (polygons == 600)
+    plan = make_plan(cs, w, xy, P, headroom)
+    for _ in range(3):
+        plan.launch()
+        assert_same(plan.result(), want)
+    plan.close()
+
+
 def test_plan_under_each_saved_tuning_matches_eager(cs, tmp_path):
     """A plan looks its shape bucket up in a tuning table and is captured under
     those values; every configuration of the table (and of the package's own
