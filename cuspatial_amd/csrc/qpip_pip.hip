@@ -1482,6 +1482,35 @@ void launch_pip_device(PipDevice const& d, hipStream_t stream)
   }
 }
 
+namespace {
+
+// Memory of the polygon-major test's pair order (PmBuffers).
+struct PmOrder {
+  dbuf<uint32_t> count, start, cursor;
+  dbuf<uint4> order, units;
+  dbuf<uint64_t> partials, total, num_units;
+
+  void reset(uint64_t polys, uint64_t pairs)
+  {
+    count.reset(polys), start.reset(polys), cursor.reset(polys);
+    order.reset(pairs), units.reset(pairs);
+    partials.reset(kScanBlocks + 1), total.reset(1), num_units.reset(1);
+  }
+  void release()
+  {
+    count.release(), start.release(), cursor.release();
+    order.release(), units.release();
+    partials.release(), total.release(), num_units.release();
+  }
+  PmBuffers get() const
+  {
+    return {count.get(), start.get(),    cursor.get(), order.get(),
+            units.get(), partials.get(), total.get(),  num_units.get()};
+  }
+};
+
+}  // namespace
+
 // The plain test's entry, also used by the batched eager call (point_base non-null:
 // point_indices are job-local and point_base[node] is the node's job's first point).
 int quadtree_point_in_polygon_entry(const uint32_t* poly_index,
@@ -1585,13 +1614,8 @@ int quadtree_point_in_polygon_entry(const uint32_t* poly_index,
     uint64_t const edges = edges_per_poly > 0 ? edges_per_poly
                            : num_polys > 0    ? static_cast<uint64_t>(num_poly_x) / num_polys
                                               : 0;
-    bool const pm_on     = polygon_group(K, num_polys, edges) > 0 && num_polys > 0;
-    dbuf<uint32_t> pm_count(pm_on ? num_polys : 1), pm_start(pm_on ? num_polys : 1),
-      pm_cursor(pm_on ? num_polys : 1);
-    dbuf<uint4> pm_order(pm_on ? K : 1), pm_units(pm_on ? K : 1);
-    dbuf<uint64_t> pm_partials(kScanBlocks + 1), pm_total(1), pm_num_units(1);
-    PmBuffers const pmb{pm_count.get(), pm_start.get(),    pm_cursor.get(), pm_order.get(),
-                        pm_units.get(), pm_partials.get(), pm_total.get(),  pm_num_units.get()};
+    bool pm_on           = polygon_group(K, num_polys, edges) > 0 && num_polys > 0;
+    PmOrder pm;
     uint64_t h_tot[2] = {0, 0};
     uint32_t h_bad[2] = {0, 0};
     for (;;) {
@@ -1610,6 +1634,18 @@ int quadtree_point_in_polygon_entry(const uint32_t* poly_index,
         exact     = true;
         continue;
       }
+      dbuf<uint64_t> n_chunks(1);
+      // The order's buffers only help: where the memory limit refuses them the test runs
+      // leaf by leaf. They go back before the hits' are asked for.
+      if (pm_on) {
+        try {
+          pm.reset(num_polys, K);
+        } catch (oom_error const&) {
+          pm.release();
+          pm_on = false;
+        }
+      }
+      PmBuffers const pmb = pm.get();
       PipArgs args{poly_index, quad_index, K, length, offset, point_indices,
                    n_pts, x, y, poly_offsets, num_polys, num_rings, ring_offsets,
                    ring_edges.get(), lines.get(), ring_amax.get(),
@@ -1624,8 +1660,8 @@ int quadtree_point_in_polygon_entry(const uint32_t* poly_index,
       args.expected_pairs = K;
       launch_pip_test(args, K, masks.get(), chunk_info.get(), bad.get() + 1,
                       pm_on ? &pmb : nullptr, stream);
+      pm.release();
       // chunks past the capacity were not tested: the scan covers those that were
-      dbuf<uint64_t> n_chunks(1);
       clamp_count_kernel<<<1, 64, 0, stream>>>(totals.get(), chunk_cap, n_chunks.get(),
                                                bad.get() + 1);
       QPIP_LAUNCH_CHECK();

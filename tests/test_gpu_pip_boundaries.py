@@ -373,6 +373,42 @@ def test_order_chosen_by_shape_matches_oracle(cs, oracle_mod, kmin, n, radius, b
             assert np.array_equal(hits[c].cpu().numpy().astype(np.int64), ref.astype(np.int64))
 
 
+def test_order_that_does_not_fit_the_memory_limit(cs):
+    """Where the memory limit holds the leaf-major test but not the polygon-major test's
+    pair order beside it, a call whose shape asks for that order runs leaf by leaf."""
+    from cuspatial_amd import _capi, autotune
+
+    args = join_of_scene(cs, *order_scene(3, 12000, 130, 5.4, 6.6))
+    L = _capi.lib()
+    want, ordered = timed_order(cs, args)
+    assert ordered
+
+    def fits(limit):
+        L.qpip_set_memory_limit(limit)
+        try:
+            with autotune.applied({"pip_polygon_group": -1}):
+                cs.quadtree_point_in_polygon(*args)
+            return True
+        except MemoryError:
+            return False
+        finally:
+            L.qpip_set_memory_limit(0)
+
+    lo, hi = 0, 1 << 30  # multiples of the pool's 512-byte grain
+    while hi - lo > 512:
+        mid = (lo + hi) // 1024 * 512
+        lo, hi = (lo, mid) if fits(mid) else (mid, hi)
+    for limit, by_polygon in ((hi, False), (hi + (16 << 20), True)):
+        L.qpip_set_memory_limit(limit)
+        try:
+            hits, ordered = timed_order(cs, args)
+        finally:
+            L.qpip_set_memory_limit(0)
+        assert ordered == by_polygon
+        for c in ("polygon_index", "point_index"):
+            assert np.array_equal(hits[c].cpu().numpy(), want[c].cpu().numpy())
+
+
 @pytest.mark.parametrize("edges", [3, 8, 63, 64, 65, 129])
 def test_signed_zeros_match_oracle(cs, oracle_mod, edges):
     """Polygons with vertices at y = +0 and y = -0 and points at both, of ring lengths
