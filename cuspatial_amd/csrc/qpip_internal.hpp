@@ -137,8 +137,8 @@ void pool_stats(size_t* live, size_t* cached);
 
 // Copies small device results (sizes, flags: 4-byte aligned, whole words) to host
 // memory and waits for the stream: one kernel writes them into pinned host memory
-// (a block taken from a list that grows to the number of concurrent calls and is
-// given back by pool_trim). A hipMemcpyAsync into pageable memory stages and waits by
+// (a block of a list that grows to the number of concurrent calls, MailboxList; pool_trim
+// frees it). A hipMemcpyAsync into pageable memory stages and waits by
 // itself: 10 to 15 us of a call's host time each. Not for a stream that captures.
 struct ReadBack {
   void* dst;

@@ -33,6 +33,7 @@
 #include <vector>
 
 #include "qpip_internal.hpp"
+#include "qpip_mailbox.hpp"
 
 namespace qpip {
 
@@ -325,45 +326,18 @@ namespace {
 
 constexpr size_t kMailboxBytes = 8192;
 
-struct Mailboxes {
-  std::mutex mu;
-  std::vector<void*> free;
-};
-
-Mailboxes& mailboxes()
+MailboxList& mailboxes()
 {
-  static Mailboxes* m = new Mailboxes;  // lives as long as any thread may call
+  static MailboxList* m = new MailboxList;  // lives as long as any thread may call
   return *m;
 }
 
-// A pinned block for one call; back in the list when the call ends. A call that throws
-// may leave a kernel in flight that still writes the block: it is not handed out again.
-class Mailbox {
- public:
-  Mailbox()
-  {
-    Mailboxes& m = mailboxes();
-    {
-      std::lock_guard<std::mutex> g(m.mu);
-      if (!m.free.empty()) {
-        p_ = m.free.back();
-        m.free.pop_back();
-        return;
-      }
-    }
-    QPIP_HIP(hipHostMalloc(&p_, kMailboxBytes, hipHostMallocPortable | hipHostMallocMapped));
-  }
-  void done()
-  {
-    Mailboxes& m = mailboxes();
-    std::lock_guard<std::mutex> g(m.mu);
-    m.free.push_back(p_);
-  }
-  uint32_t* get() const { return static_cast<uint32_t*>(p_); }
-
- private:
-  void* p_ = nullptr;
-};
+void* new_mailbox()
+{
+  void* p = nullptr;
+  QPIP_HIP(hipHostMalloc(&p, kMailboxBytes, hipHostMallocPortable | hipHostMallocMapped));
+  return p;
+}
 
 constexpr int kReadParts = 3;
 struct ReadParts {
@@ -391,7 +365,7 @@ void read_back(std::initializer_list<ReadBack> parts, hipStream_t stream)
     QPIP_HIP(hipStreamSynchronize(stream));
     return;
   }
-  Mailbox box;
+  Mailbox box(mailboxes(), current_device_nothrow, new_mailbox);
   ReadParts r{};
   int k = 0;
   for (ReadBack const& p : parts) {
@@ -401,26 +375,25 @@ void read_back(std::initializer_list<ReadBack> parts, hipStream_t stream)
   }
   uint32_t* out = nullptr;
   QPIP_HIP(hipHostGetDevicePointer(reinterpret_cast<void**>(&out), box.get(), 0));
+  box.launched();
   read_back_kernel<<<1, 256, 0, stream>>>(r, out);
   QPIP_LAUNCH_CHECK();
   QPIP_HIP(hipStreamSynchronize(stream));
-  uint32_t const* in = box.get();
+  box.landed();
+  uint32_t const* in = static_cast<uint32_t const*>(box.get());
   for (ReadBack const& p : parts) {
     std::memcpy(p.dst, in, p.bytes);
     in += p.bytes / sizeof(uint32_t);
   }
-  box.done();
 }
 
 void pool_trim()
 {
-  {
-    Mailboxes& m = mailboxes();
-    std::lock_guard<std::mutex> g(m.mu);
-    for (void* p : m.free) (void)hipHostFree(p);
-    m.free.clear();
-  }
-  DevicePool& p = pool_for_device(current_device());
+  int const dev = current_device();
+  mailboxes().trim(
+    dev, [] { return hipDeviceSynchronize() == hipSuccess; },
+    [](void* p) { (void)hipHostFree(p); });
+  DevicePool& p = pool_for_device(dev);
   std::lock_guard<std::mutex> g(p.mu);
   release_cached(p);
 }
