@@ -163,6 +163,61 @@ __device__ __forceinline__ void fold_run(NearestArgs const& a, uint64_t rs, uint
   }
 }
 
+__device__ __forceinline__ double lane_value(double v, uint32_t lane)
+{
+  uint64_t const b = static_cast<uint64_t>(__double_as_longlong(v));
+  auto half        = [&](uint64_t w) {
+    return static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(w), lane));
+  };
+  return __longlong_as_double(
+    static_cast<long long>((static_cast<uint64_t>(half(b >> 32)) << 32) | half(b)));
+}
+
+// The same fold for one point, (px, py) in every lane of a full wave: 64 pairs at a time,
+// a linestring per lane. Where all distances are positive the fold is the smallest
+// (distance, linestring), whatever the order; with a zero or a NaN among them it goes pair
+// by pair.
+__device__ __forceinline__ void fold_point(NearestArgs const& a, uint64_t rs, uint64_t re,
+                                           double px, double py, uint32_t& best_ls,
+                                           double& best_d, bool& err)
+{
+  best_ls = 0;
+  best_d  = 0.0;
+  for (uint64_t kb = rs; kb < re; kb += kWave) {
+    bool const in = kb + lane_id() < re;
+    uint32_t ls   = in ? a.pair_ls[kb + lane_id()] : 0u;
+    bool const ok = in && ls < a.num_ls;
+    if (in && !ok) err = true;
+    double d = ok ? own_linestring_distance(a, ls, px, py) : INFINITY;
+    if (ballot(ok && !(d > 0.0)) == 0) {
+      if (!ok) ls = 0xffffffffu;
+#pragma unroll
+      for (int o = kWave / 2; o > 0; o >>= 1) {
+        double const od   = __shfl_xor(d, o, kWave);
+        uint32_t const ol = __shfl_xor(ls, o, kWave);
+        if (od < d || (od == d && ol < ls)) {
+          d  = od;
+          ls = ol;
+        }
+      }
+      if (ls < a.num_ls && take_next(best_d, best_ls, d, ls)) {
+        best_ls = ls;
+        best_d  = d;
+      }
+    } else {
+      for (uint64_t m = ballot(ok); m; m &= m - 1) {
+        uint32_t const j  = static_cast<uint32_t>(__builtin_ctzll(m));
+        double const dj   = lane_value(d, j);
+        uint32_t const lj = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(ls), j));
+        if (take_next(best_d, best_ls, dj, lj)) {
+          best_ls = lj;
+          best_d  = dj;
+        }
+      }
+    }
+  }
+}
+
 __global__ void __launch_bounds__(256) nearest_fill_kernel(NearestArgs a)
 {
   uint64_t const p = static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
@@ -293,12 +348,17 @@ struct RunChunkOp {
 // (the first exception needs a distance below 2^-23 M, the second only adds to one). If
 // the reference's distance to that linestring is then within E of the float32 one it is
 // the answer. Otherwise (an exception above, two linestrings that near, a zero distance,
-// a linestring without segments, coordinates that are not finite or above 1e15) the lane
-// folds over the run's pairs, as the reference does.
+// a linestring without segments, coordinates that are not finite or above 1e15) the point
+// folds over the run's pairs, as the reference does: a few such points one after the
+// other with a linestring per lane (fold_point), many at once with the linestrings in
+// turn (fold_run), and so does every point of a run of one pair, which leaves no choice.
+// One such point had held its wave for the whole fold: 1,000 points, 20,000 linestrings
+// (1,355 per leaf) took 5.8 ms, 2.3 so and 4.5 with a wave per pair.
 //
 // Bound by the float32 instructions. 1e6 points, 20,000 linestrings of 2 to 32
 // vertices (about 15 per leaf of 61 points): one wave per pair, each segment a chain of
-// scalar loads and a double division, took 1232 us; this takes 362 us.
+// scalar loads and a double division, took 1232 us; this takes 253 us (359 with every point
+// not decided in float32 folding with the linestrings in turn).
 constexpr int kNearWaves = 4;
 struct NearSegments {
   float4 s[kWave];  // start, direction
@@ -368,7 +428,7 @@ __global__ void __launch_bounds__(kNearWaves * kWave)
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
   };
-  for (uint64_t kb = 0; kb < R; kb += kWave) {
+  for (uint64_t kb = 0; R > 1 && kb < R; kb += kWave) {
     // the next 64 pairs' vertex ranges, one per lane
     uint32_t const nj = R - kb < kWave ? static_cast<uint32_t>(R - kb) : kWave;
     uint32_t v_lo = 0, v_n = 0;  // first vertex, segments
@@ -463,10 +523,27 @@ __global__ void __launch_bounds__(kNearWaves * kWave)
   double best_d    = 0.0;
   if (own && decided) {
     best_ls = a.pair_ls[l1];
-    best_d  = own_linestring_distance(a, best_ls, px, py);
+    if (ballot(best_ls != uniform(best_ls)) == 0)  // one for all: its vertices loaded once
+      best_d = point_linestring_distance(a, uniform(best_ls), px, py);
+    else
+      best_d = own_linestring_distance(a, best_ls, px, py);
     decided = best_d > 0.0 && fabs(best_d - static_cast<double>(sqrtf(m1))) <= E;  // not NaN
   }
-  if (own && !decided) fold_run(a, rs, rs + R, px, py, best_ls, best_d, err);
+  uint64_t const todo = ballot(own && !decided);
+  if (3 * static_cast<uint64_t>(__popcll(todo)) * ((R + kWave - 1) / kWave) < R) {
+    for (uint64_t m = todo; m; m &= m - 1) {
+      uint32_t const j = static_cast<uint32_t>(__builtin_ctzll(m));
+      uint32_t ls;
+      double d;
+      fold_point(a, rs, rs + R, lane_value(px, j), lane_value(py, j), ls, d, err);
+      if (static_cast<uint32_t>(lane) == j) {
+        best_ls = ls;
+        best_d  = d;
+      }
+    }
+  } else if (own && !decided) {
+    fold_run(a, rs, rs + R, px, py, best_ls, best_d, err);
+  }
   if (own) {
     a.out_point[pos] = static_cast<uint32_t>(pos);
     a.out_ls[pos]    = best_ls;

@@ -196,6 +196,36 @@ def test_points_on_a_segment_match_oracle(cs, oracle_mod, n, at):
     assert 0 < lost.sum() < n
 
 
+@pytest.mark.parametrize("n", [3, 70, 200])
+@pytest.mark.parametrize("lines,odd", [(1, 0), (2, 1), (63, 1), (64, 1), (65, 2), (150, 3),
+                                       (150, 200), (700, 5)])
+def test_few_undecided_points_of_long_runs_match_oracle(cs, oracle_mod, n, lines, odd):
+    """Runs of one pair and of one to eleven 64-pair steps, of which a few points (or
+    most) are not decided in float32 and fold with a linestring per lane: on a vertex, on a
+    segment (zeros and NaN in the fold), between two copies of a linestring (ties to the
+    lower id), and beside a linestring without segments."""
+    rng = np.random.default_rng(lines * 1000 + n + odd)
+    x, y = rng.uniform(0, 100, n), rng.uniform(0, 100, n)
+    v = [rng.uniform(0, 100, 2) + np.cumsum(rng.normal(0, 3, (int(k), 2)), 0)
+         for k in rng.integers(2, 9, lines)]
+    if lines > 3:
+        v[lines // 2], v[-1] = v[1].copy(), v[0].copy()
+        v[2] = v[2][:1]
+    k = min(odd, n)
+    for i in range(k):
+        line = v[int(rng.integers(0, lines))]
+        if i % 3 == 0 or len(line) < 2:
+            p = line[-1]
+        elif i % 3 == 1:
+            p = line[0] + rng.uniform(0.1, 0.9) * (line[1] - line[0])
+        else:
+            p = v[0][0] + 1e-3
+        x[i], y[i] = np.clip(p, 0, 100)
+    offs = np.concatenate([[0], np.cumsum([len(a) for a in v])]).astype(np.int32)
+    c = np.concatenate(v)
+    leaf_fold(cs, oracle_mod, x, y, offs, c[:, 0].copy(), c[:, 1].copy(), (0.0, 128.0, 0.0, 128.0))
+
+
 @pytest.mark.parametrize("first", [True, False])
 def test_underflowing_segment_matches_oracle(cs, oracle_mod, first):
     """A linestring of one segment whose squared length and projection underflow: the
