@@ -338,12 +338,14 @@ struct FrontierSource {
 //   * from 2^20 nodes and 64 per box the frontiers fill the GPU at every level: 1.21
 //     million and 100 boxes 868 / 583 / 551, 1.4 million and 20,000 719 / 764 / 687, 2.18
 //     million and 20,000 1959 / 1188 / 954 (1002 with the children classified twice).
+// Two levels past the depth of a full tree of that many nodes few are left, and steps
+// take three: a join of 89,916 nodes of 15 levels and 5,000 boxes 852 -> 845 us.
 // The grid has a block per 64 boxes or 512 nodes, at most kScanBlocks and 64 at least: a
 // box meets a few nodes of a level, or it covers many and their number is the nodes'.
 // 1.21 million nodes and 100 boxes at three levels per step: 1367 us with 65 blocks (the
 // boxes alone), 874 with this many or 1024; 84 nodes and 200 boxes 27 against 31.
 struct JoinShape {
-  int levels;
+  int levels, deep;  // levels per step, and the level past which they are kJoinStep
   unsigned blocks;
 };
 
@@ -351,8 +353,10 @@ inline JoinShape join_shape(uint64_t nodes, uint64_t boxes)
 {
   uint64_t const want   = 64 + (boxes + nodes / 8) / 64;
   unsigned const blocks = static_cast<unsigned>(want < kScanBlocks ? want : kScanBlocks);
-  if (nodes <= boxes) return {kJoinStep, blocks};
-  return {nodes >= (uint64_t{1} << 20) && nodes / 64 >= boxes ? 1 : 2, blocks};
+  int deep = 2;  // log4(nodes) + 2
+  while (deep < kMaxJoinLevels && (uint64_t{1} << (2 * (deep - 1))) <= nodes) ++deep;
+  if (nodes <= boxes) return {kJoinStep, deep, blocks};
+  return {nodes >= (uint64_t{1} << 20) && nodes / 64 >= boxes ? 1 : 2, deep, blocks};
 }
 
 // The whole traversal of `depth` levels from the top elements; fr[2] are the frontiers'
@@ -363,10 +367,11 @@ void launch_join(Top const& top, TreeView const& t, BoxView const& bx, Geom cons
                  JoinShape shape, StepCount* partials, hipStream_t stream, char const* timer)
 {
   unsigned const blocks = shape.blocks;
-  for (int lvl = 0, step = 0; lvl < depth; lvl += shape.levels, ++step) {
+  for (int lvl = 0, step = 0; lvl < depth; lvl += s.levels, ++step) {
     KernelTimer kt(timer, stream);
-    s.lvl     = lvl;
-    s.levels  = depth - lvl < shape.levels ? depth - lvl : shape.levels;
+    int const take = lvl > shape.deep ? kJoinStep : shape.levels;
+    s.lvl          = lvl;
+    s.levels       = depth - lvl < take ? depth - lvl : take;
     s.fr_node = fr_node[step % 2];
     s.fr_bbox = fr_bbox[step % 2];
     if (lvl == 0) {

@@ -394,15 +394,21 @@ def test_gaussian_holes_full_size_properties(cs, oracle_mod):
     (60000, 8, 8, 40, (5000, 1 << 20)),           # more: two
     (1300000, 11, 1, 30, (1 << 20, 1 << 32)),     # from 2^20 and 64 per box: one
     (1300000, 11, 1, 40000, (1 << 20, 1 << 32)),  # ... unless there are fewer per box
+    (60000, 15, 4, 40, (5000, 1 << 17)),          # dense spots: levels past the full tree's
 ])
 def test_join_steps_match_oracle(cs, oracle_mod, n, d, ms, zones, nodes):
     """The join's levels per step and grid (join_shape): a partition of the square into
     zones, whose boxes meet many nodes, on both sides of each line. The oracle's pairs."""
     rng = np.random.default_rng(n + zones)
     ext = 1024.0
-    pts = cs.Points(rng.uniform(0, ext, n), rng.uniform(0, ext, n))
-    _, tree = cs.quadtree_on_points(pts, 0.0, ext, 0.0, ext, ext / 2**d, d, ms)
+    px, py = rng.uniform(0, ext, n), rng.uniform(0, ext, n)
+    if d == 15:
+        px[: n // 2] = 300.0 + rng.normal(0, 0.5, n // 2)
+        py[: n // 2] = 700.0 + rng.normal(0, 0.5, n // 2)
+    _, tree = cs.quadtree_on_points(cs.Points(px, py), 0.0, ext, 0.0, ext, ext / 2**d, d, ms)
     assert nodes[0] <= len(tree) < nodes[1]
+    if d == 15:
+        assert (np_(tree["level"]) == d - 1).sum() > 1000
     # columns of uneven widths, each cut into rows
     cols = max(1, int(np.sqrt(zones)))
     x = np.concatenate([[0.0], np.sort(rng.uniform(0, ext, cols - 1)), [ext]])
