@@ -553,10 +553,9 @@ __device__ __forceinline__ void unpack_hits(uint64_t const (&keep_m)[kSlots],
 // kPipPairsPerLaunch pairs, so a grid never exceeds 2^28 work-items.
 constexpr uint64_t kPipPairsPerLaunch = uint64_t{1} << 22;
 
-// Eight waves per SIMD: the compiler then keeps the kernel within 96 scalar
-// registers (spilling some of the per-polygon state to vector-register lanes,
-// none inside the edge loops); the extra wave hides more of the point gathers'
-// latency (batched join: 10.2 -> 10.0 ms per launch).
+// Seven waves per SIMD: with eight the compiler spills vector registers (us of the test,
+// seven / eight: 2e8 points in 20,000 cells 7054 / 7381, 1e8 in 100 3155 / 3306, 1e7 in
+// 20,000 400 / 441, 1e6 in 50 60 / 65).
 // Workgroups are dealt to the 8 XCDs round-robin (block b to XCD b % 8), and each
 // XCD has its own L2. Adjacent pairs usually share a leaf, whose points a wave
 // finds in L2 only if the wave that gathered them ran on the same XCD. So block b

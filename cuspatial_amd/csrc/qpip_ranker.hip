@@ -126,16 +126,11 @@ __device__ __forceinline__ void fourier4(float u, float v, int k, float (&f)[4])
 // ---------------------------------------------------------------------------------
 __global__ void __launch_bounds__(256)
   features_kernel(GridView g, uint16_t const* __restrict__ emb, double const* __restrict__ xy,
-                  int64_t n, int64_t rows, uint16_t* __restrict__ X, uint32_t* __restrict__ cells)
+                  int64_t n, uint16_t* __restrict__ X, uint32_t* __restrict__ cells)
 {
   int64_t const i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i >= rows) return;
+  if (i >= n) return;
   uint16_t* x = X + i * kIn;
-  if (i >= n) {  // padding rows: zero features
-    for (int d = 0; d < kIn; ++d) x[d] = 0;
-    cells[i] = 0;
-    return;
-  }
   Loc const L = locate_cell(g, xy[2 * i], xy[2 * i + 1]);
   cells[i]    = L.cell;
   uint16_t const* e = emb + static_cast<int64_t>(L.cell) * kEmb;
@@ -1340,8 +1335,7 @@ extern "C" int qpip_ranker_features(const qpip_ranker* model,
     StreamScope scope(stream);
     Layout const lay(model->num_cells);
     features_kernel<<<grid_for(static_cast<uint64_t>(num_points), 256, 1u << 30), 256, 0,
-                      stream>>>(g, model->params_bf16 + lay.e, xy, num_points, num_points,
-                                features, cells);
+                      stream>>>(g, model->params_bf16 + lay.e, xy, num_points, features, cells);
     QPIP_LAUNCH_CHECK();
   });
 }

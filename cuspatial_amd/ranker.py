@@ -276,7 +276,8 @@ class Ranker:
 class LocateResult:
     polygon: torch.Tensor  # int32 per point: polygon, -1 none
     tests: torch.Tensor    # uint8 per point: exact tests run by the learned pass
-    flags: torch.Tensor    # uint8: bit 0 quadtree path, bit 1 first prediction not the answer
+    # uint8: bit 0 quadtree path, bit 1 first prediction not the answer (overflowed cell: 1)
+    flags: torch.Tensor
     fallback: int          # points that took the quadtree path
     extra_pairs: tuple     # (polygon, point) pairs beyond one per point, from the fallback
     seconds: dict

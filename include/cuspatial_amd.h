@@ -356,8 +356,8 @@ QPIP_API int qpip_point_in_polygon(const double* x,
  * forbid it). Same checks, test and output as qpip_point_in_polygon, but the caller
  * passes the output, `result` (num_x INT32 in device memory), and the edge table
  * lives in a fixed device array of the library (10.75 MiB per device, kept until
- * the process ends). The call allocates nothing, queues its two kernels on `stream`
- * and returns without waiting.
+ * the process ends). The call allocates nothing, queues its kernels (three at most)
+ * on `stream` and returns without waiting.
  * Limits: at most QPIP_NOALLOC_MAX_VERTICES polygon vertices and
  * QPIP_NOALLOC_MAX_RINGS rings; larger inputs fail with QPIP_ERROR_CAPACITY.
  * Every call on one GPU uses that GPU's one scratch array: calls that overlap on
@@ -708,7 +708,7 @@ QPIP_API int qpip_ranker_adam(float* params,
  * its cell overflowed, its hit lies within the collinearity filter of an edge
  * (another polygon's test could also hold), or max_tests ran out.
  * out_tests[i]: tests run. out_flags[i]: bit 0 quadtree path, bit 1 the first
- * prediction was not the answer. All arrays are device arrays. */
+ * prediction was not the answer (an overflowed cell makes none: 1). All arrays are device arrays. */
 QPIP_API int qpip_ranker_locate(const qpip_ranker* model,
                                 const qpip_grid* grid,
                                 const int32_t* poly_offsets,
