@@ -162,6 +162,7 @@ __global__ void __launch_bounds__(256)
 }
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef bf16x8 bf16x8_any __attribute__((aligned(2)));  // of a caller's array
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef short s16x2 __attribute__((ext_vector_type(2)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
@@ -391,7 +392,7 @@ __global__ void __launch_bounds__(kMlpWaves * kWave, 1) mlp_kernel(MlpArgs a)
       uint16_t const* e = a.emb + static_cast<int64_t>(L.cell) * kEmb;
 #pragma unroll
       for (int c = 0; c < kEmb / kKT; ++c)
-        X[t][c] = *reinterpret_cast<bf16x8 const*>(e + kKT * c + 8 * g);
+        X[t][c] = *reinterpret_cast<bf16x8_any const*>(e + kKT * c + 8 * g);
       // features 64 + 8g + j: frequencies 2g (j < 4) and 2g + 1 (j >= 4)
       float f0[4], f1[4];
       fourier4(L.u, L.v, 2 * g, f0);

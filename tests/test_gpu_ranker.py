@@ -304,6 +304,25 @@ def test_locator_short_rings_equal_plain_join(env, edges, exponent, n):
         assert int(res.tests.max()) <= most
 
 
+def test_parameters_at_any_element(env):
+    """The bf16 parameters may begin at any element of a caller's array: logits and the
+    weights' gradients are those of an aligned copy."""
+    torch, cs, ranker, rk, _ = env
+    _, P, grid, xy, x, y = voronoi(env, 3000, 100, 5, 16)
+    model = ranker.Ranker(grid.num_cells, seed=2)
+    labels = torch.zeros(len(x), dtype=torch.int32, device="cuda")
+    want = model.logits(grid, xy).clone()
+    grad = model.gradients(grid, xy, labels)[0].clone()
+    held = torch.empty(model.params_bf16.numel() + 3, dtype=torch.bfloat16, device="cuda")
+    tail = grid.num_cells * 64
+    for shift in (1, 3):
+        aligned = model.params_bf16
+        model.params_bf16 = held[shift:shift + aligned.numel()].copy_(aligned)
+        assert torch.equal(model.logits(grid, xy), want)
+        assert torch.equal(model.gradients(grid, xy, labels)[0][tail:], grad[tail:])
+        model.params_bf16 = aligned
+
+
 def test_flags_of_points_without_a_prediction(env):
     """Points of a cell with too many candidates are left to the quadtree path without a
     test or a prediction (flags 1), and those of a cell without candidates have no answer
