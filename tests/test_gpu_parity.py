@@ -605,7 +605,7 @@ def test_point_in_polygon_bitmask_random(cs, oracle_mod, seed, n, npoly, layout)
 @pytest.mark.parametrize("n", [1, 63, 64, 65, 129, 600001, 2200003])
 def test_bitmask_box_filter_and_queue(cs, oracle_mod, n):
     """The bitmask test's box filter and queue at the edges of its 64-point chunks and
-    at several and eight chunks per wave: small polygons (a few points per flush),
+    at one to six chunks per wave: small polygons (a few points per flush),
     large ones (several flushes), long rings, a polygon without vertices, points a
     ULP outside a box, NaN, infinite and huge coordinates. Exact."""
     rng = np.random.default_rng(n)
