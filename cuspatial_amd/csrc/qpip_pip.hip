@@ -43,6 +43,7 @@
 //   fallback (count, then allocate; :220-234) is the only path here.
 #include <algorithm>
 #include <mutex>
+#include <type_traits>
 
 #include "qpip_pip.hpp"
 #include "qpip_scan.hpp"
@@ -324,12 +325,11 @@ __device__ __forceinline__ uint32_t high_word(double v)
 __device__ __forceinline__ float high_as_float(double v) { return __uint_as_float(high_word(v)); }
 
 // R: edges per round of the loops, whose LDS reads are in flight together.
-template <int U, int S = kStageEdges, int R = 2>
+template <int U, int S = kStageEdges, int R = 2, int N = kSlots>
 __device__ __forceinline__ void test_polygon(PipArgs const& a, uint32_t poly,
-                                             double const (&px)[kSlots],
-                                             double const (&py)[kSlots],
-                                             uint64_t const (&valid_m)[kSlots], double pmax,
-                                             uint64_t (&hit_m)[kSlots], bool& err,
+                                             double const (&px)[N], double const (&py)[N],
+                                             uint64_t const (&valid_m)[N], double pmax,
+                                             uint64_t (&hit_m)[N], bool& err,
                                              PipStage<S>* stage, uint32_t lg = 0,
                                              RingHint const* hint = nullptr)
 {
@@ -1247,8 +1247,8 @@ __global__ void __launch_bounds__(256)
 // One wave holds up to kBmChunks chunks of 64 points in LDS and takes the polygons one
 // after the other: the points inside the polygon's vertex box (box_excludes, with the
 // wave's largest coordinate in place of the point's own: a wider margin, so it keeps
-// no fewer) queue up, and every 64 of them (and the rest, in lane groups) run over
-// the ring's edges. Random points against regions: a box holds a few percent of them,
+// no fewer) queue up, and every 192 of them run over the ring's edges, three per lane;
+// the rest two per lane, or up to 64 in lane groups. Random points against regions: a box holds a few percent of them,
 // so most (point, polygon) pairs cost four comparisons instead of the ring's edges.
 // What a polygon's test reads first (its box, ring range and first ring's entries)
 // is loaded once per workgroup, one polygon per thread, instead of as a chain of
@@ -1256,7 +1256,11 @@ __global__ void __launch_bounds__(256)
 // Bound by the edge steps. 2,000,003 points, 31 polygons of 4 to 256 vertices, boxes of
 // about a tenth of the square: every point over every edge (two slots of 64 points)
 // took 2020 us, this 490 us (620 with a comparison per decision in the edge step). Two
-// edges' LDS reads in flight instead of four cost 17 us; eight change nothing.
+// edges' LDS reads in flight instead of four cost 17 us; eight change nothing. Where the
+// boxes hold most points (31 polygons of 128 edges over most of the square, 2,000,000
+// points) an edge's LDS reads serve one point per lane at 2564 us, two at 2015 and three
+// at 1887; four and six leave no registers for the short flushes (bitmask of the regions
+// above 594 and 605 us for 516). Every edge for every point takes 1584 there.
 // Six chunks: fuller flushes than four or five (45 us), and 12 waves per CU, three on
 // each SIMD, where seven and eight chunks leave room for ten (22 us).
 constexpr int kBmChunks = 6;    // 64-point chunks per wave at most
@@ -1264,6 +1268,8 @@ constexpr int kBmWaves  = 2;    // waves per workgroup
 constexpr int kBmStage  = 128;  // edges per staged batch
 constexpr int kBmRound  = 4;    // edges whose LDS reads are in flight together
 constexpr int kBmPolys  = 31;
+constexpr int kBmSlots  = 3;    // points per lane of a full flush
+constexpr uint32_t kBmFull = kBmSlots * kWave;
 
 struct BmPoly {
   PolyBox box;
@@ -1273,7 +1279,7 @@ struct BmPoly {
 struct BmWave {
   double2 p[kBmChunks * kWave];
   uint32_t bits[kBmChunks * kWave];
-  uint16_t queue[2 * kWave];
+  uint16_t queue[kBmFull + kWave];
   PipStage<kBmStage> stage;
 };
 
@@ -1349,6 +1355,28 @@ __global__ void __launch_bounds__(kBmWaves * kWave)
       test_polygon<1, kBmStage, kBmRound>(a, j, px, py, test_m, pmax, hit_m, err, &s.stage, 6u - g, &rh);
       if ((hit_m[0] >> lane) & 1ull) s.bits[slot] |= 1u << j;
     };
+    auto flush_slots = [&](auto slots, uint32_t q) {  // the same, that many per lane
+      constexpr int U = decltype(slots)::value;
+      double px[U], py[U];
+      uint64_t hit_m[U], test_m[U];
+      uint32_t slot[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        uint32_t const at = static_cast<uint32_t>(u * kWave + lane);
+        slot[u]           = s.queue[at < q ? at : 0];
+        double2 const pt  = s.p[slot[u]];
+        px[u]             = pt.x;
+        py[u]             = pt.y;
+        hit_m[u]          = 0;
+        test_m[u]         = ballot(at < q);
+      }
+      test_polygon<U, kBmStage>(a, j, px, py, test_m, pmax, hit_m, err, &s.stage, 0, &rh);
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        if ((hit_m[u] >> lane) & 1ull) s.bits[slot[u]] |= 1u << j;
+    };
+    constexpr std::integral_constant<int, kBmSlots> all_slots{};
+    constexpr std::integral_constant<int, 2> two_slots{};
     for (uint32_t c = 0; c < nc; ++c) {
       double2 const pt = s.p[c * kWave + lane];
       bool const keep  = p0 + c * kWave + lane < n &&
@@ -1361,18 +1389,22 @@ __global__ void __launch_bounds__(kBmWaves * kWave)
           static_cast<uint16_t>(c * kWave + lane);
       fence();
       qn += static_cast<uint32_t>(__popcll(km));
-      if (qn < kWave) continue;
-      flush(kWave);
+      if (qn < kBmFull) continue;
+      flush_slots(all_slots, kBmFull);
       fence();
-      uint16_t const rest = s.queue[kWave + lane];
+      uint16_t const rest = s.queue[kBmFull + lane];
       fence();
       s.queue[lane] = rest;
-      qn -= kWave;
+      qn -= kBmFull;
     }
-    if (qn > 0) {
-      fence();
+    if (qn == 0) continue;
+    fence();
+    if (qn > 2 * kWave)
+      flush_slots(all_slots, qn);
+    else if (qn > kWave)
+      flush_slots(two_slots, qn);
+    else
       flush(qn);
-    }
   }
   fence();
   for (uint32_t c = 0; c < nc; ++c) {
