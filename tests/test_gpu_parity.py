@@ -639,6 +639,37 @@ def test_bitmask_box_filter_and_queue(cs, oracle_mod, n):
         assert len(tbl[j]) == n and np.array_equal(np_(tbl[j]), ((ref >> j) & 1).astype(bool))
 
 
+@pytest.mark.parametrize("shift", [0.0, 1e6])
+@pytest.mark.parametrize("n", [300, 2000003])
+def test_bitmask_outliers(cs, oracle_mod, n, shift):
+    """Points far from every box (around 256 times the boxes' largest coordinate, and up to
+    and above 2^400), infinite and NaN in x, in y and in both, among ordinary ones on
+    vertices and beside them; also with boxes at the origin alone. Exact."""
+    rng = np.random.default_rng(n)
+    part, ring, vx, vy = star_polygons(rng, 20, 100.0, 20.0, 60.0, kmin=20, kmax=60)
+    vx, vy = vx + shift, vy + shift
+    x, y = rng.uniform(-5, 105, n) + shift, rng.uniform(-5, 105, n) + shift
+    top = max(np.abs(vx).max(), np.abs(vy).max())
+    odd = np.array([255 * top, 256 * top, 257 * top, 300 * top, 1e30, 2.0**399, 2.0**400,
+                    2.0**401, 1e305, np.inf, np.nan])
+    odd = np.concatenate([odd, -odd])
+    k = min(n // 3, 2200)
+    v, at = np.resize(odd, k), rng.permutation(n)[:k]
+    kind = rng.integers(0, 3, k)
+    x[at] = np.where(kind != 1, v, x[at])
+    y[at] = np.where(kind != 0, rng.permutation(v), y[at])
+    at = rng.permutation(n)[:k]
+    i = rng.integers(0, len(vx), k)
+    x[at], y[at] = np.nextafter(vx[i], vx[i] + rng.integers(-1, 2, k)), vy[i]
+    for size in (1.0, 0.0):  # as they are, and every polygon a point at the origin
+        px, py = vx * size, vy * size
+        ref = oracle_mod.point_in_polygon_bitmask(x, y, part, ring, px, py)
+        got = cs.point_in_polygon_bitmask(cs.Points(x, y, device="cuda"),
+                                          cs.Polygons(part, ring, px, py, device="cuda"))
+        assert np.array_equal(np_(got).astype(np.int64), ref.astype(np.int64))
+        assert size == 0.0 or (ref != 0).sum() > n // 10
+
+
 @pytest.mark.parametrize("n", [1, 64, 65, 128, 129, 600001, 1048577])
 @pytest.mark.parametrize("polygons", [1, 5, 31])
 def test_bitmask_of_few_vertices_and_the_line(cs, oracle_mod, n, polygons):
